@@ -482,4 +482,265 @@ __device__ __forceinline__ void coopRows(const KArgs& a, bool act, double x, dou
     }
 }
 
+// ------------------------------------------------ neighbours in batches
+// A neighbour sum keeps the reference's order: each accumulator takes its
+// terms one after the other.  What a term costs -- the gathers of the
+// neighbour's data, a square root and a division, several hundred cycles of
+// dependent FP64 operations -- need not be serial, though.  The neighbours
+// are handed to the operator in batches: it forms the batch's terms side by
+// side without branches (a neighbour that fails a test contributes +0.0,
+// which leaves every sum as it is) and adds them in order.
+//
+// With L > 1 lanes per particle, neighbour c0 + b L + l of a batch belongs to
+// lane l of the particle's L neighbouring lanes, and every lane adds every
+// lane's term in that order (addOrdered), so all L hold the same sums.  One
+// lane per particle leaves a small system at a fraction of a wavefront per
+// SIMD, each of them waiting out ~120 neighbours one by one: the viscosity
+// of 1,728 particles took 47 us and takes 9.4 us with 16 lanes.  Adding L
+// terms L times costs issue slots, so L falls as the particles fill the chip
+// (lanesPerParticle).
+template <int B_, bool LIST_, class E>
+struct NbrBatch {
+    static constexpr int B = B_;
+    static constexpr bool list = LIST_;
+    int j[B_];
+    double x[B_], y[B_], z[B_], w[B_];   // w: P4.w (list) or the type (walk)
+    E e[B_];                             // load(j)
+    bool ok[B_];                         // false past the particle's last neighbour
+};
+template <class T>
+__device__ __forceinline__ int nbrType(const KArgs& a, const T& t, int b) {
+    return T::list ? p4TypeOf(a, t.w[b]) : (int)t.w[b];
+}
+
+// value of lane l of the group of L lanes
+template <int L, int l>
+__device__ __forceinline__ int groupLane(int v) {
+    static_assert(L == 2 || L == 4 || L == 16, "groups of 2, 4 or 16 lanes");
+    // DPP: quad_perm (2: [l, l, l + 2, l + 2], 4: [l, l, l, l]) or row_newbcast l
+    return __builtin_amdgcn_update_dpp(0, v, L == 2 ? (l ? 0xf5 : 0xa0) : L == 4 ? l * 0x55 : 0x150 + l, 0xf, 0xf, true);
+}
+template <int L, int l>
+__device__ __forceinline__ double groupLane(double v) {
+    return __hiloint2double(groupLane<L, l>(__double2hiint(v)), groupLane<L, l>(__double2loint(v)));
+}
+template <int L, int l = 0>
+__device__ __forceinline__ void addOrdered(double& acc, double t) {
+    if constexpr (L == 1) {
+        acc += t;
+    } else if constexpr (l < L) {
+        acc += groupLane<L, l>(t);
+        addOrdered<L, l + 1>(acc, t);
+    }
+}
+template <int L>
+__device__ __forceinline__ int groupSumInt(int v) {
+    for (int o = L / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+// the smaller of the lanes' values, by the comparison "if (m > v) m = v"
+template <int L>
+__device__ __forceinline__ double groupMin(double m) {
+    for (int o = L / 2; o > 0; o >>= 1) {
+        const double v = __shfl_xor(m, o, 64);
+        if (m > v) m = v;
+    }
+    return m;
+}
+// lane within its group and particle slot, L lanes per particle
+template <int L>
+__device__ __forceinline__ int groupLaneId() { return L == 1 ? 0 : (int)(threadIdx.x & (L - 1)); }
+template <int L>
+__device__ __forceinline__ int groupSlot() { return (int)((blockIdx.x * blockDim.x + threadIdx.x) / L); }
+
+// The list of slot i (column-major [K][N], K a multiple of 32) in batches: G
+// entries per lane are gathered together and handed to body B at a time.
+// Entries past the row's end are read (L G divides 32, so they lie in the
+// array) and replaced by the particle itself: the list addresses then depend
+// on the wave-uniform c0 only.
+template <int L, int B, int G, class Load, class Body>
+__device__ __forceinline__ void listBatches(const KArgs& a, const int* nbr, const int* cnt, int i, Load&& load,
+                                            Body&& body) {
+    static_assert(32 % (L * G) == 0 && G % B == 0, "a batch must divide the list's column padding");
+    const int n = cnt[i];
+    if (n <= 0) return;
+    const int l = groupLaneId<L>();
+    const size_t N = a.N;
+    const int* __restrict__ col = nbr + ((size_t)l * N + i);
+    const double4* __restrict__ P4 = a.P4;
+    const bool periodic = periodicDomain(a.P);
+    using E = decltype(load(0));
+    int k[G];
+#pragma unroll
+    for (int b = 0; b < G; b++) k[b] = col[(size_t)(b * L) * N];
+    for (int c0 = 0; c0 < n; c0 += L * G) {
+        int j[G];
+        double4 q[G];
+        E e[G];
+#pragma unroll
+        for (int b = 0; b < G; b++) {
+            j[b] = c0 + b * L + l < n ? (periodic ? (int)((unsigned)k[b] & kListSlotMask) : k[b]) : i;
+            q[b] = P4[j[b]];
+            e[b] = load(j[b]);
+        }
+        if (periodic) {
+            // entries carry the ghost shift in bits 30-31 (1: bPBC -1, 2: +1)
+#pragma unroll
+            for (int b = 0; b < G; b++) {
+                const unsigned g = (unsigned)k[b] >> 30;
+                const int pbc = g == 1u ? -1 : (g == 2u ? 1 : 0);
+                q[b].x = q[b].x + pbc * a.P.periodic_length[0];
+                q[b].y = q[b].y + pbc * a.P.periodic_length[1];
+                q[b].z = q[b].z + pbc * a.P.periodic_length[2];
+            }
+        }
+        // the next batch's slots, issued after the gathers: loads complete in
+        // issue order, so waiting for the gathers does not wait for these
+        if (c0 + L * G < n) {
+#pragma unroll
+            for (int b = 0; b < G; b++) k[b] = col[(size_t)(c0 + (G + b) * L) * N];
+        }
+#pragma unroll
+        for (int h = 0; h < G; h += B) {
+            NbrBatch<B, true, E> t;
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                t.j[b] = j[h + b];
+                t.x[b] = q[h + b].x;
+                t.y[b] = q[h + b].y;
+                t.z[b] = q[h + b].z;
+                t.w[b] = q[h + b].w;
+                t.e[b] = e[h + b];
+                t.ok[b] = c0 + (h + b) * L + l < n;
+            }
+            body(t);
+        }
+    }
+}
+
+// The candidates of a bucket walk around (x, y, z), in walk order and L at a
+// time: f(j, xj, yj, zj, pbc, ok) for candidate c0 + l of a stencil row (of a
+// bucket in a periodic domain; pbc: its ghost shift).  Every lane of the
+// group makes every call; ok is false for the particle itself and past the
+// row's end.
+template <int L, class F>
+__device__ __forceinline__ void walkGroup(const KArgs& a, int i, double x, double y, double z, F&& f) {
+    const mps_params& P = a.P;
+    const int c[3] = {(int)((x - P.domain_min[0]) * P.inv_bucket_side + KEPS),
+                      (int)((y - P.domain_min[1]) * P.inv_bucket_side + KEPS),
+                      (int)((z - P.domain_min[2]) * P.inv_bucket_side + KEPS)};
+    const int d3 = (int)(P.dim - 2.0);
+    const int nx = P.num_buckets_x, ny = P.num_buckets_y, nz = P.num_buckets_z;
+    const double* __restrict__ X = a.D[DX];
+    const double* __restrict__ Y = a.D[DY];
+    const double* __restrict__ Z = a.D[DZ];
+    const int l = groupLaneId<L>();
+    const bool periodic = periodicDomain(P);
+    const int pd = P.periodic_dir[0] ? 0 : (P.periodic_dir[1] ? 1 : 2);
+    auto run = [&](int s, int e, int pbc) {
+        double px = 0.0, py = 0.0, pz = 0.0;
+        if (periodic) {
+            px = pbc * P.periodic_length[0];
+            py = pbc * P.periodic_length[1];
+            pz = pbc * P.periodic_length[2];
+        }
+        for (int c0 = s; c0 < e; c0 += L) {
+            const int j = min(c0 + l, e - 1);
+            double xj = X[j], yj = Y[j], zj = Z[j];
+            if (periodic) {
+                xj = xj + px;
+                yj = yj + py;
+                zj = zj + pz;
+            }
+            f(j, xj, yj, zj, pbc, c0 + l < e && j != i);
+        }
+    };
+    for (int jz = (c[2] - 1) * d3; jz <= (c[2] + 1) * d3; jz++) {
+        if (jz < 0 || jz >= nz) continue;
+        for (int jy = c[1] - 1; jy <= c[1] + 1; jy++) {
+            if (jy < 0 || jy >= ny) continue;
+            if (!periodic) {
+                const int row = jz * P.num_buckets_xy + jy * nx;
+                const int jx0 = max(c[0] - 1, 0), jx1 = min(c[0] + 1, nx - 1);
+                if (jx0 > jx1) continue;
+                // buckets jx0 .. jx1 of one row are contiguous in slot order
+                run(a.cellStart[row + jx0], a.cellStart[row + jx1 + 1], 0);
+            } else {
+                // ghost layers 0 and n - 1 of the periodic axis: walkCellsPeriodic
+                for (int jx = c[0] - 1; jx <= c[0] + 1; jx++) {
+                    if (jx < 0 || jx >= nx) continue;
+                    int bx = jx, by = jy, bz = jz, pbc = 0;
+                    int& bd = pd == 0 ? bx : (pd == 1 ? by : bz);
+                    const int nd = pd == 0 ? nx : (pd == 1 ? ny : nz);
+                    if (bd == 0) { bd = nd - 2; pbc = -1; }
+                    else if (bd == nd - 1) { bd = 1; pbc = 1; }
+                    const int key = bz * P.num_buckets_xy + by * nx + bx;
+                    run(a.cellStart[key], a.cellStart[key + 1], pbc);
+                }
+            }
+        }
+    }
+}
+
+// Neighbours of slot i in batches: from the list (SMALL: the small-radius
+// one, for operators whose radii are at most re_s or the collision distance)
+// or from a bucket walk, whose candidates come one per lane.
+template <bool LIST, bool SMALL, int L, int B, int G, class Load, class Body>
+__device__ __forceinline__ void forBatches(const KArgs& a, int i, double x, double y, double z, Load&& load,
+                                           Body&& body) {
+    if constexpr (LIST) {
+        listBatches<L, B, G>(a, SMALL ? a.nbrS : a.nbr, SMALL ? a.nbrCntS : a.nbrCnt, i, load, body);
+    } else {
+        const int* __restrict__ T = a.I[ITYPE];
+        auto one = [&](int j, double xj, double yj, double zj, bool ok) {
+            NbrBatch<1, false, decltype(load(0))> t;
+            t.j[0] = j;
+            t.x[0] = xj;
+            t.y[0] = yj;
+            t.z[0] = zj;
+            t.w[0] = (double)T[j];
+            t.e[0] = load(j);
+            t.ok[0] = ok;
+            body(t);
+        };
+        if constexpr (L == 1)
+            walkCellsPos(a, i, x, y, z, [&](int j, double xj, double yj, double zj) { one(j, xj, yj, zj, true); });
+        else
+            walkGroup<L>(a, i, x, y, z, [&](int j, double xj, double yj, double zj, int, bool ok) { one(j, xj, yj, zj, ok); });
+    }
+}
+struct NoLoad {
+    __device__ __forceinline__ NoExtra operator()(int) const { return NoExtra{}; }
+};
+
+// weights of a batch: one uniform branch on the weight type, the square roots
+// and divisions side by side
+template <int B>
+__device__ __forceinline__ void wgtBatch(const double (&d)[B], double re, int t, double (&w)[B]) {
+    switch (t) {
+        case 1:
+#pragma unroll
+            for (int b = 0; b < B; b++) w[b] = re / d[b] + d[b] / re - 2.0;
+            break;
+        case 2:
+#pragma unroll
+            for (int b = 0; b < B; b++) w[b] = re / d[b] - d[b] / re;
+            break;
+        case 3:
+#pragma unroll
+            for (int b = 0; b < B; b++) w[b] = (1.0 - d[b] / re) * (1.0 - d[b] / re) * (1.0 - d[b] / re);
+            break;
+        case 4:
+#pragma unroll
+            for (int b = 0; b < B; b++) w[b] = (1.0 - d[b] / re) * (1.0 - d[b] / re);
+            break;
+        default:
+#pragma unroll
+            for (int b = 0; b < B; b++) w[b] = re / d[b] - 1.0;
+            break;
+    }
+}
+// true when no lane of the wave has a term (the batch can be passed over)
+__device__ __forceinline__ bool noneInWave(bool any) { return __builtin_amdgcn_ballot_w64(any) == 0; }
+
 }  // namespace mpsgpu

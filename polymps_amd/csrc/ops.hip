@@ -397,11 +397,11 @@ __global__ __launch_bounds__(64) void kMaskToList(KArgs a, const unsigned* mask,
 
 // ------------------------------------------------------------- viscosity
 // MpsViscosity::calcViscosity (src/MpsViscosity.cpp:20-102)
-template <bool LIST>
-__global__ void kViscosity(KArgs a) {
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kViscosity(KArgs a) {
     // gathers 64 B per neighbour: the XCD-contiguous order keeps them in one
     // L2 (HBM fetch 7.0 -> 1.9 GB per launch at 1.73M, 1.65 -> 1.56 ms)
-    const int i = xcdSlotId();
+    const int i = xcdSlotId() / L;
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
@@ -415,29 +415,42 @@ __global__ void kViscosity(KArgs a) {
     const double ux = a.D[DU][i], uy = a.D[DV][i], uz = a.D[DW][i];
     const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
     double ax = 0, ay = 0, az = 0;
-    auto term = [&](double xj, double yj, double zj, int tj, double uj, double vj, double wj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_l2 && (d2 < dm2 || pw)) {
-            const double wL = wgt(sqrt(d2), P.re_l, P.weight_type);
-            const double nu = (tj == P.wall) ? nuW : nuF;
-            ax += (uj - ux) * wL * nu;
-            ay += (vj - uy) * wL * nu;
-            az += (wj - uz) * wL * nu;
-        }
+    // with the list, the packed velocities (V4) are gathered with the positions
+    auto vel = [&](int j) {
+        if constexpr (LIST) return a.V4[j];
+        else return make_double4(a.D[DU][j], a.D[DV][j], a.D[DW][j], 0.0);
     };
-    if (LIST) {
-        // positions and packed velocities (V4) of a batch gathered together
-        listNbrsQV(a, a.V4, i, [&](int, const double4& q, const double4& v) {
-            term(q.x, q.y, q.z, p4TypeOf(a, q.w), v.x, v.y, v.z);
-        });
-    } else {
-        forNbrsPosType<false>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj, int tj) {
-            term(xj, yj, zj, tj, a.D[DU][j], a.D[DV][j], a.D[DW][j]);
-        });
-    }
+    forBatches<LIST, false, L, B, G>(a, i, xi, yi, zi, vel, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], t0[nb], t1[nb], t2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2 < P.re_l2) & ((d2 < dm2) | pw);
+            any = any | ok[b];
+            d[b] = sqrt(d2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_l, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double nu = (nbrType(a, t, b) == P.wall) ? nuW : nuF;
+            t0[b] = ok[b] ? (t.e[b].x - ux) * w[b] * nu : 0.0;
+            t1[b] = ok[b] ? (t.e[b].y - uy) * w[b] * nu : 0.0;
+            t2[b] = ok[b] ? (t.e[b].z - uz) * w[b] * nu : 0.0;
+        }
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            addOrdered<L>(ax, t0[b]);
+            addOrdered<L>(ay, t1[b]);
+            addOrdered<L>(az, t2[b]);
+        }
+    });
+    if (groupLaneId<L>() != 0) return;
     a.D[DAX][i] = P.coeff_visc_multiphase * ax;
     a.D[DAY][i] = P.coeff_visc_multiphase * ay;
     a.D[DAZ][i] = P.coeff_visc_multiphase * az;
@@ -663,9 +676,9 @@ __global__ void kCompact(KArgs a, int* outList, int cap, const int* slotOf) {
 
 // ------------------------------------------------------------ collisions
 // MpsParticleCollision::checkParticleCollisions (src/MpsParticleCollision.cpp:22-119)
-template <bool LIST>
-__global__ void kCollisionPC(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kCollisionPC(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     if (a.I[ITYPE][i] != P.fluid) return;
@@ -675,25 +688,43 @@ __global__ void kCollisionPC(KArgs a) {
     const double ux = a.D[DU][i], uy = a.D[DV][i], uz = a.D[DW][i];
     const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
     double dux = 0, duy = 0, duz = 0;
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.dist_collision_limit2 && (d2 < dm2 || pw)) {
-            double fDT = (ux - a.D[DU][j]) * v0 + (uy - a.D[DV][j]) * v1 + (uz - a.D[DW][j]) * v2;
-            if (fDT > 0.0) {
-                const bool fj = a.I[ITYPE][j] == P.fluid;
-                const double mj = fj ? phaseDensity(a, j) : P.dns_wall;
-                fDT *= P.restitution_collision * mj / (mi + mj) / d2;
-                if (fj) {
-                    dux -= v0 * fDT; duy -= v1 * fDT; duz -= v2 * fDT;
-                } else {
-                    dux -= 2.0 * v0 * fDT; duy -= 2.0 * v1 * fDT; duz -= 2.0 * v2 * fDT;
+    forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2 < P.dist_collision_limit2) & ((d2 < dm2) | pw);
+            any = any | ok[b];
+        }
+        if (noneInWave(any)) return;   // pairs this close are rare
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            double t0 = 0.0, t1 = 0.0, t2 = 0.0;
+            if (ok[b]) {
+                const int j = t.j[b];
+                const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+                const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+                double fDT = (ux - a.D[DU][j]) * v0 + (uy - a.D[DV][j]) * v1 + (uz - a.D[DW][j]) * v2;
+                if (fDT > 0.0) {
+                    const bool fj = a.I[ITYPE][j] == P.fluid;
+                    const double mj = fj ? phaseDensity(a, j) : P.dns_wall;
+                    fDT *= P.restitution_collision * mj / (mi + mj) / d2;
+                    // dux -= v0 fDT: the negated term is added
+                    t0 = fj ? -(v0 * fDT) : -(2.0 * v0 * fDT);
+                    t1 = fj ? -(v1 * fDT) : -(2.0 * v1 * fDT);
+                    t2 = fj ? -(v2 * fDT) : -(2.0 * v2 * fDT);
                 }
             }
+            addOrdered<L>(dux, t0);
+            addOrdered<L>(duy, t1);
+            addOrdered<L>(duz, t2);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     a.D[DDVX][i] = dux; a.D[DDVY][i] = duy; a.D[DDVZ][i] = duz;
 }
 
@@ -925,9 +956,9 @@ __global__ void kUpdateNear(KArgs a) {
 }
 
 // MpsPndNeigh::calcWallNPCD (src/MpsPndNeigh.cpp:105-195)
-template <bool LIST>
-__global__ void kWallNPCD(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kWallNPCD(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     if (!(a.I[ITYPE][i] == P.fluid && a.I[INEARWALL][i])) return;
@@ -936,16 +967,32 @@ __global__ void kWallNPCD(KArgs a) {
     double n[3], R[9], ns;
     reflectSqrt(xi, xm, n, R, &ns);
     double nx = 0, ny = 0, nz = 0;
-    forNbrsPosS<LIST>(a, i, xi[0], xi[1], xi[2], [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi[0], v1 = yj - xi[1], v2 = zj - xi[2];
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - xm[0], w1 = yj - xm[1], w2 = zj - xm[2];
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && dm2 < P.re_s2 && d2 < dm2) {
-            const double wS = wgt(sqrt(dm2), P.re_s, P.weight_type);
-            nx += w0 * wS; ny += w1 * wS; nz += w2 * wS;
+    forBatches<LIST, true, L, B, G>(a, i, xi[0], xi[1], xi[2], NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], w0[nb], w1[nb], w2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi[0], v1 = t.y[b] - xi[1], v2 = t.z[b] - xi[2];
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            w0[b] = t.x[b] - xm[0];
+            w1[b] = t.y[b] - xm[1];
+            w2[b] = t.z[b] - xm[2];
+            const double dm2 = w0[b] * w0[b] + w1[b] * w1[b] + w2[b] * w2[b];
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & (dm2 < P.re_s2) & (d2 < dm2);
+            any = any | ok[b];
+            d[b] = sqrt(dm2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            addOrdered<L>(nx, ok[b] ? w0[b] * w[b] : 0.0);
+            addOrdered<L>(ny, ok[b] ? w1[b] * w[b] : 0.0);
+            addOrdered<L>(nz, ok[b] ? w2[b] * w[b] : 0.0);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     const double w0 = xi[0] - xm[0], w1 = xi[1] - xm[1], w2 = xi[2] - xm[2];
     const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
     if (dm2 < P.re_s2) {
@@ -959,58 +1006,85 @@ __global__ void kWallNPCD(KArgs a) {
 
 // ------------------------------------------------------ correction matrix
 // MpsVectorMatrix::correctionMatrix + inverseMatrix (src/MpsVectorMatrix.cpp:20-165)
-__device__ __forceinline__ void inverse3(double* M, int dim) {
+// DIM is a template parameter so that every index is known at compile time
+// and the matrices stay in registers (with a run-time bound they were moved
+// to 72 KB of LDS per block, which left two wavefronts per SIMD).
+template <int DIM>
+__device__ __forceinline__ void inverse3(double (&M)[9]) {
     double A[9], B[9];
+#pragma unroll
     for (int q = 0; q < 9; q++) A[q] = M[q];
-    if (dim == 2) { A[2] = A[5] = A[6] = A[7] = 0.0; A[8] = 1.0; }
+    if (DIM == 2) { A[2] = A[5] = A[6] = A[7] = 0.0; A[8] = 1.0; }
+#pragma unroll
     for (int q = 0; q < 9; q++) B[q] = (q % 4 == 0) ? 1.0 : 0.0;
     const double det = (A[0] * A[4] * A[8] + A[1] * A[5] * A[6] + A[2] * A[3] * A[7]) -
                        (A[2] * A[4] * A[6] + A[1] * A[3] * A[8] + A[0] * A[5] * A[7]);
-    if (det <= KEPS) {
-        for (int q = 0; q < 9; q++) M[q] = (q % 4 == 0) ? 1.0 : 0.0;
-        return;
-    }
-    for (int k = 0; k < dim; k++)
-        for (int r = 0; r < dim; r++) {
+#pragma unroll
+    for (int k = 0; k < DIM; k++)
+#pragma unroll
+        for (int r = 0; r < DIM; r++) {
             if (r == k) continue;
             const double m = A[r * 3 + k] / A[k * 3 + k];
-            for (int c = 0; c < dim; c++) {
+#pragma unroll
+            for (int c = 0; c < DIM; c++) {
                 A[r * 3 + c] -= m * A[k * 3 + c];
                 B[r * 3 + c] -= m * B[k * 3 + c];
             }
         }
-    for (int r = 0; r < dim; r++)
-        for (int c = 0; c < dim; c++) B[r * 3 + c] /= A[r * 3 + r];
-    for (int q = 0; q < 9; q++) M[q] = B[q];
+#pragma unroll
+    for (int r = 0; r < DIM; r++)
+#pragma unroll
+        for (int c = 0; c < DIM; c++) B[r * 3 + c] /= A[r * 3 + r];
+    const bool singular = det <= KEPS;
+#pragma unroll
+    for (int q = 0; q < 9; q++) M[q] = singular ? ((q % 4 == 0) ? 1.0 : 0.0) : B[q];
 }
 
-template <bool LIST>
-__global__ void kCorrectionMatrix(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kCorrectionMatrix(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
+    // (wS v_r) v_c and (wS v_c) v_r round differently, so all nine are summed
     double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-            const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-            const double inv = 1.0 / d2;
-            M[0] += wS * v0 * v0 * inv; M[1] += wS * v0 * v1 * inv; M[2] += wS * v0 * v2 * inv;
-            M[3] += wS * v1 * v0 * inv; M[4] += wS * v1 * v1 * inv; M[5] += wS * v1 * v2 * inv;
-            M[6] += wS * v2 * v0 * inv; M[7] += wS * v2 * v1 * inv; M[8] += wS * v2 * v2 * inv;
+    forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], inv[nb], v[nb][3];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            v[b][0] = t.x[b] - xi;
+            v[b][1] = t.y[b] - yi;
+            v[b][2] = t.z[b] - zi;
+            const double d2 = v[b][0] * v[b][0] + v[b][1] * v[b][1] + v[b][2] * v[b][2];
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & ((d2 < dm2) | pw);
+            any = any | ok[b];
+            d[b] = sqrt(d2);
+            inv[b] = 1.0 / d2;
         }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++)
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+#pragma unroll
+                for (int c = 0; c < 3; c++)
+                    addOrdered<L>(M[r * 3 + c], ok[b] ? w[b] * v[b][r] * v[b][c] * inv[b] : 0.0);
     });
+    if (groupLaneId<L>() != 0) return;
+#pragma unroll
     for (int q = 0; q < 9; q++) M[q] *= -P.coeff_press_grad;
-    inverse3(M, (int)P.dim);
-    if (a.I[INNEIGH][i] < 4)
-        for (int q = 0; q < 9; q++) M[q] = (q % 4 == 0) ? 1.0 : 0.0;
-    for (int q = 0; q < 9; q++) a.D[DCM0 + q][i] = M[q];
+    if ((int)P.dim == 2) inverse3<2>(M);
+    else inverse3<3>(M);
+    const bool few = a.I[INNEIGH][i] < 4;
+#pragma unroll
+    for (int q = 0; q < 9; q++) a.D[DCM0 + q][i] = few ? ((q % 4 == 0) ? 1.0 : 0.0) : M[q];
 }
 
 // ------------------------------------------------------------------ PND
@@ -1053,9 +1127,9 @@ __global__ void kInitialPnd(KArgs a) {
 }
 
 // MpsPndNeigh::calcPndnNeighNPCD (src/MpsPndNeigh.cpp:199-331)
-template <bool LIST>
-__global__ void kPndNeighNPCD(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kPndNeighNPCD(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
@@ -1063,22 +1137,42 @@ __global__ void kPndNeighNPCD(KArgs a) {
     const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
     double ni = 0.0, wSum = 0.0;
     double c0 = a.D[DNPX][i], c1 = a.D[DNPY][i], c2 = a.D[DNPZ][i];
-    int nn = a.I[INNWALL][i];
-    forNbrsPos<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_l2 && (d2 < dm2 || pw)) {
-            nn += 1;
-            if (d2 < P.re_s2) {
-                const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-                ni += wS;
-                c0 += v0 * wS; c1 += v1 * wS; c2 += v2 * wS;
-                wSum += wS;
-            }
+    int nn = 0;
+    forBatches<LIST, false, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d2[nb], v0[nb], v1[nb], v2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            v0[b] = t.x[b] - xi;
+            v1[b] = t.y[b] - yi;
+            v2[b] = t.z[b] - zi;
+            d2[b] = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2[b] < P.re_l2) & ((d2[b] < dm2) | pw);
+            nn += ok[b] ? 1 : 0;
+            ok[b] = ok[b] & (d2[b] < P.re_s2);
+            any = any | ok[b];
+        }
+        // a quarter of the large list is within re_s
+        if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+        double d[nb], w[nb];
+#pragma unroll
+        for (int b = 0; b < nb; b++) d[b] = sqrt(d2[b]);
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double wS = ok[b] ? w[b] : 0.0;
+            addOrdered<L>(ni, wS);
+            addOrdered<L>(c0, ok[b] ? v0[b] * wS : 0.0);
+            addOrdered<L>(c1, ok[b] ? v1[b] * wS : 0.0);
+            addOrdered<L>(c2, ok[b] ? v2[b] * wS : 0.0);
         }
     });
+    wSum = ni;   // the same terms in the same order
+    nn = a.I[INNWALL][i] + groupSumInt<L>(nn);
+    if (groupLaneId<L>() != 0) return;
     a.I[INNEIGH][i] = nn;
     const double small = ni + a.D[DPNDWALL][i];
     if (P.pnd_type == MPS_PND_SUM_WIJ || P.pnd_type == MPS_PND_MEAN_SUM_WIJ) {
@@ -1093,9 +1187,9 @@ __global__ void kPndNeighNPCD(KArgs a) {
 }
 
 // calcPndDiffusiveTerm (src/MpsPndNeigh.cpp:334-489)
-template <bool LIST>
-__global__ void kPndDiffusive(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kPndDiffusive(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
@@ -1108,39 +1202,65 @@ __global__ void kPndDiffusive(KArgs a) {
     const double Pi = a.D[DPRESS][i];
     const bool fi = a.I[ITYPE][i] == P.fluid;
     double MC[9];
+#pragma unroll
     for (int q = 0; q < 9; q++) MC[q] = a.D[DCM0 + q][i];
     double Di = 0.0, DivV = 0.0;
     const double flagDi = 1.0;
-    forNbrsPos<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_l2 && (d2 < dm2 || pw)) {
-            const double dst = sqrt(d2);
-            const double wL = wgt(dst, P.re_l, P.weight_type);
-            if (fi && a.I[ITYPE][j] == P.fluid) {
-                const double rhoj = rhoOf(a, j);
+    forBatches<LIST, false, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double v0[nb], v1[nb], v2[nb], d2[nb], d[nb], w[nb];
+        bool ok[nb], small[nb], any = false, anyS = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            v0[b] = t.x[b] - xi;
+            v1[b] = t.y[b] - yi;
+            v2[b] = t.z[b] - zi;
+            d2[b] = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2[b] < P.re_l2) & ((d2[b] < dm2) | pw);
+            small[b] = ok[b] & (d2[b] < P.re_s2);
+            any = any | ok[b];
+            anyS = anyS | small[b];
+            d[b] = sqrt(d2[b]);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_l, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            double term = 0.0;
+            if (ok[b] && fi && a.I[ITYPE][t.j[b]] == P.fluid) {
+                const double rhoj = rhoOf(a, t.j[b]);
                 const double pgh = -2.0 * (rho * rhoj / (rho + rhoj)) *
-                                   (P.gravity[0] * v0 + P.gravity[1] * v1 + P.gravity[2] * v2);
-                const double Pj = a.D[DPRESS][j];
-                Di += P.time_step / rho * P.coeff_visc_multiphase * (Pj - Pi - pgh) * wL;
+                                   (P.gravity[0] * v0[b] + P.gravity[1] * v1[b] + P.gravity[2] * v2[b]);
+                const double Pj = a.D[DPRESS][t.j[b]];
+                term = P.time_step / rho * P.coeff_visc_multiphase * (Pj - Pi - pgh) * w[b];
             }
-            if (d2 < P.re_s2) {
+            addOrdered<L>(Di, term);
+        }
+        if (noneInWave(anyS)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            double term = 0.0;
+            if (small[b]) {
+                const int j = t.j[b];
                 const double vx = a.D[DU][j] - ux, vy = a.D[DV][j] - uy, vz = a.D[DW][j] - uz;
-                const double wS = wgt(dst, P.re_s, P.weight_type);
                 if (!P.gradient_correction) {
-                    if (ni > KEPS)
-                        DivV += (P.dim / P.pnd_small_zero) * (a.D[DPNDI][j] / ni) * (vx * v0 + vy * v1 + vz * v2) * wS / d2;
+                    term = (P.dim / P.pnd_small_zero) * (a.D[DPNDI][j] / ni) *
+                           (vx * v0[b] + vy * v1[b] + vz * v2[b]) * w[b] / d2[b];
+                    if (!(ni > KEPS)) term = 0.0;
                 } else {
-                    const double q0 = (v0 * MC[0] + v1 * MC[1] + v2 * MC[2]);
-                    const double q1 = (v0 * MC[3] + v1 * MC[4] + v2 * MC[5]);
-                    const double q2 = (v0 * MC[6] + v1 * MC[7] + v2 * MC[8]);
-                    DivV += (P.dim / P.pnd_small_zero) * (vx * q0 + vy * q1 + vz * q2) * wS / d2;
+                    const double q0 = (v0[b] * MC[0] + v1[b] * MC[1] + v2[b] * MC[2]);
+                    const double q1 = (v0[b] * MC[3] + v1[b] * MC[4] + v2[b] * MC[5]);
+                    const double q2 = (v0[b] * MC[6] + v1[b] * MC[7] + v2[b] * MC[8]);
+                    term = (P.dim / P.pnd_small_zero) * (vx * q0 + vy * q1 + vz * q2) * w[b] / d2[b];
                 }
             }
+            addOrdered<L>(DivV, term);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     a.D[DAUX1][i] = ni * (1.0 + P.time_step * (-DivV + Di * flagDi));
     a.D[DDIVU][i] = DivV;
     a.D[DDIFF][i] = Di;
@@ -1239,29 +1359,41 @@ __global__ void kUpdatePnd(KArgs a) {
 }
 
 // meanPndParticlesWallDummySurface (src/MpsPndNeigh.cpp:777-852), first pass
-template <bool LIST>
-__global__ void kMeanPndWDS(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kMeanPndWDS(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
-    a.D[DAUX1][i] = 0.0;
-    a.D[DAUX2][i] = 0.0;
-    if (!(a.I[ITYPE][i] == P.wall || a.I[IBC][i] == P.surface)) return;
-    const bool pw = P.wall_type == MPS_WALL_PARTICLE;
-    const double xi = PX(i), yi = PY(i), zi = PZ(i);
-    const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
     double up = 0, dn = 0;
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-            const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-            up += a.D[DPNDI][j] * wS;
-            dn += wS;
-        }
-    });
+    if (a.I[ITYPE][i] == P.wall || a.I[IBC][i] == P.surface) {
+        const bool pw = P.wall_type == MPS_WALL_PARTICLE;
+        const double xi = PX(i), yi = PY(i), zi = PZ(i);
+        const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
+        auto pnd = [&](int j) { return a.D[DPNDI][j]; };
+        forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, pnd, [&](const auto& t) {
+            constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+            double d[nb], w[nb];
+            bool ok[nb], any = false;
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+                const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+                const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+                const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+                ok[b] = t.ok[b] & (d2 < P.re_s2) & ((d2 < dm2) | pw);
+                any = any | ok[b];
+                d[b] = sqrt(d2);
+            }
+            if (noneInWave(any)) return;
+            wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                addOrdered<L>(up, ok[b] ? t.e[b] * w[b] : 0.0);
+                addOrdered<L>(dn, ok[b] ? w[b] : 0.0);
+            }
+        });
+    }
+    if (groupLaneId<L>() != 0) return;
     a.D[DAUX1][i] = up;
     a.D[DAUX2][i] = dn;
 }
@@ -1540,50 +1672,69 @@ __global__ void kPressExplicit(KArgs a) {
 }
 
 // calcVelDivergence (src/MpsPressure.cpp:479-551)
-template <bool LIST>
-__global__ void kVelDivergence(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kVelDivergence(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
-    a.D[DDIVU][i] = 0.0;
-    if (a.I[ITYPE][i] != P.fluid) return;
-    const bool pw = P.wall_type == MPS_WALL_PARTICLE;
-    const double ni = a.D[DPNDI][i];
-    const double xi = PX(i), yi = PY(i), zi = PZ(i);
-    const double ux = a.D[DU][i], uy = a.D[DV][i], uz = a.D[DW][i];
-    const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
-    double MC[9];
-    for (int q = 0; q < 9; q++) MC[q] = a.D[DCM0 + q][i];
     double DivV = 0.0;
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-            const double vx = a.D[DU][j] - ux, vy = a.D[DV][j] - uy, vz = a.D[DW][j] - uz;
-            const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-            if (!P.gradient_correction) {
-                if (ni > KEPS)
-                    DivV += (P.dim / P.pnd_small_zero) * (a.D[DPNDI][j] / ni) * (vx * v0 + vy * v1 + vz * v2) * wS / d2;
-            } else {
-                const double q0 = (v0 * MC[0] + v1 * MC[1] + v2 * MC[2]);
-                const double q1 = (v0 * MC[3] + v1 * MC[4] + v2 * MC[5]);
-                const double q2 = (v0 * MC[6] + v1 * MC[7] + v2 * MC[8]);
-                DivV += (P.dim / P.pnd_small_zero) * (vx * q0 + vy * q1 + vz * q2) * wS / d2;
+    if (a.I[ITYPE][i] == P.fluid) {
+        const bool pw = P.wall_type == MPS_WALL_PARTICLE;
+        const double ni = a.D[DPNDI][i];
+        const double xi = PX(i), yi = PY(i), zi = PZ(i);
+        const double ux = a.D[DU][i], uy = a.D[DV][i], uz = a.D[DW][i];
+        const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
+        double MC[9];
+#pragma unroll
+        for (int q = 0; q < 9; q++) MC[q] = a.D[DCM0 + q][i];
+        auto vel = [&](int j) { return make_double3(a.D[DU][j], a.D[DV][j], a.D[DW][j]); };
+        forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, vel, [&](const auto& t) {
+            constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+            double v0[nb], v1[nb], v2[nb], d2[nb], d[nb], w[nb];
+            bool ok[nb], any = false;
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                v0[b] = t.x[b] - xi;
+                v1[b] = t.y[b] - yi;
+                v2[b] = t.z[b] - zi;
+                d2[b] = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+                const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+                const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+                ok[b] = t.ok[b] & (d2[b] < P.re_s2) & ((d2[b] < dm2) | pw);
+                any = any | ok[b];
+                d[b] = sqrt(d2[b]);
             }
-        }
-    });
+            if (noneInWave(any)) return;
+            wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double vx = t.e[b].x - ux, vy = t.e[b].y - uy, vz = t.e[b].z - uz;
+                double term;
+                bool add = ok[b];
+                if (!P.gradient_correction) {
+                    add = add && ni > KEPS;
+                    term = (P.dim / P.pnd_small_zero) * (a.D[DPNDI][t.j[b]] / ni) *
+                           (vx * v0[b] + vy * v1[b] + vz * v2[b]) * w[b] / d2[b];
+                } else {
+                    const double q0 = (v0[b] * MC[0] + v1[b] * MC[1] + v2[b] * MC[2]);
+                    const double q1 = (v0[b] * MC[3] + v1[b] * MC[4] + v2[b] * MC[5]);
+                    const double q2 = (v0[b] * MC[6] + v1[b] * MC[7] + v2[b] * MC[8]);
+                    term = (P.dim / P.pnd_small_zero) * (vx * q0 + vy * q1 + vz * q2) * w[b] / d2[b];
+                }
+                addOrdered<L>(DivV, add ? term : 0.0);
+            }
+        });
+    }
+    if (groupLaneId<L>() != 0) return;
     a.D[DDIVU][i] = DivV;
 }
 
-// calcPressGradient (src/MpsPressure.cpp:1217-1338)
 // calcPressGradient (src/MpsPressure.cpp:1217-1338): acc = relax grad p / rho,
 // and with PRED predictionPressGradient (:932-1028): acc += (1 - relax)
 // grad p / rho without the gradient correction
-template <bool LIST, bool PRED>
+template <bool LIST, bool PRED, int L, int B, int G>
 __device__ __forceinline__ void pressGradientBody(const KArgs& a) {
-    const int i = slotId();
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
@@ -1593,44 +1744,72 @@ __device__ __forceinline__ void pressGradientBody(const KArgs& a) {
     const double Pi = a.D[DPRESS][i], ni = a.D[DPNDI][i];
     double pmin = Pi;
     double MC[9];
+#pragma unroll
     for (int q = 0; q < 9; q++) MC[q] = PRED ? 0.0 : a.D[DCM0 + q][i];
     const double* __restrict__ PR = a.D[DPRESS];
-    if (gt == 0 || gt == 2)
-        forNbrsPosSX<LIST>(a, i, xi, yi, zi, PR, [&](int j, double xj, double yj, double zj, auto pOf) {
-            const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-            const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-            if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-                const double pj = pOf();
-                if (pmin > pj) pmin = pj;
+    auto press = [PR](int j) { return PR[j]; };
+    if (gt == 0 || gt == 2) {
+        forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, press, [&](const auto& t) {
+            constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+                const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+                const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+                const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+                const bool ok = t.ok[b] & (d2 < P.re_s2) & ((d2 < dm2) | pw);
+                if (ok & (pmin > t.e[b])) pmin = t.e[b];
             }
         });
+        pmin = groupMin<L>(pmin);
+    }
     double ax = 0, ay = 0, az = 0;
-    forNbrsPosSX<LIST>(a, i, xi, yi, zi, PR, [&](int j, double xj, double yj, double zj, auto pOf) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-            double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-            const double pj = pOf();
-            if (gt == 0) wS *= (pj - pmin) / d2;
-            else if (gt == 1) wS *= (pj + Pi) / d2;
-            else if (gt == 2) wS *= (pj + Pi - 2.0 * pmin) / d2;
-            else if (gt == 3) {
-                const double nj = a.D[DPNDI][j];
-                if (ni > KEPS && nj > KEPS) wS *= (ni * pj / nj + nj * Pi / ni) / d2;
-            }
-            if (PRED || !P.gradient_correction) {
-                ax += v0 * wS; ay += v1 * wS; az += v2 * wS;
-            } else {
-                ax += (v0 * MC[0] + v1 * MC[1] + v2 * MC[2]) * wS;
-                ay += (v0 * MC[3] + v1 * MC[4] + v2 * MC[5]) * wS;
-                az += (v0 * MC[6] + v1 * MC[7] + v2 * MC[8]) * wS;
+    forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, press, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], d2[nb], v0[nb], v1[nb], v2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            v0[b] = t.x[b] - xi;
+            v1[b] = t.y[b] - yi;
+            v2[b] = t.z[b] - zi;
+            d2[b] = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2[b] < P.re_s2) & ((d2[b] < dm2) | pw);
+            any = any | ok[b];
+            d[b] = sqrt(d2[b]);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+        if (gt == 0) {
+#pragma unroll
+            for (int b = 0; b < nb; b++) w[b] *= (t.e[b] - pmin) / d2[b];
+        } else if (gt == 1) {
+#pragma unroll
+            for (int b = 0; b < nb; b++) w[b] *= (t.e[b] + Pi) / d2[b];
+        } else if (gt == 2) {
+#pragma unroll
+            for (int b = 0; b < nb; b++) w[b] *= (t.e[b] + Pi - 2.0 * pmin) / d2[b];
+        } else if (gt == 3) {
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double nj = a.D[DPNDI][t.j[b]];
+                if (ni > KEPS && nj > KEPS) w[b] *= (ni * t.e[b] / nj + nj * Pi / ni) / d2[b];
             }
         }
+        const bool plain = PRED || !P.gradient_correction;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double q0 = plain ? v0[b] : (v0[b] * MC[0] + v1[b] * MC[1] + v2[b] * MC[2]);
+            const double q1 = plain ? v1[b] : (v0[b] * MC[3] + v1[b] * MC[4] + v2[b] * MC[5]);
+            const double q2 = plain ? v2[b] : (v0[b] * MC[6] + v1[b] * MC[7] + v2[b] * MC[8]);
+            addOrdered<L>(ax, ok[b] ? q0 * w[b] : 0.0);
+            addOrdered<L>(ay, ok[b] ? q1 * w[b] : 0.0);
+            addOrdered<L>(az, ok[b] ? q2 * w[b] : 0.0);
+        }
     });
+    if (groupLaneId<L>() != 0) return;
     const double rho = rhoOf(a, i);
     if (PRED) {
         const double f = 1.0 - P.relax_press;
@@ -1643,17 +1822,17 @@ __device__ __forceinline__ void pressGradientBody(const KArgs& a) {
         a.D[DAZ][i] = P.relax_press * az * P.coeff_press_grad / rho;
     }
 }
-template <bool LIST>
-__global__ void kPressGradient(KArgs a) { pressGradientBody<LIST, false>(a); }
-template <bool LIST>
-__global__ void kPredPressGradient(KArgs a) { pressGradientBody<LIST, true>(a); }
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kPressGradient(KArgs a) { pressGradientBody<LIST, false, L, B, G>(a); }
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kPredPressGradient(KArgs a) { pressGradientBody<LIST, true, L, B, G>(a); }
 
 // calcWallPressGradient + repulsive forces (src/MpsPressure.cpp:1341-1611);
 // with PRED predictionWallPressGradient (:1031-1214): factor 1 - relax and
 // no wall force
-template <bool LIST, bool PRED>
+template <bool LIST, bool PRED, int L, int B, int G>
 __device__ __forceinline__ void wallPressGradientBody(const KArgs& a) {
-    const int i = slotId();
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     if (!(a.I[ITYPE][i] == P.fluid && a.I[INEARWALL][i])) return;
@@ -1668,39 +1847,70 @@ __device__ __forceinline__ void wallPressGradientBody(const KArgs& a) {
     double pmin = Pi;
     double n[3], R[9], ns;
     reflectSqrt(xi, xm, n, R, &ns);
-    if (gt == 0 || gt == 2)
-        forNbrsPos<LIST>(a, i, xi[0], xi[1], xi[2], [&](int j, double xj, double yj, double zj) {
-            const double v0 = xj - xi[0], v1 = yj - xi[1], v2 = zj - xi[2];
-            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-            const double w0 = xj - xm[0], w1 = yj - xm[1], w2 = zj - xm[2];
-            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-            if (d2 < P.re_s2 && d2 < dm2) {
-                const double pj = a.D[DPRESS][j];
-                if (pmin > pj) pmin = pj;
+    // every pair that counts is within re_s: the small-radius list holds them
+    const double* __restrict__ PR = a.D[DPRESS];
+    auto press = [PR](int j) { return PR[j]; };
+    if (gt == 0 || gt == 2) {
+        forBatches<LIST, true, L, B, G>(a, i, xi[0], xi[1], xi[2], press, [&](const auto& t) {
+            constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double v0 = t.x[b] - xi[0], v1 = t.y[b] - xi[1], v2 = t.z[b] - xi[2];
+                const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+                const double w0 = t.x[b] - xm[0], w1 = t.y[b] - xm[1], w2 = t.z[b] - xm[2];
+                const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+                const bool ok = t.ok[b] & (d2 < P.re_s2) & (d2 < dm2);
+                if (ok & (pmin > t.e[b])) pmin = t.e[b];
             }
         });
+        pmin = groupMin<L>(pmin);
+    }
     double ax = 0, ay = 0, az = 0;
-    auto term = [&](double Pj, double nj, double w0, double w1, double w2, double dm2) {
-        double wS = wgt(sqrt(dm2), P.re_s, P.weight_type);
-        if (gt == 0) wS *= (Pj - pmin) / dm2;
-        else if (gt == 1) wS *= (Pj + Pi) / dm2;
-        else if (gt == 2) wS *= (Pj + Pi - 2.0 * pmin) / dm2;
+    // the weight of a mirror pair at distance^2 dm2, from the kernel weight w
+    auto scaled = [&](double w, double Pj, double nj, double dm2) {
+        if (gt == 0) w *= (Pj - pmin) / dm2;
+        else if (gt == 1) w *= (Pj + Pi) / dm2;
+        else if (gt == 2) w *= (Pj + Pi - 2.0 * pmin) / dm2;
         else if (gt == 3) {
-            if (ni > KEPS && nj > KEPS) wS *= (ni * Pj / nj + nj * Pi / ni) / dm2;
+            if (ni > KEPS && nj > KEPS) w *= (ni * Pj / nj + nj * Pi / ni) / dm2;
         }
-        ax += w0 * wS; ay += w1 * wS; az += w2 * wS;
+        return w;
     };
-    forNbrsPos<LIST>(a, i, xi[0], xi[1], xi[2], [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi[0], v1 = yj - xi[1], v2 = zj - xi[2];
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - xm[0], w1 = yj - xm[1], w2 = zj - xm[2];
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && dm2 < P.re_s2 && d2 < dm2) term(a.D[DPRESS][j], a.D[DPNDI][j], w0, w1, w2, dm2);
+    forBatches<LIST, true, L, B, G>(a, i, xi[0], xi[1], xi[2], press, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], dm2[nb], w0[nb], w1[nb], w2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi[0], v1 = t.y[b] - xi[1], v2 = t.z[b] - xi[2];
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            w0[b] = t.x[b] - xm[0];
+            w1[b] = t.y[b] - xm[1];
+            w2[b] = t.z[b] - xm[2];
+            dm2[b] = w0[b] * w0[b] + w1[b] * w1[b] + w2[b] * w2[b];
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & (dm2[b] < P.re_s2) & (d2 < dm2[b]);
+            any = any | ok[b];
+            d[b] = sqrt(dm2[b]);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double nj = gt == 3 ? a.D[DPNDI][t.j[b]] : 0.0;
+            const double wS = scaled(w[b], t.e[b], nj, dm2[b]);
+            addOrdered<L>(ax, ok[b] ? w0[b] * wS : 0.0);
+            addOrdered<L>(ay, ok[b] ? w1[b] * wS : 0.0);
+            addOrdered<L>(az, ok[b] ? w2[b] * wS : 0.0);
+        }
     });
+    if (groupLaneId<L>() != 0) return;
     {
         const double w0 = xi[0] - xm[0], w1 = xi[1] - xm[1], w2 = xi[2] - xm[2];
         const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (dm2 < P.re_s2) term(Pi, ni, w0, w1, w2, dm2);
+        if (dm2 < P.re_s2) {
+            const double wS = scaled(wgt(sqrt(dm2), P.re_s, P.weight_type), Pi, ni, dm2);
+            ax += w0 * wS; ay += w1 * wS; az += w2 * wS;
+        }
     }
     double f0 = 0.0, f1 = 0.0, f2 = 0.0;
     if (ns < P.re_repulsive_force && ns > KEPS) {
@@ -1734,15 +1944,15 @@ __device__ __forceinline__ void wallPressGradientBody(const KArgs& a) {
         a.D[DFWZ][i] = a.D[DFWZ][i] + -g2 * vol;
     }
 }
-template <bool LIST>
-__global__ void kWallPressGradient(KArgs a) { wallPressGradientBody<LIST, false>(a); }
-template <bool LIST>
-__global__ void kPredWallPressGradient(KArgs a) { wallPressGradientBody<LIST, true>(a); }
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kWallPressGradient(KArgs a) { wallPressGradientBody<LIST, false, L, B, G>(a); }
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kPredWallPressGradient(KArgs a) { wallPressGradientBody<LIST, true, L, B, G>(a); }
 
 // calcWall{Slip,NoSlip}Viscosity (src/MpsViscosity.cpp:1527-1910)
-template <bool LIST>
-__global__ void kWallViscosity(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kWallViscosity(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     if (!(a.I[ITYPE][i] == P.fluid && a.I[INEARWALL][i])) return;
@@ -1785,25 +1995,38 @@ __global__ void kWallViscosity(KArgs a) {
     else nuI = 0.0;
     nuI = nuI / dnsI;
     double ax = 0, ay = 0, az = 0;
-    forNbrsPos<LIST>(a, i, xi[0], xi[1], xi[2], [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi[0], v1 = yj - xi[1], v2 = zj - xi[2];
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - xm[0], w1 = yj - xm[1], w2 = zj - xm[2];
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_l2 && dm2 < P.re_l2 && d2 < dm2) {
-            const double wL = wgt(sqrt(dm2), P.re_l, P.weight_type);
+    auto vel = [&](int j) { return make_double3(a.D[DU][j], a.D[DV][j], a.D[DW][j]); };
+    forBatches<LIST, false, L, B, G>(a, i, xi[0], xi[1], xi[2], vel, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi[0], v1 = t.y[b] - xi[1], v2 = t.z[b] - xi[2];
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            const double w0 = t.x[b] - xm[0], w1 = t.y[b] - xm[1], w2 = t.z[b] - xm[2];
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2 < P.re_l2) & (dm2 < P.re_l2) & (d2 < dm2);
+            any = any | ok[b];
+            d[b] = sqrt(dm2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_l, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
             double nu = nuJ;
             if (nn) {
-                const double mj = a.D[DMEU][j];
+                const double mj = a.D[DMEU][t.j[b]];
                 if ((meu + mj) > KEPS) nu = 2.0 * meu * mj / (meu + mj);
                 else nu = 0.0;
                 nu = nu / dnsI;
             }
-            ax += (a.D[DU][j] - umx) * wL * nu;
-            ay += (a.D[DV][j] - umy) * wL * nu;
-            az += (a.D[DW][j] - umz) * wL * nu;
+            addOrdered<L>(ax, ok[b] ? (t.e[b].x - umx) * w[b] * nu : 0.0);
+            addOrdered<L>(ay, ok[b] ? (t.e[b].y - umy) * w[b] * nu : 0.0);
+            addOrdered<L>(az, ok[b] ? (t.e[b].z - umz) * w[b] * nu : 0.0);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     {
         const double w0 = xi[0] - xm[0], w1 = xi[1] - xm[1], w2 = xi[2] - xm[2];
         const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
@@ -1871,29 +2094,42 @@ __global__ void kCommitStaged(KArgs a, int dst0) {
 }
 
 // calcConcAndConcGradient (src/MpsShifting.cpp:432-576), concentration pass
-template <bool LIST>
-__global__ void kShift2Conc(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kShift2Conc(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     const bool pw = P.wall_type == MPS_WALL_PARTICLE;
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
     double c = 0.0;
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-        if (d2 < P.re_s2 && (d2 < dm2 || pw)) c += wgt(sqrt(d2), P.re_s, P.weight_type);
+    forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & ((d2 < dm2) | pw);
+            any = any | ok[b];
+            d[b] = sqrt(d2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) addOrdered<L>(c, ok[b] ? w[b] : 0.0);
     });
+    if (groupLaneId<L>() != 0) return;
     c += a.D[DPNDWALL][i];
     a.D[DCONC][i] = c / P.pnd_small_zero;
 }
 // gradient pass: new positions staged in dvel slots
-template <bool LIST>
-__global__ void kShift2Grad(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kShift2Grad(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     double nx = PX(i), ny = PY(i), nz = PZ(i);
@@ -1903,27 +2139,43 @@ __global__ void kShift2Grad(KArgs a) {
         const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
         const double ci = a.D[DCONC][i];
         double g0 = 0, g1 = 0, g2 = 0;
-        forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-            const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-            const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
-            const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
-            if (d2 < P.re_s2 && (d2 < dm2 || pw)) {
-                const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-                const double cj = a.D[DCONC][j];
-                g0 += (ci + cj) * v0 * wS / d2;
-                g1 += (ci + cj) * v1 * wS / d2;
-                g2 += (ci + cj) * v2 * wS / d2;
+        forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+            constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+            double d[nb], w[nb], d2[nb], v0[nb], v1[nb], v2[nb];
+            bool ok[nb], any = false;
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                v0[b] = t.x[b] - xi;
+                v1[b] = t.y[b] - yi;
+                v2[b] = t.z[b] - zi;
+                d2[b] = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+                const double w0 = t.x[b] - mx, w1 = t.y[b] - my, w2 = t.z[b] - mz;
+                const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+                ok[b] = t.ok[b] & (d2[b] < P.re_s2) & ((d2[b] < dm2) | pw);
+                any = any | ok[b];
+                d[b] = sqrt(d2[b]);
+            }
+            if (noneInWave(any)) return;
+            wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+            for (int b = 0; b < nb; b++) {
+                const double cc = ci + a.D[DCONC][t.j[b]];
+                addOrdered<L>(g0, ok[b] ? cc * v0[b] * w[b] / d2[b] : 0.0);
+                addOrdered<L>(g1, ok[b] ? cc * v1[b] * w[b] / d2[b] : 0.0);
+                addOrdered<L>(g2, ok[b] ? cc * v2[b] * w[b] / d2[b] : 0.0);
             }
         });
         g0 *= -P.coeff_press_grad; g1 *= -P.coeff_press_grad; g2 *= -P.coeff_press_grad;
-        a.D[DGCX][i] = g0; a.D[DGCY][i] = g1; a.D[DGCZ][i] = g2;
+        if (groupLaneId<L>() == 0) {
+            a.D[DGCX][i] = g0; a.D[DGCY][i] = g1; a.D[DGCZ][i] = g2;
+        }
         if (a.I[IBC][i] == P.inner) {
             nx = nx - P.coeff_shifting2 * g0;
             ny = ny - P.coeff_shifting2 * g1;
             nz = nz - P.coeff_shifting2 * g2;
         }
     }
+    if (groupLaneId<L>() != 0) return;
     a.D[DDVX][i] = nx; a.D[DDVY][i] = ny; a.D[DDVZ][i] = nz;
 }
 // calcWallConcAndConcGradient (src/MpsShifting.cpp:578-692)
@@ -1977,25 +2229,38 @@ __global__ void kShift2Wall(KArgs a) {
 }
 
 // updateVelocityParticlesWallDummy (src/MpsParticleVelPos.cpp:100-158)
-template <bool LIST>
-__global__ void kWallDummyVelocity(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kWallDummyVelocity(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
     if (a.I[ITYPE][i] != P.dummy_wall) return;
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     double dx = 0, dy = 0, dz = 0, ni = 0;
-    forNbrsPos<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        if (d2 < P.re_l2 && a.I[ITYPE][j] == P.fluid) {
-            const double wL = wgt(sqrt(d2), P.re_l, P.weight_type);
-            ni += wL;
-            dx += a.D[DU][j] * wL;
-            dy += a.D[DV][j] * wL;
-            dz += a.D[DW][j] * wL;
+    forBatches<LIST, false, L, B, G>(a, i, xi, yi, zi, NoLoad{}, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double v0 = t.x[b] - xi, v1 = t.y[b] - yi, v2 = t.z[b] - zi;
+            const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+            ok[b] = t.ok[b] & (d2 < P.re_l2) & (nbrType(a, t, b) == P.fluid);
+            any = any | ok[b];
+            d[b] = sqrt(d2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_l, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const int j = t.j[b];
+            addOrdered<L>(ni, ok[b] ? w[b] : 0.0);
+            addOrdered<L>(dx, ok[b] ? a.D[DU][j] * w[b] : 0.0);
+            addOrdered<L>(dy, ok[b] ? a.D[DV][j] * w[b] : 0.0);
+            addOrdered<L>(dz, ok[b] ? a.D[DW][j] * w[b] : 0.0);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     if (ni > KEPS) {
         a.D[DU][i] = 2.0 * 0.0 - dx / ni;
         a.D[DV][i] = 2.0 * 0.0 - dy / ni;
@@ -2013,6 +2278,37 @@ __global__ void kWallDummyVelocity(KArgs a) {
     do {                                                                            \
         if (ctx->listValid) hipLaunchKernelGGL(K<true>, dim3(g), dim3(kBlock), 0, ctx->stream, a); \
         else hipLaunchKernelGGL(K<false>, dim3(g), dim3(kBlock), 0, ctx->stream, a); \
+    } while (0)
+// Lanes per particle of the batched operators (kern_common.h, NbrBatch).  At
+// 8,192 particles 16 lanes each make two wavefronts per SIMD of the chip, at
+// 81,920 four lanes make five: below these lines the kernels wait on one
+// particle's chain of neighbours and more lanes shorten it, above them the
+// lanes' repeated adds cost more issue slots than they hide.  Us per launch
+// with 1 / 4 / 16 lanes at 1,728, 44,100 and 216,000 particles: viscosity 47 /
+// 18 / 9.3, 51 / 32 / 44, 162 / 122 / 191; PND 42 / 17 / 10, 49 / 31 / 49, 101
+// / 103 / 205; pressure gradient 24 / 10 / 5.8, 26 / 18 / 23, 66 / 61 / 96;
+// wall viscosity 48 / 19 / 11, 46 / 28 / 43, 102 / 68 / 126.
+static int lanesPerParticle(const Ctx* ctx) { return ctx->N <= 8192 ? 16 : (ctx->N <= 81920 ? 4 : 0); }
+#define LX(K, LIST, l, b, g_) \
+    hipLaunchKernelGGL((K<LIST, l, b, g_>), dim3(gridFor(ctx->N, kBlock / (l))), dim3(kBlock), 0, ctx->stream, a)
+// from a bucket walk
+#define LWB(K)                                              \
+    do {                                                    \
+        if (lanesPerParticle(ctx) == 16) LX(K, false, 16, 1, 1); \
+        else if (lanesPerParticle(ctx) == 4) LX(K, false, 4, 1, 1); \
+        else LX(K, false, 1, 1, 1);                         \
+    } while (0)
+// from the list if there is one; l, b, g_: lanes, terms side by side and
+// gathers in flight of a launch that fills the chip in 3-D.  The short rows of
+// a 2-D case (28 neighbours, 12 in the small radius) would spend a large part
+// of a wider batch past their end: one lane and batches of four there.
+#define LTB(K, l, b, g_)                                    \
+    do {                                                    \
+        if (!ctx->listValid) LWB(K);                        \
+        else if (lanesPerParticle(ctx) == 16) LX(K, true, 16, 2, 2); \
+        else if (lanesPerParticle(ctx) == 4) LX(K, true, 4, 2, 2);   \
+        else if ((int)P.dim == 2) LX(K, true, 1, 2, 4);     \
+        else LX(K, true, l, b, g_);                         \
     } while (0)
 #define LW(K) hipLaunchKernelGGL(K<false>, dim3(g), dim3(kBlock), 0, ctx->stream, a)
 
@@ -2310,24 +2606,40 @@ int launchCompaction(Ctx* ctx) {
 
 // extrapolatePressParticlesWallDummy (src/MpsPressure.cpp:792-846); in place
 // is safe: only wall / dummy slots are written and only fluid slots are read.
-template <bool LIST>
-__global__ void kExtrapolateWallDummy2(KArgs a) {
-    const int i = slotId();
+template <bool LIST, int L, int B, int G>
+__global__ __launch_bounds__(kBlock) void kExtrapolateWallDummy2(KArgs a) {
+    const int i = groupSlot<L>();
     if (!live(a, i)) return;
     const mps_params& P = a.P;
-    const int t = a.I[ITYPE][i];
-    if (!(t == P.dummy_wall || (P.mps_type == MPS_WEAKLY && t == P.wall))) return;
+    const int ti = a.I[ITYPE][i];
+    if (!(ti == P.dummy_wall || (P.mps_type == MPS_WEAKLY && ti == P.wall))) return;
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     double ni = 0.0, pr = 0.0;
-    forNbrsPosS<LIST>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        if (d2 < P.re_s2 && a.I[ITYPE][j] == P.fluid) {
-            const double wS = wgt(sqrt(d2), P.re_s, P.weight_type);
-            ni += wS;
-            pr += (a.D[DPRESS][j] - rhoOf(a, j) * (P.gravity[0] * v0 + P.gravity[1] * v1 + P.gravity[2] * v2)) * wS;
+    auto press = [&](int j) { return a.D[DPRESS][j]; };
+    forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, press, [&](const auto& t) {
+        constexpr int nb = std::remove_reference_t<decltype(t)>::B;
+        double d[nb], w[nb], v0[nb], v1[nb], v2[nb];
+        bool ok[nb], any = false;
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            v0[b] = t.x[b] - xi;
+            v1[b] = t.y[b] - yi;
+            v2[b] = t.z[b] - zi;
+            const double d2 = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & (a.I[ITYPE][t.j[b]] == P.fluid);
+            any = any | ok[b];
+            d[b] = sqrt(d2);
+        }
+        if (noneInWave(any)) return;
+        wgtBatch(d, P.re_s, P.weight_type, w);
+#pragma unroll
+        for (int b = 0; b < nb; b++) {
+            const double p = t.e[b] - rhoOf(a, t.j[b]) * (P.gravity[0] * v0[b] + P.gravity[1] * v1[b] + P.gravity[2] * v2[b]);
+            addOrdered<L>(ni, ok[b] ? w[b] : 0.0);
+            addOrdered<L>(pr, ok[b] ? p * w[b] : 0.0);
         }
     });
+    if (groupLaneId<L>() != 0) return;
     if (pr < 0.0) return;
     a.D[DPRESS][i] = (ni > 0) ? pr / ni : pr;
 }
@@ -2371,15 +2683,17 @@ int launchOp(Ctx* ctx, const char* op) {
             if (!ctx->V4) MPS_HIP(hipMalloc(&ctx->V4, sizeof(double4) * (size_t)ctx->N));
             a.V4 = ctx->V4;
             hipLaunchKernelGGL(kPackVel, dim3(g), dim3(kBlock), 0, ctx->stream, a, ctx->V4);
-            L1(kViscosity<true>);
+            // four lanes also at the largest: neighbouring entries share cache
+            // lines (1.73M particles: 995 us, one lane 1,185)
+            LTB(kViscosity, 4, 4, 4);
         }
-        else if (ctx->P.domain_type_bc == 1) LW(kViscosity);   // walk through the periodic ghosts
+        else if (ctx->P.domain_type_bc == 1) LWB(kViscosity);   // walk through the periodic ghosts
         else hipLaunchKernelGGL(kViscosityWalk, dim3(gridFor(ctx->N, kWave)), dim3(kWave), 0, ctx->stream, a);
     }
     else if (o == "add_gravity") L1(kAddGravity);
     else if (o == "prediction") L1(kPrediction);
     else if (o == "collision") {
-        if (P.collision_type == MPS_COLLISION_PC) LT(kCollisionPC);
+        if (P.collision_type == MPS_COLLISION_PC) LTB(kCollisionPC, 2, 2, 4);
         else LT(kCollisionDPC);
         hipLaunchKernelGGL(kApplyDvel, dim3(g), dim3(kBlock), 0, ctx->stream, a, P.collision_type == MPS_COLLISION_DPC ? 1 : 0);
         if (P.collision_type == MPS_COLLISION_DPC) ctx->listValid = false;
@@ -2391,15 +2705,15 @@ int launchOp(Ctx* ctx, const char* op) {
             if (rc) return rc;
         }
     } else if (o == "update_near_mesh") L1(kUpdateNear);
-    else if (o == "wall_npcd") LT(kWallNPCD);
-    else if (o == "correction_matrix") LT(kCorrectionMatrix);
+    else if (o == "wall_npcd") LTB(kWallNPCD, 2, 2, 4);
+    else if (o == "correction_matrix") LTB(kCorrectionMatrix, 1, 2, 4);
     else if (o == "initial_pnd") LT(kInitialPnd);
-    else if (o == "pnd_neigh_npcd") LT(kPndNeighNPCD);
+    else if (o == "pnd_neigh_npcd") LTB(kPndNeighNPCD, 2, 2, 4);
     else if (o == "pnd_diffusive") {
-        LT(kPndDiffusive);
+        LTB(kPndDiffusive, 2, 2, 4);
         if (P.wall_type == MPS_WALL_POLYGON) LT(kWallPndDiffusive);
         L1(kUpdatePnd);
-        LT(kMeanPndWDS);
+        LTB(kMeanPndWDS, 2, 2, 4);
         L1(kMeanPndWDSFinish);
     } else if (o == "mean_pnd") {
         if (P.wall_type == MPS_WALL_POLYGON) LT(kMeanWallPnd);
@@ -2422,13 +2736,13 @@ int launchOp(Ctx* ctx, const char* op) {
     else if (o == "normal_particles") LT(kNormalParticles);
     else if (o == "wall_normal_particles") LT(kWallNormalParticles);
     else if (o == "press_explicit") L1(kPressExplicit);
-    else if (o == "vel_divergence") LT(kVelDivergence);
+    else if (o == "vel_divergence") LTB(kVelDivergence, 2, 2, 4);
     else if (o == "wall_vel_divergence") LT(kWallVelDivergence);
-    else if (o == "extrapolate_wall_dummy") LT(kExtrapolateWallDummy2); else if (o == "press_gradient") LT(kPressGradient);
-    else if (o == "wall_press_gradient") LT(kWallPressGradient);
-    else if (o == "prediction_press_gradient") LT(kPredPressGradient);
-    else if (o == "prediction_wall_press_gradient") LT(kPredWallPressGradient);
-    else if (o == "wall_viscosity") LT(kWallViscosity);
+    else if (o == "extrapolate_wall_dummy") LTB(kExtrapolateWallDummy2, 2, 2, 4); else if (o == "press_gradient") LTB(kPressGradient, 2, 2, 4);
+    else if (o == "wall_press_gradient") LTB(kWallPressGradient, 2, 2, 4);
+    else if (o == "prediction_press_gradient") LTB(kPredPressGradient, 2, 2, 4);
+    else if (o == "prediction_wall_press_gradient") LTB(kPredWallPressGradient, 2, 2, 4);
+    else if (o == "wall_viscosity") LTB(kWallViscosity, 2, 2, 4);
     else if (o == "correction") {
         hipLaunchKernelGGL(kCorrection, dim3(g), dim3(kBlock), 0, ctx->stream, a);   // g <= redCap partials
         hipLaunchKernelGGL(kVelMaxFinish, dim3(1), dim3(1024), 0, ctx->stream, a, g);
@@ -2438,8 +2752,8 @@ int launchOp(Ctx* ctx, const char* op) {
             LW(kShift1);
             hipLaunchKernelGGL(kCommitStaged, dim3(g), dim3(kBlock), 0, ctx->stream, a, (int)DU);
         } else if (P.shifting_type == 2) {
-            LW(kShift2Conc);
-            LW(kShift2Grad);
+            LWB(kShift2Conc);
+            LWB(kShift2Grad);
             hipLaunchKernelGGL(kCommitStaged, dim3(g), dim3(kBlock), 0, ctx->stream, a, (int)DX);
             if (P.wall_type == MPS_WALL_POLYGON) {
                 LW(kShift2Wall);
@@ -2447,7 +2761,7 @@ int launchOp(Ctx* ctx, const char* op) {
             }
             ctx->listValid = false;
         }
-    } else if (o == "wall_dummy_velocity") LW(kWallDummyVelocity);
+    } else if (o == "wall_dummy_velocity") LWB(kWallDummyVelocity);
     else {
         ctx->err = "unknown operator " + o;
         return MPS_E_ARG;

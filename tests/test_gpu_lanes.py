@@ -1,0 +1,95 @@
+"""Operators at every number of lanes per particle (needs a gfx950 GPU).
+
+The neighbour sums run with 16, 4 or fewer lanes per particle, chosen by the
+particle count.  Their terms are added in the reference's order whatever the
+split, so each operator equals the oracle bit for bit; the sizes here lie on
+both sides of the lines between the splits and leave wavefronts and batches
+partly filled.
+"""
+import numpy as np
+import pytest
+
+from polymps_amd import configs
+from tests.parity_util import check, new_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def _velocity(n, seed, dim):
+    v = 2.0 * configs.splitmix64_uniform(seed, 3 * n).reshape(n, 3) - 1.0
+    if dim == 2:
+        v[:, 2] = 0.0
+    return v.reshape(-1)
+
+
+def _dam3d(nx, ny, nz):
+    l0 = 0.6 / nx
+    b = (nx * l0, ny * l0, nz * l0)
+    # a strong jitter: some pairs closer than the collision distance, ragged neighbour counts
+    w = configs.dam3d_inc(l0=l0, tank=(1.61, b[1], 2.0 * b[2]), block=b, seed=9, jitter=0.2)
+    w.vel = _velocity(w.n, 31, 3)
+    return w
+
+
+@pytest.mark.parametrize("shape", [(7, 5, 3), (24, 6, 12), (32, 16, 16), (31, 17, 16), (64, 32, 40), (65, 32, 40)])
+def test_polygon_wall_operators(built, shape):
+    w = _dam3d(*shape)
+    print(f"lanes {shape} {w.n}", flush=True)
+    g, o = new_pair(w)
+
+    def both(gop, oop, fields):
+        g.call(gop)
+        o.call(oop)
+        check(g, o, fields, f"{w.n} {gop}")
+
+    g.call("bucket_update"); o.call("update_buckets")
+    both("viscosity", "viscosity", ["acc"])          # bucket walk
+    g.call("build_neighbor_list")
+    both("viscosity", "viscosity", ["acc"])          # list
+    both("mesh_closest_point", "closest_point", ["riw2", "mirror"])
+    both("mesh_update_near", "update_near_mesh", ["near_wall"])
+    both("wall_npcd", "wall_npcd", ["npcd"])
+    both("pnd_neigh_npcd", "pnd_neigh_npcd", ["num_neigh", "pnd_small", "npcd", "npcd2"])
+    p = 1e4 * configs.splitmix64_uniform(77, w.n)
+    g.set("press", p); o.set("press", p)
+    both("correction_matrix", "correction_matrix", ["cm1", "cm2", "cm3"])
+    both("vel_divergence", "vel_divergence", [])
+    o.call("wall_vel_divergence")
+    check(g, o, ["div_u"], f"{w.n} vel_divergence")
+    both("press_gradient", "press_gradient", ["acc"])
+    both("wall_press_gradient", "wall_press_gradient", ["acc", "force_wall"])
+    both("wall_viscosity", "wall_viscosity", ["acc", "force_wall"])
+    both("collision", "collision", ["vel"])
+    assert np.any(g.get("vel") != w.vel)   # some pairs collided
+
+
+@pytest.mark.parametrize("l0", [0.02, 0.005, 0.0025, 0.00125])
+def test_particle_wall_operators(built, l0):
+    w = configs.dam2d_wc_long(l0=l0, jitter=0.1)
+    w.vel = _velocity(w.n, 32, 2)
+    print(f"lanes 2-D {w.n}", flush=True)
+    g, o = new_pair(w)
+
+    def both(gop, oops, fields):
+        g.call(gop)
+        for op in oops:
+            o.call(op)
+        check(g, o, fields, f"{w.n} {gop}")
+
+    g.call("bucket_update"); o.call("update_buckets")
+    g.call("build_neighbor_list")
+    both("viscosity", ["viscosity"], ["acc"])
+    both("pnd_neigh_npcd", ["pnd_neigh_npcd"], ["num_neigh", "pnd_small"])
+    p = 1e4 * configs.splitmix64_uniform(78, w.n)
+    pn = g.get("pnd_small")   # a PND as the step leaves it
+    for s in (g, o):
+        s.set("press", p)
+        s.set("pndi", pn)
+    both("correction_matrix", ["correction_matrix"], ["cm1", "cm2", "cm3"])
+    both("pnd_diffusive", ["pnd_diffusive", "update_pnd", "mean_pnd_wall_dummy_surface"], ["pndi", "div_u", "diffusive"])
+    both("update_bc", ["update_bc"], ["bc"])
+    both("extrapolate_wall_dummy", ["extrapolate_wall_dummy"], ["press"])
+    both("press_gradient", ["press_gradient"], ["acc"])
+    both("collision", ["collision"], ["vel"])
+    both("wall_dummy_velocity", ["wall_dummy_velocity"], ["vel"])   # bucket walks from here
+    both("shifting", ["shifting"], ["pos"])
