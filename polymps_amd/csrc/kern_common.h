@@ -682,6 +682,19 @@ __device__ __forceinline__ void walkGroup(const KArgs& a, int i, double x, doubl
     }
 }
 
+// Lanes of the own group with the predicate set, as a mask of L bits, and
+// how many of them come before this lane.
+template <int L>
+__device__ __forceinline__ unsigned long long groupBallot(bool c) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(c);
+    if constexpr (L == 64) return m;
+    else return (m >> (threadIdx.x & 63 & ~(L - 1))) & ((1ull << L) - 1ull);
+}
+template <int L>
+__device__ __forceinline__ int groupRank(unsigned long long m) {
+    return __popcll(m & ((1ull << groupLaneId<L>()) - 1ull));
+}
+
 // Neighbours of slot i in batches: from the list (SMALL: the small-radius
 // one, for operators whose radii are at most re_s or the collision distance)
 // or from a bucket walk, whose candidates come one per lane.

@@ -244,60 +244,71 @@ __global__ __launch_bounds__(kWave) void kBuildList(KArgs a, unsigned* mask, int
     if (SMALL) cntS[i] = totalS;
 }
 
-// Lists of the particles whose candidate rows overflowed the mask windows,
-// from a per-particle walk in walk order (no window limit), both radii.
-__global__ __launch_bounds__(256) void kFixList(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS,
-                                                const int* fixList, double r2, double r2s, const int* gate) {
-    if (gate != nullptr && *gate == 0) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.is[I_FIXCNT]) return;
-    const int i = fixList[t];
+// The lists of one particle from a bucket walk by L lanes: each chunk of L
+// candidates is tested side by side and the hits are written at their ranks,
+// so the entries keep the walk order.  Periodic domains keep the ghost shift
+// of an entry in its bits 30-31 (listBatches) and have one list only.
+template <int L>
+__device__ __forceinline__ void listOfParticle(const KArgs& a, int i, int* nbr, int* cnt, int* nbrS, int* cntS,
+                                               double r2, double r2s) {
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     const size_t N = a.N;
+    const bool periodic = periodicDomain(a.P);
     int c = 0, cs = 0;
-    walkCellsPos(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
+    walkGroup<L>(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj, int pbc, bool ok) {
         const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
         const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        if (!(d2 < r2)) return;
-        if (c < a.K) nbr[(size_t)c * N + i] = j;
-        c++;
-        if (d2 < r2s) {
-            if (cs < a.KS) nbrS[(size_t)cs * N + i] = j;
-            cs++;
-        }
+        const bool hit = ok & (d2 < r2);
+        const unsigned long long m = groupBallot<L>(hit);
+        if (m == 0) return;
+        const int k = c + groupRank<L>(m);
+        if (hit && k < a.K) nbr[(size_t)k * N + i] = (int)((unsigned)j | (pbc < 0 ? 1u << 30 : (pbc > 0 ? 2u << 30 : 0u)));
+        c += __popcll(m);
+        if (nbrS == nullptr) return;
+        const bool hitS = hit & (d2 < r2s);
+        const unsigned long long ms = groupBallot<L>(hitS);
+        const int ks = cs + groupRank<L>(ms);
+        if (hitS && ks < a.KS) nbrS[(size_t)ks * N + i] = j;
+        cs += __popcll(ms);
     });
+    if (groupLaneId<L>() != 0) return;
     if (c > a.K) { atomicMax(&a.is[I_OVERFLOW], c); c = a.K; }
     if (cs > a.KS) { atomicMax(&a.is[I_OVERFLOW], cs); cs = a.KS; }
     cnt[i] = c;
-    cntS[i] = cs;
+    if (nbrS != nullptr) cntS[i] = cs;
 }
 
-// Periodic domains: the list is built by a per-particle walk through the
-// ghost layers (walkCellsPeriodic); each entry keeps its ghost shift in bits
-// 30-31 for listNbrsQ.
-__global__ __launch_bounds__(256) void kBuildListWalk(KArgs a, int* nbr, int* cnt, double r2) {
-    const int i = slotId();
+// Lists of the particles whose candidate rows overflowed the mask windows,
+// one wavefront each: few particles, which one lane apiece would walk ~1,400
+// candidates of 27 buckets one by one.  nbrS null: the large list only.
+constexpr int kQueueBlocks = 1024;   // blocks of a launch over a queue of unknown length
+__global__ __launch_bounds__(256) void kFixList(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS,
+                                                const int* fixList, double r2, double r2s, const int* gate) {
+    if (gate != nullptr && *gate == 0) return;
+    const int n = a.is[I_FIXCNT];
+    for (int t = groupSlot<64>(); t < n; t += gridDim.x * (blockDim.x / 64))
+        listOfParticle<64>(a, fixList[t], nbr, cnt, nbrS, cntS, r2, r2s);
+}
+
+// Lists of every particle by group walks (L lanes per particle), with the
+// packed positions: periodic domains (their stencil goes through the ghost
+// layers) and systems too small to fill the chip with kBuildList, whose
+// wavefronts of 64 particles go through their candidates one by one.
+template <int L>
+__global__ __launch_bounds__(256) void kBuildListGroup(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS, double r2,
+                                                       double r2s, const int* gate) {
+    if (gate != nullptr && *gate == 0) return;
+    const int i = groupSlot<L>();
     if (i >= a.N) return;
-    const double xi = PX(i), yi = PY(i), zi = PZ(i);
-    a.P4[i] = make_double4(xi, yi, zi, (double)a.I[ITYPE][i]);
+    if (groupLaneId<L>() == 0) a.P4[i] = make_double4(PX(i), PY(i), PZ(i), (double)a.I[ITYPE][i]);
     if (!live(a, i)) {
-        cnt[i] = 0;
+        if (groupLaneId<L>() == 0) {
+            cnt[i] = 0;
+            if (nbrS != nullptr) cntS[i] = 0;
+        }
         return;
     }
-    const size_t N = a.N;
-    int c = 0;
-    walkCellsPeriodic(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj, int pbc) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        if (!(d2 < r2)) return;
-        if (c < a.K) nbr[(size_t)c * N + i] = (int)((unsigned)j | (pbc < 0 ? 1u << 30 : (pbc > 0 ? 2u << 30 : 0u)));
-        c++;
-    });
-    if (c > a.K) {
-        atomicMax(&a.is[I_OVERFLOW], c);
-        c = a.K;
-    }
-    cnt[i] = c;
+    listOfParticle<L>(a, i, nbr, cnt, nbrS, cntS, r2, r2s);
 }
 
 // Start slot of stencil row r of a particle in bucket (ix, iy, iz), or -1
@@ -2341,8 +2352,22 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
         r2 = (std::sqrt(r2) + skin) * (std::sqrt(r2) + skin);
         r2s = (std::sqrt(r2s) + skin) * (std::sqrt(r2s) + skin);
     }
-    if (P.domain_type_bc == 1) {
-        hipLaunchKernelGGL(kBuildListWalk, dim3(g), dim3(kBlock), 0, ctx->stream, a, ctx->nbr, ctx->nbrCnt, r2);
+    // Group walks for periodic domains, and where the particles do not fill
+    // the chip.  Us per build with both radii, masks and decode against group
+    // walks of 64 / 16 lanes: 110 / 11 / 18 at 1,728 particles, 124 / 42 / 41
+    // at 13,824, 165 / 119 / 97 at 44,100, 214 / 220 / 171 at 81,312, 231 /
+    // 339 / 253 at 125,000; 2-D 43 / 9 / 8 at 6,332, 55 / 69 / 36 at 85,292.
+    // (A caller's narrower mask_words asks for the mask path.)
+    const int lanes = lanesPerParticle(ctx);
+    if (P.domain_type_bc == 1 || (lanes != 0 && ctx->maskW == ctx->maskWAlloc)) {
+        int* const nS = P.domain_type_bc != 1 && small ? ctx->nbrS : nullptr;
+        int* const cS = nS ? ctx->nbrCntS : nullptr;
+        if (lanes == 16)
+            hipLaunchKernelGGL(kBuildListGroup<64>, dim3(gridFor(ctx->N, kBlock / 64)), dim3(kBlock), 0, ctx->stream, a,
+                               ctx->nbr, ctx->nbrCnt, nS, cS, r2, r2s, gate);
+        else
+            hipLaunchKernelGGL(kBuildListGroup<16>, dim3(gridFor(ctx->N, kBlock / 16)), dim3(kBlock), 0, ctx->stream, a,
+                               ctx->nbr, ctx->nbrCnt, nS, cS, r2, r2s, gate);
         MPS_HIP(hipGetLastError());
         ctx->listValid = true;
         return MPS_OK;
@@ -2372,8 +2397,8 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
         return MPS_E_UNSUPPORTED;
     }
 #undef M2L
-    hipLaunchKernelGGL(kFixList, dim3(g), dim3(kBlock), 0, ctx->stream, a, ctx->nbr, ctx->nbrCnt, ctx->nbrS,
-                       ctx->nbrCntS, ctx->fixList, r2, r2s, gate);
+    hipLaunchKernelGGL(kFixList, dim3(std::min(gridFor(ctx->N, 4), kQueueBlocks)), dim3(kBlock), 0, ctx->stream, a,
+                       ctx->nbr, ctx->nbrCnt, small ? ctx->nbrS : nullptr, ctx->nbrCntS, ctx->fixList, r2, r2s, gate);
     MPS_HIP(hipGetLastError());
     ctx->listValid = true;
     return MPS_OK;
@@ -2423,37 +2448,15 @@ __global__ __launch_bounds__(256) void kListRefresh(KArgs a, int* patch, double 
 }
 
 // The list of each queued particle from its own stencil walk, in walk order
-// (the order of kBuildList + kMaskToList).
+// (the order of kBuildList + kMaskToList), one wavefront per particle: of the
+// 216,000-particle dam break's a few hundred change their stencil centre in a
+// step (one lane each: 206 us per launch).
 __global__ __launch_bounds__(256) void kPatchList(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS, const int* patch,
                                                   double r2, double r2s) {
     if (a.is[I_REBUILD]) return;   // the whole list was rebuilt
-    const int t = slotId();
-    if (t >= a.is[I_PATCHCNT]) return;
-    const int i = patch[t];
-    const double xi = PX(i), yi = PY(i), zi = PZ(i);
-    const size_t N = a.N;
-    int c = 0, cs = 0;
-    walkCellsPos(a, i, xi, yi, zi, [&](int j, double xj, double yj, double zj) {
-        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
-        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-        if (!(d2 < r2)) return;
-        if (c < a.K) nbr[(size_t)c * N + i] = j;
-        c++;
-        if (d2 < r2s) {
-            if (cs < a.KS) nbrS[(size_t)cs * N + i] = j;
-            cs++;
-        }
-    });
-    if (c > a.K) {
-        atomicMax(&a.is[I_OVERFLOW], c);
-        c = a.K;
-    }
-    if (cs > a.KS) {
-        atomicMax(&a.is[I_OVERFLOW], cs);
-        cs = a.KS;
-    }
-    cnt[i] = c;
-    cntS[i] = cs;
+    const int n = a.is[I_PATCHCNT];
+    for (int t = groupSlot<64>(); t < n; t += gridDim.x * (blockDim.x / 64))
+        listOfParticle<64>(a, patch[t], nbr, cnt, nbrS, cntS, r2, r2s);
 }
 
 // Drops from a kept row the entries that lie outside the list radius at the
@@ -2524,8 +2527,9 @@ int launchListKeepRefresh(Ctx* ctx, double skin) {
     MPS_HIP(hipGetLastError());
     int rc = launchBuildList(ctx, 0.0, ctx->is + I_REBUILD);
     if (rc) return rc;
-    hipLaunchKernelGGL(kPatchList, dim3(g), dim3(kBlock), 0, ctx->stream, a, ctx->nbr, ctx->nbrCnt, ctx->nbrS,
-                       ctx->nbrCntS, ctx->patchList, listRadius2(ctx->P), listRadiusS2(ctx->P));
+    hipLaunchKernelGGL(kPatchList, dim3(std::min(gridFor(ctx->N, 4), kQueueBlocks)), dim3(kBlock), 0, ctx->stream, a,
+                       ctx->nbr, ctx->nbrCnt, ctx->nbrS, ctx->nbrCntS, ctx->patchList, listRadius2(ctx->P),
+                       listRadiusS2(ctx->P));
     // Below a skin of 0.04 l0 the extra entries are too few to upset the
     // consumers (PPE assembly 2.12 ms untightened at 0.04 l0 against 4.7 ms at
     // 0.06 l0) and the tightening's read of the whole list would cost more.
