@@ -504,7 +504,7 @@ int mps_create(mps_ctx** out, const mps_params* p, int n, int device) {
     MPS_HIP(hipMalloc(&ctx->is, sizeof(int) * NIS));
     ctx->redCap = std::max(kRedBlocks, gridFor(n, 256));
     MPS_HIP(hipMalloc(&ctx->red, sizeof(double) * (3 * ctx->redCap + 16)));
-    MPS_HIP(hipMalloc(&ctx->asmRed, sizeof(double) * (3 * ctx->redCap + 16)));
+    MPS_HIP(hipMalloc(&ctx->asmRed, sizeof(double) * 2 * (size_t)std::max(kRedBlocks, gridFor(n, 16))));
     if (p->fluid_type == 1) {   // granular phase: carried per-step fields, bed-level grid
         for (int q = 0; q < kNNCarriedCount; q++) MPS_HIP(hipMalloc(&ctx->DaltNN[q], nd));
         MPS_HIP(hipMalloc(&ctx->IaltPtype, ni));

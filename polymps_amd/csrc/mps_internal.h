@@ -247,6 +247,7 @@ struct Ctx {
     int lastPass2Iters = 8;          // iterations of the last solve's second refinement pass
     bool r0Fresh = false;        // cgR and asmRed hold b - A x of the current guess and its partials (assembly)
     bool r0FreshMixed = false;   // ... in the mixed solve's partial order (else the FP64 CG's, with 1/diag)
+    int asmBlocks = 0;           // blocks (partials) of the last assembly
     double* asmRed = nullptr;    // block partials of the assembly's first residual (no other kernel writes them)
     unsigned long long* red64 = nullptr;   // result of reduceCounts (allocated on first use)
     // solver kind of the last PPE assembly (MPS_SOLVER_* / precision), -1 when

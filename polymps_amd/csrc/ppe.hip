@@ -58,57 +58,66 @@ __device__ __forceinline__ void ppeWindowBegin(const KArgs& a, int i, int* sS, i
     const int iy = (int)((yi - P.domain_min[1]) * P.inv_bucket_side + KEPS);
     const int iz = (int)((zi - P.domain_min[2]) * P.inv_bucket_side + KEPS);
     const int w = threadIdx.x >> 6;
-    for (int r = 0; r < rows; r++) {
-        int s = 0, e = 0;
-        if (has) {
-            const int jz = ((int)P.dim == 3) ? iz - 1 + r / 3 : 0;
-            const int jy = iy - 1 + r % 3;
-            if (!(jz < 0 || jz >= P.num_buckets_z || jy < 0 || jy >= P.num_buckets_y)) {
-                const int row = jz * P.num_buckets_xy + jy * P.num_buckets_x;
-                int jx0 = ix - 1, jx1 = ix + 1;
-                if (jx0 < 0) jx0 = 0;
-                if (jx1 >= P.num_buckets_x) jx1 = P.num_buckets_x - 1;
-                if (jx0 <= jx1) {
-                    s = a.cellStart[row + jx0];
-                    e = a.cellStart[row + jx1 + 1];
-                }
-            }
+    // every row's range in flight at once, then the reductions
+    int rs[9], re[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        rs[r] = 0;
+        re[r] = 0;
+        const int jz = ((int)P.dim == 3) ? iz - 1 + r / 3 : 0;
+        const int jy = iy - 1 + r % 3;
+        const int jx0 = max(ix - 1, 0), jx1 = min(ix + 1, P.num_buckets_x - 1);
+        if (has && r < rows && jz >= 0 && jz < P.num_buckets_z && jy >= 0 && jy < P.num_buckets_y && jx0 <= jx1) {
+            const int row = jz * P.num_buckets_xy + jy * P.num_buckets_x;
+            rs[r] = a.cellStart[row + jx0];
+            re[r] = a.cellStart[row + jx1 + 1];
         }
-        const int mn = waveMinInt(e > s ? s : INT_MAX);
-        const int mx = waveMaxInt(e > s ? e : INT_MIN);
+    }
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        if (r >= rows) break;
+        const int mn = waveMinInt(re[r] > rs[r] ? rs[r] : INT_MAX);
+        const int mx = waveMaxInt(re[r] > rs[r] ? re[r] : INT_MIN);
         if ((threadIdx.x & 63) == 0) {
             ps[w][r] = mn;
             pe[w][r] = mx;
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        // per stencil row the union over the block; starts and ends ascend
+    if (threadIdx.x < 64) {
+        // lane r: row r's union over the block; then starts and ends ascend
         // with the row, so overlapping neighbours merge in one pass
-        int m = 0, W = 0;
-        for (int r = 0; r < rows; r++) {
-            int s = INT_MAX, e = INT_MIN;
-            for (int q = 0; q < (int)(blockDim.x >> 6); q++) {
-                s = min(s, ps[q][r]);
-                e = max(e, pe[q][r]);
+        int s = INT_MAX, e = INT_MIN;
+        if (threadIdx.x < rows)
+            for (int q = 0; q < kB / 64; q++) {
+                s = min(s, ps[q][threadIdx.x]);
+                e = max(e, pe[q][threadIdx.x]);
             }
-            if (s >= e) continue;
-            if (m > 0 && s <= sE[m - 1]) {
-                if (e > sE[m - 1]) {
-                    W += e - sE[m - 1];
-                    sE[m - 1] = e;
+        int m = 0, W = 0, last = 0;
+        for (int r = 0; r < rows; r++) {
+            const int sr = __builtin_amdgcn_readlane(s, r), er = __builtin_amdgcn_readlane(e, r);
+            if (sr >= er) continue;
+            if (m > 0 && sr <= last) {
+                if (er > last) {
+                    W += er - last;
+                    last = er;
                 }
             } else {
-                sS[m] = s;
-                sE[m] = e;
-                sB[m] = W;
-                W += e - s;
+                if (threadIdx.x == 0) {
+                    sS[m] = sr;
+                    sB[m] = W;
+                }
+                W += er - sr;
+                last = er;
                 m++;
             }
+            if (threadIdx.x == 0) sE[m - 1] = last;
         }
-        sB[m] = W;
-        sM = m;
-        sOut = (W > kWinMax || periodicDomain(P)) ? 1 : 0;
+        if (threadIdx.x == 0) {
+            sB[m] = W;
+            sM = m;
+            sOut = (W > kWinMax || periodicDomain(P)) ? 1 : 0;
+        }
     }
     __syncthreads();
 }
@@ -420,6 +429,233 @@ __global__ __launch_bounds__(256) void kPpeAssemble(KArgs a, double* val, unsign
         }
     }
     // the partials kTrueResidualFinish (|r|^2, |b|^2) or kCgStartFinish (|b|^2, |r|^2) sums
+    if (RES) {
+        if (bFirst) writePartials(a, bn2, rn2);
+        else writePartials(a, rn2, bn2);
+    }
+}
+// ----------------------------------------- assembly, several lanes per row
+// The window table of each 256-row block alone (kPpeAssemble makes it on the
+// way; the group assembly's workgroups hold a part of such a block).
+__global__ __launch_bounds__(256) void kPpeWindow(KArgs a, int* win) {
+    __shared__ int wS[9], wE[9], wB[10], wM, wOut;
+    ppeWindowBegin(a, slotId(), wS, wE, wB, wM, wOut);
+    if (threadIdx.x != 0) return;
+    int* t = win + (size_t)blockIdx.x * kWinStride;
+    t[0] = wOut;
+    t[1] = wM;
+    for (int k = 0; k < wM; k++) t[2 + k] = wS[k];
+    for (int k = 0; k <= wM; k++) t[11 + k] = wB[k];
+}
+
+// One row by L lanes, each with the neighbours c0 + l of a chunk: what the
+// row's entries cost (gathers, a square root and a division, the window
+// search) runs side by side, the sums are added in order (addOrdered), and
+// an entry finds its place in the row, its column step and its window step
+// from the ballots of the entries before it.  The result is assembleRow's.
+template <bool LIST, bool TRANS, bool RES, int L>
+__device__ __forceinline__ void assembleRowGroup(const KArgs& a, int i, double* val, unsigned short* col, int* esc,
+                                                 int* cnt, double* diag, double* b, float* val32, float* diag32,
+                                                 float* invd32, double* invd64, double* x, double* r, double& rn2,
+                                                 double& bn2, unsigned char* lc8, unsigned short* lcEsc, const int* wS,
+                                                 const int* wB, int wM, bool& outside, int& nEsc, int& nLc) {
+    const mps_params& P = a.P;
+    const int l = groupLaneId<L>();
+    const bool lv = live(a, i);
+    const int bci = lv ? a.I[IBC][i] : P.other;
+    if (!lv || bci == P.other || bci == P.surface) {
+        if (l != 0) return;
+        cnt[i] = 0; diag[i] = 1.0; b[i] = 0.0;
+        if (invd32) { invd32[i] = 1.0f; diag32[i] = 1.0f; }
+        if (invd64) invd64[i] = 1.0;
+        if (RES) {
+            if (lv) {
+                const double ri = 0.0 - 1.0 * x[i];
+                r[i] = ri;
+                rn2 = ri * ri;
+            } else {
+                x[i] = 0.0;
+                r[i] = 0.0;
+            }
+        }
+        return;
+    }
+    const bool pw = P.wall_type == MPS_WALL_PARTICLE;
+    const double xi = a.D[DX][i], yi = a.D[DY][i], zi = a.D[DZ][i];
+    const double mx = a.D[DMX][i], my = a.D[DMY][i], mz = a.D[DMZ][i];
+    const double rho = phaseDensity(a, i);
+    const double farWall2 = 4.0 * P.re_l2;   // assembleRow
+    const int* __restrict__ BC = a.I[IBC];
+    const double* __restrict__ RIW2 = a.D[DRIW2];
+    const int KE = ellWidth(a.K);
+    const bool periodic = periodicDomain(P);
+    const bool flags = LIST && a.p4Flags;
+    const int base = threadIdx.x & 63 & ~(L - 1);   // lane 0 of the group in its wavefront
+    double sum = 0.0, rhs = 0.0, ax = 0.0;
+    int c = 0, ne = 0, nle = 0, prev = -1, prevLc = -1;
+    bool full = false;
+    auto guess = [x](int j) { return RES ? x[j] : 0.0; };
+    forBatches<LIST, false, L, 1, 2>(a, i, xi, yi, zi, guess, [&](const auto& t) {
+        const int j = t.j[0];
+        const double xj = t.x[0], yj = t.y[0], zj = t.z[0];
+        const double v0 = xj - xi, v1 = yj - yi, v2 = zj - zi;
+        const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+        const bool in = t.ok[0] & (d2 < P.re_l2);
+        if (noneInWave(in)) return;
+        double d2T = d2;
+        int pbc = 0;
+        if (TRANS && periodic) {
+            const int pd = P.periodic_dir[0] ? 0 : (P.periodic_dir[1] ? 1 : 2);
+            const double raw = a.D[DX + pd][j], sh = (pd == 0) ? xj : ((pd == 1) ? yj : zj);
+            pbc = sh > raw ? 1 : (sh < raw ? -1 : 0);
+            if (pbc != 0) {
+                const double u0 = (xi + (-pbc) * P.periodic_length[0]) - a.D[DX][j];
+                const double u1 = (yi + (-pbc) * P.periodic_length[1]) - a.D[DY][j];
+                const double u2 = (zi + (-pbc) * P.periodic_length[2]) - a.D[DZ][j];
+                d2T = u0 * u0 + u1 * u1 + u2 * u2;
+            }
+        }
+        const double w0 = xj - mx, w1 = yj - my, w2 = zj - mz;
+        const double dm2 = w0 * w0 + w1 * w1 + w2 * w2;
+        const double wL = wgt(sqrt(d2), P.re_l, P.weight_type);
+        const double mij = wL * P.coeff_ppe;
+        const bool okRow = in & ((d2 < dm2) | pw);
+        const bool dummy = nbrType(a, t, 0) == P.dummy_wall;
+        const bool dRow = okRow & dummy;
+        if (!noneInWave(dRow)) {
+            double pgh = 0.0;
+            if (dRow) pgh = P.coeff_ppe * (rhoOf(a, j) * (v0 * P.gravity[0] + v1 * P.gravity[1] + v2 * P.gravity[2]) * wL);
+            addOrdered<L>(rhs, dRow ? -pgh : 0.0);
+        }
+        addOrdered<L>(sum, okRow && !dummy ? -mij : 0.0);
+        const int fj = flags ? p4FlagBits(t.w[0]) : 0;
+        const bool innerJ = in && (flags ? (fj & 1) != 0 : BC[j] == P.inner);
+        bool put = false;
+        if (!TRANS) {
+            put = okRow && !dummy && innerJ;
+        } else if (innerJ) {
+            put = pw || (flags ? (fj & 2) != 0 : RIW2[j] >= farWall2);
+            if (!put) {
+                const double ix = xi + (-pbc) * P.periodic_length[0], iy = yi + (-pbc) * P.periodic_length[1],
+                             iz = zi + (-pbc) * P.periodic_length[2];
+                const double u0 = ix - a.D[DMX][j], u1 = iy - a.D[DMY][j], u2 = iz - a.D[DMZ][j];
+                put = d2T < u0 * u0 + u1 * u1 + u2 * u2;
+            }
+        }
+        put = put && !full;
+        // the entry's place and the entry before it
+        const unsigned long long below = (1ull << l) - 1ull;
+        const unsigned long long m = groupBallot<L>(put);
+        const int cc = c + __popcll(m & below);
+        const unsigned long long lower = m & below;
+        const int src = lower ? 63 - __builtin_clzll(lower) : 0;
+        const int pj = __shfl(j, base + src, 64);
+        const int dj = j - (lower ? pj : prev);
+        const bool delta = (lower != 0 || prev >= 0) && dj > 0 && dj < 65536;
+        const unsigned long long me = groupBallot<L>(put && !delta);
+        const int ke = ne + __popcll(me & below);
+        bool fits = put && cc < a.K && (delta || ke < kPpeEsc);
+        const unsigned long long bad = groupBallot<L>(put && !fits);
+        if (bad) {   // the row ends before its first entry that does not fit (reported as a capacity error)
+            fits = fits && l < __builtin_ctzll(bad);
+            full = true;
+        }
+        const unsigned long long ms = groupBallot<L>(fits);
+        double mv = mij;
+        if (TRANS && d2T != d2) mv = wgt(sqrt(d2T), P.re_l, P.weight_type) * P.coeff_ppe;
+        int lc = -1;
+        if (lc8) {
+            for (int k = 0; k < wM; k++) {
+                const int S = wS[k], B0 = wB[k];
+                if (j >= S && j - S < wB[k + 1] - B0) lc = B0 + (j - S);
+            }
+            const int pl = __shfl(lc, base + src, 64);
+            const int plc = lower ? pl : prevLc;
+            const int dl = lc - plc;
+            const bool step = plc >= 0 && lc >= 0 && dl > 0 && dl < 256;
+            const unsigned long long ml = groupBallot<L>(fits && !step);
+            if (fits) {
+                if (lc < 0) outside = true;
+                if (!step) {
+                    const int kl = nle + __popcll(ml & below);
+                    if (lc >= 0 && kl < kLcEsc) lcEsc[ellElem(kl, i, kLcEsc)] = (unsigned short)lc;
+                    else outside = true;
+                }
+                lc8[(ellElem(cc >> 3, i, KE >> 3) << 3) | (size_t)(cc & 7)] = (unsigned char)(step ? dl : 0);
+            }
+            nle += __popcll(ml);
+        }
+        if (fits) {
+            val[ellIdx64(cc, i, KE)] = mv;
+            const size_t e4 = ellIdx4(cc, i, KE);
+            if (val32) val32[e4] = (float)mv;
+            col[e4] = delta ? (unsigned short)dj : (unsigned short)0;
+            if (!delta) esc[(size_t)ke * a.N + i] = j;
+        }
+        if (RES) addOrdered<L>(ax, fits ? mv * t.e[0] : 0.0);
+        c += __popcll(ms);
+        ne += __popcll(me & ms);
+        if (ms) {
+            const int last = base + 63 - __builtin_clzll(ms);
+            prev = __shfl(j, last, 64);
+            prevLc = __shfl(lc, last, 64);
+        }
+    });
+    if (l != 0) return;
+    if (full) atomicMax(&a.is[I_OVERFLOW], a.K + 1);
+    nEsc = ne;
+    nLc = nle;
+    sum -= P.alpha_compressibility * rho / (P.time_step * P.time_step);
+    if (P.mps_type == MPS_IMPLICIT_PND_DIVU)
+        rhs += -P.coeff_ppe_source * rho * (a.D[DPNDKI][i] - P.pnd_small_zero) +
+               (1.0 - P.relax_pnd) * rho * a.D[DDIVU][i] / P.time_step;
+    else
+        rhs += -P.coeff_ppe_source * rho * (a.D[DPNDSMALL][i] - P.pnd_small_zero);
+    cnt[i] = c;
+    diag[i] = sum;
+    b[i] = rhs;
+    if (invd32) {
+        invd32[i] = (sum != 0.0) ? (float)(1.0 / sum) : 1.0f;
+        diag32[i] = (float)sum;
+    }
+    if (invd64) invd64[i] = (sum != 0.0) ? 1.0 / sum : 1.0;
+    if (RES) {
+        const double ri = rhs - (sum * x[i] + ax);
+        r[i] = ri;
+        rn2 = ri * ri;
+        bn2 = rhs * rhs;
+    }
+}
+
+template <bool LIST, bool TRANS, bool RES, int L>
+__global__ __launch_bounds__(256) void kPpeAssembleGroup(KArgs a, double* val, unsigned short* col, int* esc, int* cnt,
+                                                         double* diag, double* b, float* val32, float* diag32,
+                                                         float* invd32, double* invd64, double* x, double* r,
+                                                         int bFirst, unsigned char* lc8, unsigned short* lcEsc,
+                                                         int* win) {
+    __shared__ int wS[9], wB[10], wM;
+    const int i = groupSlot<L>();
+    int* const t = lc8 ? win + (size_t)(blockIdx.x / L) * kWinStride : nullptr;   // 256 / L rows per workgroup
+    if (lc8) {
+        if (threadIdx.x < 9) wS[threadIdx.x] = t[2 + threadIdx.x];
+        if (threadIdx.x < 10) wB[threadIdx.x] = t[11 + threadIdx.x];
+        if (threadIdx.x == 0) wM = t[1];
+        __syncthreads();
+    }
+    double rn2 = 0.0, bn2 = 0.0;
+    bool outside = false;
+    int nEsc = 0, nLc = 0;
+    if (i < a.N)
+        assembleRowGroup<LIST, TRANS, RES, L>(a, i, val, col, esc, cnt, diag, b, val32, diag32, invd32, invd64, x, r,
+                                              rn2, bn2, lc8, lcEsc, wS, wB, lc8 ? wM : 0, outside, nEsc, nLc);
+    nEsc = waveSumInt(nEsc);
+    nLc = waveSumInt(nLc);
+    const bool out = lc8 && __builtin_amdgcn_ballot_w64(outside) != 0;
+    if ((threadIdx.x & 63) == 0) {
+        if (nEsc) atomicAdd(&a.is[I_NESC], nEsc);
+        if (nLc) atomicAdd(&a.is[I_NLCESC], nLc);
+        if (out) atomicOr(t, 1);
+    }
     if (RES) {
         if (bFirst) writePartials(a, bn2, rn2);
         else writePartials(a, rn2, bn2);
@@ -1135,6 +1371,45 @@ int ppeAssemble(Ctx* ctx) {
     unsigned char* lc8 = wins ? ctx->aLc8 : nullptr;
     unsigned short* lcEsc = wins ? ctx->aLcEsc : nullptr;
     int* win = wins ? ctx->aWin : nullptr;
+    // Several lanes per row where one lane per row leaves the chip idle (a
+    // row's ~120 entries one after the other take ~180 us whatever the count).
+    // Us with one lane / 4 / 16 lanes and the window kernel: 178 / 70 / 33 at
+    // 1,728 rows, 192 / 94 / 114 at 13,824, 201 / 140 / 275 at 44,100, 231 /
+    // 240 / 490 at 81,312 (FP64 and mixed alike).
+    const int lanes = ctx->N <= 8192 ? 16 : (ctx->N <= 65536 ? 4 : 0);
+    if (lanes != 0) {
+        ctx->asmBlocks = gridFor(ctx->N, kB / lanes);
+        if (wins) hipLaunchKernelGGL(kPpeWindow, dim3(g), dim3(kB), 0, ctx->stream, a, win);
+#define ASMG(L, TT, R, LL)                                                                                     \
+    hipLaunchKernelGGL((kPpeAssembleGroup<L, TT, R, LL>), dim3(ctx->asmBlocks), dim3(kB), 0, ctx->stream, a,   \
+                       ctx->aVal, ctx->aCol, ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->D[DPPEB], v32, d32, i32,   \
+                       invd64, x, ctx->cgR, bFirst, lc8, lcEsc, win)
+#define ASMGL(L, TT, R)                        \
+    do {                                       \
+        if (lanes == 16) ASMG(L, TT, R, 16);   \
+        else ASMG(L, TT, R, 4);                \
+    } while (0)
+#define ASMGR(L, TT)                 \
+    do {                             \
+        if (res) ASMGL(L, TT, true); \
+        else ASMGL(L, TT, false);    \
+    } while (0)
+        if (ctx->listValid) {
+            if (T) ASMGR(true, true); else ASMGR(true, false);
+        } else {
+            if (T) ASMGR(false, true); else ASMGR(false, false);
+        }
+#undef ASMGR
+#undef ASMGL
+#undef ASMG
+        MPS_HIP(hipGetLastError());
+        ctx->r0Fresh = res;
+        ctx->r0FreshMixed = mixed;
+        ctx->winValid = wins;
+        ctx->asmMode = asmModeOf(ctx->P);
+        return MPS_OK;
+    }
+    ctx->asmBlocks = g;
 #define ASM(L, TT, R)                                                                                          \
     hipLaunchKernelGGL((kPpeAssemble<L, TT, R>), dim3(g), dim3(kB), 0, ctx->stream, a, ctx->aVal, ctx->aCol,   \
                        ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->D[DPPEB], v32, d32, i32, invd64, x, ctx->cgR, bFirst, \
@@ -1464,7 +1739,7 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
     ctx->r0Fresh = false;
     KArgs a0 = a;
     if (fresh) a0.red = ctx->asmRed;
-    hipLaunchKernelGGL(kCgStartFinish, dim3(1), dim3(1024), 0, s, a0, nb, tol);
+    hipLaunchKernelGGL(kCgStartFinish, dim3(1), dim3(1024), 0, s, a0, fresh ? ctx->asmBlocks : nb, tol);
     hipLaunchKernelGGL(kCgZeroX, dim3(nb), dim3(kB), 0, s, a, c.x);
     hipLaunchKernelGGL(kCgInitP, dim3(nb), dim3(kB), 0, s, a, c);
     hipLaunchKernelGGL(kCgInitPFinish, dim3(1), dim3(1024), 0, s, a, nb);
@@ -1537,7 +1812,7 @@ static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int bat
         ctx->r0Fresh = false;
         KArgs a0 = a;
         if (fresh) a0.red = ctx->asmRed;
-        hipLaunchKernelGGL(kTrueResidualFinish, dim3(1), dim3(1024), 0, s, a0, nb);
+        hipLaunchKernelGGL(kTrueResidualFinish, dim3(1), dim3(1024), 0, s, a0, fresh ? ctx->asmBlocks : nb);
         if ((rc = readStatus(ctx, nullptr, 0))) return rc;
         const double rn2 = ctx->hostScalars[S_TRUE_RN2], bn2 = ctx->hostScalars[S_BN2];
         if (!std::isfinite(rn2) || !std::isfinite(bn2)) break;   // reported by ppeSolve

@@ -93,3 +93,47 @@ def test_particle_wall_operators(built, l0):
     both("collision", ["collision"], ["vel"])
     both("wall_dummy_velocity", ["wall_dummy_velocity"], ["vel"])   # bucket walks from here
     both("shifting", ["shifting"], ["pos"])
+
+
+def _sorted_coo(rp, cols, vals, transpose):
+    r = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    if transpose:
+        r, cols = cols, r
+    k = np.lexsort((cols, r))
+    return r[k], cols[k], vals[k]
+
+
+@pytest.mark.parametrize("shape", [(7, 5, 3), (32, 16, 16), (31, 17, 16), (64, 32, 32), (65, 32, 32)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_assembly(built, shape, precision):
+    """The assembled system with 16, 4 and one lane per row: entries and
+    right-hand side bit for bit, and the mixed solve's FP32 entries, codes and
+    first residual through the solution they give."""
+    w = _dam3d(*shape)
+    w.params.precision_mode = precision
+    print(f"assembly {shape} {w.n} precision {precision}", flush=True)
+    g, o = new_pair(w)
+    g.call("init")
+    o.call("init")
+    g.set("press", o.get("press"))
+    guess = o.get("press") * 0.9
+    for s in (g, o):
+        s.set("ppe_x", guess)
+    g.call("ppe_assemble")
+    o.call("assemble_ppe")
+    a = _sorted_coo(*g.ppe_matrix(), transpose=False)
+    b = _sorted_coo(*o.ppe_matrix(), transpose=True)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    check(g, o, ["ppe_b"], f"{w.n} ppe_assemble")
+    # every row group writes its window indices: the blocks are served from
+    # windows, and the same solve gathered from global memory agrees in bits
+    assert g.scalar("ppe_window_blocks") == (w.n + 255) // 256
+    g.call("ppe_solve")
+    windowed = g.get("ppe_x")
+    assert g.scalar("true_residual") <= 1e-8
+    g.set_scalar("ppe_window", 0)
+    g.set("ppe_x", guess)
+    g.call("ppe_assemble")
+    g.call("ppe_solve")
+    assert np.array_equal(windowed, g.get("ppe_x"))
