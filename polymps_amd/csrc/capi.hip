@@ -544,12 +544,12 @@ int mps_destroy(mps_ctx* ctx) {
         if (ctx->DaltNN[q]) hipFree(ctx->DaltNN[q]);
     void* bufs[] = {ctx->cellStart, ctx->cellCount, ctx->key, ctx->rank, ctx->order, ctx->order2, ctx->slotOf,
                     ctx->bvh, ctx->bvhTri, ctx->scanTmp, ctx->outList, ctx->nbrMask, ctx->nbr, ctx->nbrCnt, ctx->P4, ctx->mV, ctx->mF, ctx->mN, ctx->wtab,
-                    ctx->aVal, ctx->aCol, ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->aVal32, ctx->aLc8, ctx->aLcEsc, ctx->aWin,
+                    ctx->aVal, ctx->aCol, ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->aVal32, ctx->aLc8, ctx->aLcEsc, ctx->aLc16, ctx->aWin,
                     ctx->aDiagInv32,
                     ctx->aDiag32, ctx->cgR, ctx->cgP,
                     ctx->cgZ, ctx->cgQ, ctx->cgInvD, ctx->cgX, ctx->fR, ctx->fP, ctx->fZ, ctx->fQ, ctx->fX,
                     ctx->bcgR0, ctx->bcgY, ctx->bcgS, ctx->bcgT, ctx->patchList, ctx->fixList, ctx->V4, ctx->nbrMaskS, ctx->nbrS, ctx->nbrCntS,
-                    ctx->ds, ctx->is, ctx->red, ctx->asmRed, ctx->red64, ctx->IaltPtype, ctx->bedKeys, ctx->bedIdx};
+                    ctx->ds, ctx->is, ctx->red, ctx->asmRed, ctx->gridBar, ctx->gridPart, ctx->gridP2, ctx->red64, ctx->IaltPtype, ctx->bedKeys, ctx->bedIdx};
     for (void* b : bufs)
         if (b) hipFree(b);
     freeSlot(ctx->extraMesh[0]);

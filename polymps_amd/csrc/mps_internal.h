@@ -53,8 +53,11 @@ enum DScalar { S_VELMAX, S_ABSNEW, S_ABSOLD, S_RHSN2, S_THR, S_RN2, S_ALPHA, S_B
                S_NNZ,   // PPE entries of the last assembly, counted on the device when profiling
                NDS };
 // device scalar slots (int)
-enum IScalar { I_NLIVE, I_OUTCNT, I_OVERFLOW, I_CG_ITER, I_CG_DONE, I_COMPACT_OVF, I_NESC,
-               I_BCG_RESTART, I_BCG_RESTARTS, I_REBUILD, I_PATCHCNT, I_FIXCNT, I_NLCESC, NIS };
+enum IScalar { I_NLIVE, I_OUTCNT, I_OVERFLOW, I_CG_ITER, I_CG_OUTER, I_CG_DONE, I_COMPACT_OVF,
+               I_NESC, I_NLCESC, I_NOWIN,   // zeroed together by each assembly; I_NOWIN: no solve in one launch
+               I_BCG_RESTART, I_BCG_RESTARTS, I_REBUILD, I_PATCHCNT, I_FIXCNT,
+               I_GRID_LATE,   // a solve in one launch left without a result
+               NIS };
 
 constexpr int kWallTable = 50;
 // escaped (non-delta) columns per PPE row: the first entry and stencil-row
@@ -208,6 +211,8 @@ struct Ctx {
     unsigned char* aLc8 = nullptr;    // ELL, groups of 8: one-byte window index codes (step or 0 = escape)
     unsigned short* aLcEsc = nullptr; // ELL, kLcEsc per row: the escapes' absolute window indices
     int* aWin = nullptr;              // per 256-row block: the LDS window table of the mixed SpMV
+    unsigned short* aLc16 = nullptr;  // ellIdx4: 16-bit window indices (solves in one launch)
+    bool win16Valid = false;          // the last assembly wrote them
     bool winValid = false;            // the last assembly wrote windows
     bool ppeWindow = true;            // scalar ppe_window: build and use the windows
     float* aDiagInv32 = nullptr;
@@ -247,6 +252,12 @@ struct Ctx {
     int lastPass2Iters = 8;          // iterations of the last solve's second refinement pass
     bool r0Fresh = false;        // cgR and asmRed hold b - A x of the current guess and its partials (assembly)
     bool r0FreshMixed = false;   // ... in the mixed solve's partial order (else the FP64 CG's, with 1/diag)
+    // solves in one launch (allocated on first use): barrier counters,
+    // block sums, the second search direction; whether the device holds the grid (per precision)
+    unsigned* gridBar = nullptr;
+    double* gridPart = nullptr;
+    double* gridP2 = nullptr;
+    int oneLaunchFits[2] = {-1, -1};
     int asmBlocks = 0;           // blocks (partials) of the last assembly
     double* asmRed = nullptr;    // block partials of the assembly's first residual (no other kernel writes them)
     unsigned long long* red64 = nullptr;   // result of reduceCounts (allocated on first use)

@@ -40,6 +40,19 @@ constexpr int kB = 256;
 //   [11 + k] its LDS offset (k = 0 .. m; offset m = the window's size).
 constexpr int kWinMax = 5000;    // slots: 20 KB of FP32 / 40 KB of FP64 values per block
 constexpr int kWinStride = 24;   // ints per block in the table
+// The same windows, with indices of 16 bits, serve a solve in one launch:
+// FP64 slots of the LDS its blocks have (one block of 1,024 threads per CU up
+// to 65,536 rows, two of 512 above), and the widest window it takes, else
+// I_NOWIN is raised and the solve is launched in pieces.  Up to 65,536 rows a
+// window wider than the LDS is staged in parts; above, a block that did so
+// would keep all others waiting for longer than the pieces take (83,204 rows
+// of a collapsed column, windows of 20,000 slots: 0.95 ms per solve against
+// 0.73).
+__host__ __device__ __forceinline__ int win16Lds(int N) { return N <= 65536 ? 16384 : 9216; }
+__host__ __device__ __forceinline__ int win16Max(int N) { return N <= 65536 ? 65535 : 9216; }
+
+constexpr int kOneLaunchMax = 131072;   // rows (window indices of 16 bits are kept for these, ensureWindows)
+constexpr int kFullMax = 16384;         // rows whose whole vector fits a block's LDS (periodic domains)
 
 // The block's window from its rows' current stencil rows (rows with
 // entries only), merged; every thread returns the segments in sS/sE/sB.
@@ -85,14 +98,32 @@ __device__ __forceinline__ void ppeWindowBegin(const KArgs& a, int i, int* sS, i
     }
     __syncthreads();
     if (threadIdx.x < 64) {
-        // lane r: row r's union over the block; then starts and ends ascend
-        // with the row, so overlapping neighbours merge in one pass
+        // lane r: row r's union over the block, sorted by start (a row that
+        // few of the block's particles look at may start before the row
+        // ahead of it: sparse flow), then merged in one pass
+        __shared__ int us[9], ue[9];
         int s = INT_MAX, e = INT_MIN;
         if (threadIdx.x < rows)
             for (int q = 0; q < kB / 64; q++) {
                 s = min(s, ps[q][threadIdx.x]);
                 e = max(e, pe[q][threadIdx.x]);
             }
+        int rank = 0;
+        for (int q = 0; q < rows; q++) {
+            const int sq = __builtin_amdgcn_readlane(s, q);
+            rank += (sq < s || (sq == s && q < (int)threadIdx.x)) ? 1 : 0;
+        }
+        if (threadIdx.x < rows) {
+            us[rank] = s;
+            ue[rank] = e;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (threadIdx.x < rows) {
+            s = us[threadIdx.x];
+            e = ue[threadIdx.x];
+        }
         int m = 0, W = 0, last = 0;
         for (int r = 0; r < rows; r++) {
             const int sr = __builtin_amdgcn_readlane(s, r), er = __builtin_amdgcn_readlane(e, r);
@@ -131,13 +162,13 @@ __device__ __forceinline__ void ppeWindowBegin(const KArgs& a, int i, int* sS, i
 // (segments wS/wE/wB, wM of them) as a one-byte step from the previous
 // entry's, or an escape to the next of the row's absolute indices; outside =
 // some column is not in the window or the row's indices do not fit the code.
-template <bool LIST, bool TRANS, bool RES>
+template <bool LIST, bool TRANS, bool RES, bool W16>
 __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, unsigned short* col, int* esc,
                                             int* cnt, double* diag, double* b, float* val32, float* diag32,
                                             float* invd32, double* invd64, double* x, double* r, double& rn2,
                                             double& bn2, unsigned char* lc8, unsigned short* lcEsc, const int* wS,
                                             const int* wE, const int* wB, int wM, bool& outside, int& nEsc,
-                                            int& nLc) {
+                                            int& nLc, unsigned short* lc16, bool& outside16) {
     if (!live(a, i)) {
         cnt[i] = 0; diag[i] = 1.0; b[i] = 0.0;
         if (invd32) { invd32[i] = 1.0f; diag32[i] = 1.0f; }
@@ -178,14 +209,15 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
     typedef float F4 __attribute__((ext_vector_type(4)));
     typedef unsigned short U4 __attribute__((ext_vector_type(4)));
     F4 g32 = {0.0f, 0.0f, 0.0f, 0.0f};   // the current group of four FP32 values / codes
-    U4 gcd = {0, 0, 0, 0};
+    U4 gcd = {0, 0, 0, 0}, g16 = {0, 0, 0, 0};
     // window index codes: eight one-byte codes per group (lc8), the escapes'
     // absolute indices in lcEsc
     unsigned g8lo = 0, g8hi = 0;
     int prevLc = -1, nle = 0;
     // the window segment of the current column (columns ascend)
     int wk = 0, curS = 0, curE = 0, curB = 0;
-    if (lc8 && wM > 0) {
+    const bool windowed = W16 || lc8 != nullptr;
+    if (windowed && wM > 0) {
         curS = wS[0];
         curE = wE[0];
         curB = wB[0];
@@ -268,7 +300,8 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
                 // FP32 values and codes leave in groups of four (ellIdx4)
                 const float f = (float)mv;
                 const unsigned short cd = delta ? (unsigned short)dj : (unsigned short)0;
-                if (lc8) {
+                unsigned short c16 = 0;   // W16
+                if (windowed) {
                     while (wk < wM && j >= curE) {
                         wk++;
                         if (wk < wM) {
@@ -279,7 +312,11 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
                     }
                     int lc = -1;
                     if (wk < wM && j >= curS) lc = curB + (j - curS);
-                    else outside = true;
+                    else {
+                        outside = true;
+                        if (W16) outside16 = true;
+                    }
+                    if (W16) c16 = (unsigned short)max(lc, 0);
                     // code: the step from the previous entry's index (1-255)
                     // or 0, an escape to the next absolute index of the row
                     // (at most kLcEsc per row, or the block gathers from
@@ -293,25 +330,26 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
                     if (prevLc >= 0 && lc >= 0 && dl > 0 && dl < 256) {
                         code = (unsigned)dl;
                     } else {
-                        if (lc >= 0 && nle < kLcEsc) lcEsc[ellElem(nle, i, kLcEsc)] = (unsigned short)lc;
+                        if (lc >= 0 && nle < kLcEsc && (!W16 || lc8)) lcEsc[ellElem(nle, i, kLcEsc)] = (unsigned short)lc;
                         else outside = true;
                         nle++;
                     }
                     prevLc = lc;
                     if (c & 4) g8hi |= code << (8 * (c & 3));
                     else g8lo |= code << (8 * (c & 3));
-                    if ((c & 7) == 7) reinterpret_cast<uint2*>(lc8)[ellElem(c >> 3, i, KE >> 3)] = make_uint2(g8lo, g8hi);
+                    if ((c & 7) == 7 && (!W16 || lc8)) reinterpret_cast<uint2*>(lc8)[ellElem(c >> 3, i, KE >> 3)] = make_uint2(g8lo, g8hi);
                 }
                 switch (c & 3) {
-                    case 0: g32.x = f; gcd.x = cd; break;
-                    case 1: g32.y = f; gcd.y = cd; break;
-                    case 2: g32.z = f; gcd.z = cd; break;
-                    default: g32.w = f; gcd.w = cd; break;
+                    case 0: g32.x = f; gcd.x = cd; g16.x = c16; break;
+                    case 1: g32.y = f; gcd.y = cd; g16.y = c16; break;
+                    case 2: g32.z = f; gcd.z = cd; g16.z = c16; break;
+                    default: g32.w = f; gcd.w = cd; g16.w = c16; break;
                 }
                 if ((c & 3) == 3) {
                     const size_t gi = ellElem(c >> 2, i, KE >> 2);
                     if (val32) reinterpret_cast<F4*>(val32)[gi] = g32;
                     reinterpret_cast<U4*>(col)[gi] = gcd;
+                    if (W16) reinterpret_cast<U4*>(lc16)[gi] = g16;
                 }
                 if (RES) ax += mv * xOf();
                 if (!delta) {
@@ -340,6 +378,7 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
         const size_t gi = ellElem(c >> 2, i, KE >> 2);
         if (val32) reinterpret_cast<F4*>(val32)[gi] = g32;
         reinterpret_cast<U4*>(col)[gi] = gcd;
+        if (W16) reinterpret_cast<U4*>(lc16)[gi] = g16;
     }
     if (lc8 && (c & 7)) reinterpret_cast<uint2*>(lc8)[ellElem(c >> 3, i, KE >> 3)] = make_uint2(g8lo, g8hi);
     if (full) atomicMax(&a.is[I_OVERFLOW], c + 1);   // reported as a capacity error after the step
@@ -367,11 +406,13 @@ __device__ __forceinline__ void assembleRow(const KArgs& a, int i, double* val, 
     }
 }
 
-template <bool LIST, bool TRANS, bool RES>
+// W16: with the 16-bit window indices of a solve in one launch
+template <bool LIST, bool TRANS, bool RES, bool W16>
 __global__ __launch_bounds__(256) void kPpeAssemble(KArgs a, double* val, unsigned short* col, int* esc, int* cnt,
                                                     double* diag, double* b, float* val32, float* diag32,
                                                     float* invd32, double* invd64, double* x, double* r,
-                                                    int bFirst, unsigned char* lc8, unsigned short* lcEsc, int* win);
+                                                    int bFirst, unsigned char* lc8, unsigned short* lcEsc, int* win,
+                                                    unsigned short* lc16);
 
 // ------------------------------------------------------------ reductions
 // Every vector kernel runs one thread per row; each block leaves a pair of
@@ -396,20 +437,24 @@ __device__ __forceinline__ void writePartials(const KArgs& a, double s0, double 
 }
 
 // lc8 / lcEsc / win: window index codes and escapes, the block's window table
-template <bool LIST, bool TRANS, bool RES>
+template <bool LIST, bool TRANS, bool RES, bool W16>
 __global__ __launch_bounds__(256) void kPpeAssemble(KArgs a, double* val, unsigned short* col, int* esc, int* cnt,
                                                     double* diag, double* b, float* val32, float* diag32,
                                                     float* invd32, double* invd64, double* x, double* r,
-                                                    int bFirst, unsigned char* lc8, unsigned short* lcEsc, int* win) {
+                                                    int bFirst, unsigned char* lc8, unsigned short* lcEsc, int* win,
+                                                    unsigned short* lc16) {
     __shared__ int wS[9], wE[9], wB[10], wM, wOut;
     const int i = slotId();
-    if (lc8) ppeWindowBegin(a, i, wS, wE, wB, wM, wOut);
+    if (win) {
+        ppeWindowBegin(a, i, wS, wE, wB, wM, wOut);
+        if (W16 && threadIdx.x == 0 && wB[wM] > win16Max(a.N)) a.is[I_NOWIN] = 1;
+    }
     double rn2 = 0.0, bn2 = 0.0;
-    bool outside = false;
+    bool outside = false, outside16 = false;
     int nEsc = 0, nLc = 0;
     if (i < a.N)
-        assembleRow<LIST, TRANS, RES>(a, i, val, col, esc, cnt, diag, b, val32, diag32, invd32, invd64, x, r, rn2,
-                                      bn2, lc8, lcEsc, wS, wE, wB, lc8 ? wM : 0, outside, nEsc, nLc);
+        assembleRow<LIST, TRANS, RES, W16>(a, i, val, col, esc, cnt, diag, b, val32, diag32, invd32, invd64, x, r, rn2,
+                                      bn2, lc8, lcEsc, wS, wE, wB, win ? wM : 0, outside, nEsc, nLc, lc16, outside16);
     // escaped columns and window index escapes: one atomic per wavefront
     nEsc = waveSumInt(nEsc);
     nLc = waveSumInt(nLc);
@@ -417,8 +462,9 @@ __global__ __launch_bounds__(256) void kPpeAssemble(KArgs a, double* val, unsign
         if (nEsc) atomicAdd(&a.is[I_NESC], nEsc);
         if (nLc) atomicAdd(&a.is[I_NLCESC], nLc);
     }
-    if (lc8) {
+    if (win) {
         if (__builtin_amdgcn_ballot_w64(outside) != 0 && (threadIdx.x & 63) == 0) atomicOr(&wOut, 1);
+        if (W16 && __builtin_amdgcn_ballot_w64(outside16) != 0 && (threadIdx.x & 63) == 0) a.is[I_NOWIN] = 1;
         __syncthreads();
         if (threadIdx.x == 0) {
             int* t = win + (size_t)blockIdx.x * kWinStride;
@@ -446,6 +492,7 @@ __global__ __launch_bounds__(256) void kPpeWindow(KArgs a, int* win) {
     t[1] = wM;
     for (int k = 0; k < wM; k++) t[2 + k] = wS[k];
     for (int k = 0; k <= wM; k++) t[11 + k] = wB[k];
+    if (wB[wM] > win16Max(a.N) && !periodicDomain(a.P)) a.is[I_NOWIN] = 1;
 }
 
 // One row by L lanes, each with the neighbours c0 + l of a chunk: what the
@@ -458,7 +505,8 @@ __device__ __forceinline__ void assembleRowGroup(const KArgs& a, int i, double* 
                                                  int* cnt, double* diag, double* b, float* val32, float* diag32,
                                                  float* invd32, double* invd64, double* x, double* r, double& rn2,
                                                  double& bn2, unsigned char* lc8, unsigned short* lcEsc, const int* wS,
-                                                 const int* wB, int wM, bool& outside, int& nEsc, int& nLc) {
+                                                 const int* wB, int wM, bool& outside, int& nEsc, int& nLc,
+                                                 unsigned short* lc16, bool& outside16) {
     const mps_params& P = a.P;
     const int l = groupLaneId<L>();
     const bool lv = live(a, i);
@@ -564,11 +612,16 @@ __device__ __forceinline__ void assembleRowGroup(const KArgs& a, int i, double* 
         double mv = mij;
         if (TRANS && d2T != d2) mv = wgt(sqrt(d2T), P.re_l, P.weight_type) * P.coeff_ppe;
         int lc = -1;
+        for (int k = 0; k < wM; k++) {
+            const int S = wS[k], B0 = wB[k];
+            if (j >= S && j - S < wB[k + 1] - B0) lc = B0 + (j - S);
+        }
+        if (lc16 && fits) {   // a periodic domain's window is the whole vector
+            const int e = periodic ? j : lc;
+            if (e < 0) outside16 = true;
+            lc16[ellIdx4(cc, i, KE)] = (unsigned short)max(e, 0);
+        }
         if (lc8) {
-            for (int k = 0; k < wM; k++) {
-                const int S = wS[k], B0 = wB[k];
-                if (j >= S && j - S < wB[k + 1] - B0) lc = B0 + (j - S);
-            }
             const int pl = __shfl(lc, base + src, 64);
             const int plc = lower ? pl : prevLc;
             const int dl = lc - plc;
@@ -632,22 +685,23 @@ __global__ __launch_bounds__(256) void kPpeAssembleGroup(KArgs a, double* val, u
                                                          double* diag, double* b, float* val32, float* diag32,
                                                          float* invd32, double* invd64, double* x, double* r,
                                                          int bFirst, unsigned char* lc8, unsigned short* lcEsc,
-                                                         int* win) {
+                                                         int* win, unsigned short* lc16) {
     __shared__ int wS[9], wB[10], wM;
     const int i = groupSlot<L>();
-    int* const t = lc8 ? win + (size_t)(blockIdx.x / L) * kWinStride : nullptr;   // 256 / L rows per workgroup
-    if (lc8) {
+    int* const t = win ? win + (size_t)(blockIdx.x / L) * kWinStride : nullptr;   // 256 / L rows per workgroup
+    if (win) {
         if (threadIdx.x < 9) wS[threadIdx.x] = t[2 + threadIdx.x];
         if (threadIdx.x < 10) wB[threadIdx.x] = t[11 + threadIdx.x];
         if (threadIdx.x == 0) wM = t[1];
         __syncthreads();
     }
     double rn2 = 0.0, bn2 = 0.0;
-    bool outside = false;
+    bool outside = false, outside16 = false;
     int nEsc = 0, nLc = 0;
     if (i < a.N)
         assembleRowGroup<LIST, TRANS, RES, L>(a, i, val, col, esc, cnt, diag, b, val32, diag32, invd32, invd64, x, r,
-                                              rn2, bn2, lc8, lcEsc, wS, wB, lc8 ? wM : 0, outside, nEsc, nLc);
+                                              rn2, bn2, lc8, lcEsc, wS, wB, win ? wM : 0, outside, nEsc, nLc, lc16,
+                                              outside16);
     nEsc = waveSumInt(nEsc);
     nLc = waveSumInt(nLc);
     const bool out = lc8 && __builtin_amdgcn_ballot_w64(outside) != 0;
@@ -656,6 +710,7 @@ __global__ __launch_bounds__(256) void kPpeAssembleGroup(KArgs a, double* val, u
         if (nLc) atomicAdd(&a.is[I_NLCESC], nLc);
         if (out) atomicOr(t, 1);
     }
+    if (__builtin_amdgcn_ballot_w64(outside16) != 0 && (threadIdx.x & 63) == 0) a.is[I_NOWIN] = 1;
     if (RES) {
         if (bFirst) writePartials(a, bn2, rn2);
         else writePartials(a, rn2, bn2);
@@ -893,6 +948,7 @@ struct CgPtrs {
     const unsigned char* lc8;
     const unsigned short* lcEsc;
     const int* win;
+    const unsigned short* lc16;   // 16-bit window indices (ellIdx4; solves in one launch)
 };
 
 // Row from the block's LDS window, in the order of ellRow (FP32: batches of
@@ -1212,6 +1268,505 @@ __global__ void kMxApply(KArgs a, CgPtrs c) {
     if (i < a.N && live(a, i)) c.x[i] += c.fd[i];
 }
 
+// ------------------------------------------------ solves in one launch
+// Systems of up to kOneLaunchMax rows are solved by one launch.
+// Launched piece by piece, an iteration is an SpMV whose lanes each go through
+// a row of ~120 entries, two one-block finishes of its sums and two vector
+// updates: 34 us at 1,728 rows (SpMV 11, the other four 3.3 each and the gaps
+// between them), 60 at 83,204 (SpMV 36).  Here L lanes share a row, a block
+// keeps its rows' x, r, p and 1/diag in registers from one iteration to the
+// next, every block adds the block sums itself, and the blocks meet at two
+// grid barriers per iteration: after p.q and after |r|^2, r.z.  The next
+// search direction needs no third one: z is published before the second
+// barrier and the last p earlier, so each block forms z + beta p for the
+// slots of its window as it stages them, as the rows' owners do.
+//
+// What other blocks read (z, p, x, block sums) is stored and loaded at agent
+// scope: the eight XCDs' L2 caches are not coherent with each other, and a
+// release fence would write back a whole L2 per block.
+//
+// Lanes per row and threads per block: 16 and 1,024 (64 rows) up to 16,384
+// rows, 4 and 1,024 (256 rows) up to 65,536, 2 and 512 up to 131,072: at most
+// 256 blocks of 1,024 or 512 of 512 threads, which the chip holds at once.
+// With one lane (216,000 rows) the launch took 95 us per iteration against 77
+// for the pieces.
+//
+// The grid is no larger than what the device holds (asked of the runtime), so
+// on a device of its own every block is running when it waits.  Where other
+// work keeps blocks out (another context's solve in one launch, at worst,
+// waiting for the same CUs), the wait ends after kSpinMax polls, every block
+// leaves, and the solve is repeated in pieces.  (A cooperative launch would
+// settle this in the runtime, at the price of draining the stream before and
+// after it: 40-60 us per solve.)
+constexpr int kGridBars = 9;            // counters: eight groups of blocks, the root (one cache line each)
+constexpr int kBarStride = 32;          // unsigned per cache line
+constexpr int kSpinMax = 1 << 16;       // polls (of about 0.7 us) before a barrier gives up
+
+template <class T>
+__device__ __forceinline__ T loadAgent(const T* p) {
+    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void storeAgent(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Barrier number `epoch` (from 1) over the grid.  The blocks count in eight
+// groups (blocks are dealt round-robin to the XCDs) and the last block of a
+// group counts at the root, which all poll: 256 blocks on one counter take
+// 3.7 us.  The threads' agent-scope stores have completed when it is counted.
+// false: a block did not arrive in time, every block leaves.
+__device__ __forceinline__ bool gridBarrier(unsigned* bar, unsigned epoch, int* lateFlag) {
+    __shared__ int late;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // the wave's own stores
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned g = blockIdx.x & 7u, size = (gridDim.x - g + 7u) >> 3, groups = min(gridDim.x, 8u);
+        unsigned* const root = bar + 8 * kBarStride;
+        if (__hip_atomic_fetch_add(bar + g * kBarStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u ==
+            epoch * size)
+            __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int spin = 0;
+        while (loadAgent(root) < epoch * groups && ++spin < kSpinMax) __builtin_amdgcn_s_sleep(1);
+        late = spin >= kSpinMax ? 1 : 0;
+        if (late) atomicOr(lateFlag, 1);
+    }
+    __syncthreads();
+    return late == 0;
+}
+// the last block out puts the counters back to zero
+__device__ __forceinline__ void leaveGrid(unsigned* bar) {
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    unsigned* const out = bar + kGridBars * kBarStride;
+    if (__hip_atomic_fetch_add(out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x) {
+        for (int k = 0; k <= kGridBars; k++) storeAgent(bar + k * kBarStride, 0u);
+    }
+}
+
+// The wave's sum in every lane, by row shifts and row broadcasts (DPP): a
+// shuffle step goes through the LDS, six of them take half a microsecond.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dppAdd(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double waveSumDpp(double v) {
+    v = dppAdd<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8: lane 15 of a row holds its sum
+    v = dppAdd<0x112, 0xf>(v);
+    v = dppAdd<0x114, 0xf>(v);
+    v = dppAdd<0x118, 0xf>(v);
+    v = dppAdd<0x142, 0xa>(v);   // row_bcast15 into rows 1 and 3, row_bcast31 into rows 2 and 3
+    v = dppAdd<0x143, 0xc>(v);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// S sums over the block's threads, the same in every thread and every block
+template <int S>
+__device__ __forceinline__ void addThreads(double (&v)[S], double (&t)[S]) {
+    __shared__ double sh[S][16];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+        const double w = waveSumDpp(v[c]);
+        if ((threadIdx.x & 63) == 0) sh[c][threadIdx.x >> 6] = w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+        t[c] = 0.0;
+        for (int q = 0; q < (int)(blockDim.x >> 6); q++) t[c] += sh[c][q];
+    }
+}
+// the sums the blocks of this launch published (at most two per thread)
+template <int S>
+__device__ __forceinline__ void sumPublished(const double* part, double (&t)[S]) {
+    double v[S];
+#pragma unroll
+    for (int c = 0; c < S; c++) v[c] = 0.0;
+    for (int q = threadIdx.x; q < (int)gridDim.x; q += blockDim.x)
+#pragma unroll
+        for (int c = 0; c < S; c++) v[c] += loadAgent(part + (size_t)q * S + c);
+    addThreads<S>(v, t);
+}
+// the sums an earlier launch left
+template <int S>
+__device__ __forceinline__ void sumLeft(const double* part, int n, double (&t)[S]) {
+    double v[S];
+#pragma unroll
+    for (int c = 0; c < S; c++) v[c] = 0.0;
+    for (int q = threadIdx.x; q < n; q += blockDim.x)
+#pragma unroll
+        for (int c = 0; c < S; c++) v[c] += part[(size_t)q * S + c];
+    addThreads<S>(v, t);
+}
+// the block's sums for the others
+template <int S>
+__device__ __forceinline__ void publishSums(double* part, double s0, double s1) {
+    double v[S], t[S];
+    v[0] = s0;
+    if constexpr (S == 2) v[1] = s1;
+    addThreads<S>(v, t);
+    if (threadIdx.x == 0) {
+        storeAgent(part + (size_t)blockIdx.x * S, t[0]);
+        if constexpr (S == 2) storeAgent(part + (size_t)blockIdx.x * S + 1, t[1]);
+    }
+}
+
+// A block's window: its segments' first slots and window entries (the
+// segments past the last one start past the window's end), its size.
+struct Window {
+    int first[9], entry[9], W;
+};
+__device__ __forceinline__ Window loadWindow(const int* t, bool full, int N) {
+    Window w;
+    const int m = full ? 1 : t[1];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        w.first[k] = full ? 0 : __builtin_amdgcn_readfirstlane(t[2 + k]);
+        w.entry[k] = k == 0 ? 0 : __builtin_amdgcn_readfirstlane(k < m ? t[11 + k] : INT_MAX);
+    }
+    w.W = full ? N : __builtin_amdgcn_readfirstlane(t[11 + m]);
+    return w;
+}
+// Entries q0 .. q0 + m - 1 of the window of a published vector, formed by
+// f(slot); eight loads per thread in flight (agent-scope loads come from
+// beyond the L2).
+template <class T, class F>
+__device__ __forceinline__ void stageWindowBy(const Window& w, T* win, int q0, int m, F&& f) {
+    constexpr int U = 8;
+    __syncthreads();   // the rows have read the last window
+    const int nt = blockDim.x;
+    for (int e = threadIdx.x; e < m; e += U * nt) {
+        int slot[U];
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int q = q0 + min(e + u * nt, m - 1);
+            int d = w.first[0];   // slot - window entry
+#pragma unroll
+            for (int k = 1; k < 9; k++) d = q >= w.entry[k] ? w.first[k] - w.entry[k] : d;
+            slot[u] = q + d;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (u == 0 || e + u * nt < m) v[u] = f(slot[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (u == 0 || e + u * nt < m) win[e + u * nt] = v[u];
+    }
+    __syncthreads();
+}
+
+// The row's products with window entries q0 .. q0 + m - 1, lane l taking the groups of four entries l, l + L, ...;
+// values in FP32 are summed four at a time in FP32, everything else in FP64.
+template <class T, int L>
+__device__ __forceinline__ double rowWindow(const CgPtrs& c, const T* __restrict__ val, const T* win, int q0, int m,
+                                            int n, int KE, int i, double acc) {
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    typedef float F4 __attribute__((ext_vector_type(4)));
+#pragma unroll 2
+    for (int g = groupLaneId<L>(); 4 * g < n; g += L) {
+        const EllU4 k = reinterpret_cast<const EllU4*>(c.lc16)[ellElem(g, i, KE >> 2)];
+        T v[4];
+        if (sizeof(T) == 8) {
+            const D2 a0 = reinterpret_cast<const D2*>(val)[ellElem(2 * g, i, KE >> 1)];
+            const D2 a1 = reinterpret_cast<const D2*>(val)[ellElem(2 * g + 1, i, KE >> 1)];
+            v[0] = (T)a0.x; v[1] = (T)a0.y; v[2] = (T)a1.x; v[3] = (T)a1.y;
+        } else {
+            const F4 a0 = reinterpret_cast<const F4*>(val)[ellElem(g, i, KE >> 2)];
+            v[0] = (T)a0.x; v[1] = (T)a0.y; v[2] = (T)a0.z; v[3] = (T)a0.w;
+        }
+        const int rem = n - 4 * g;
+        unsigned kk[4] = {k.x, rem > 1 ? k.y : k.x, rem > 2 ? k.z : k.x, rem > 3 ? k.w : k.x};
+        bool in[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            kk[q] -= (unsigned)q0;   // below the part: wraps to a large number
+            in[q] = q < rem && kk[q] < (unsigned)m;
+            kk[q] = in[q] ? kk[q] : 0u;
+        }
+        if (sizeof(T) == 8) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc += in[q] ? (double)(v[q] * win[kk[q]]) : 0.0;
+        } else {
+            T s = in[0] ? v[0] * win[kk[0]] : (T)0;
+#pragma unroll
+            for (int q = 1; q < 4; q++) s += in[q] ? v[q] * win[kk[q]] : (T)0;
+            acc += (double)s;
+        }
+    }
+    return acc;
+}
+
+// Row i's product with a published vector by its L lanes, whose sums are
+// added pairwise.  The window is staged whole where it fits the block's LDS
+// (`cap` entries), else part by part: late in a flow a few blocks of every
+// grid lie along its sparse edge and look at most of the domain, and all
+// others wait for them (41,472 particles: 0.83 ms per solve where such blocks
+// read slot by slot, 0.31 with parts).  Every thread of the block.
+template <class T, int L, class F>
+__device__ __forceinline__ double rowPublished(const CgPtrs& c, const T* __restrict__ val, const Window& w, T* win,
+                                               int cap, int n, int KE, int i, double acc, F&& f) {
+    if (groupLaneId<L>() != 0) acc = 0.0;
+#pragma unroll 1
+    for (int q0 = 0; q0 < w.W; q0 += cap) {
+        const int m = min(cap, w.W - q0);
+        stageWindowBy<T>(w, win, q0, m, f);
+        acc = rowWindow<T, L>(c, val, win, q0, m, n, KE, i, acc);
+    }
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o, 64);
+    return acc;
+}
+
+struct OneLaunch {
+    unsigned* bar;       // kGridBars counters and the exit counter, zero before and after the launch
+    double* part;        // block sums, 2 per block, two areas
+    double* p2;          // second search-direction buffer (FP64: N doubles; mixed: N floats)
+    const double* asmRed;   // the assembly's sums (null: the first residual is computed here)
+    int asmBlocks;
+    int full;            // windows: the whole vector (periodic domains)
+    double tol, tolIn;
+    int maxIt, maxOuter;
+};
+extern __shared__ __align__(16) unsigned char oneLaunchLds[];
+
+// solveFp64 in one launch: the first residual (from the assembly or computed
+// here), the Jacobi-PCG, the true residual of its result and the pressure.
+template <int L, int BT>
+__global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaunch o) {
+    double* const win = reinterpret_cast<double*>(oneLaunchLds);
+    const int i = blockIdx.x * (BT / L) + threadIdx.x / L;
+    const bool row = i < a.N;
+    const bool own = row && groupLaneId<L>() == 0;   // the row's lane that stores and counts
+    const int* const table = c.win + (size_t)(blockIdx.x * (BT / L) / kB) * kWinStride;
+    if (!o.full && a.is[I_NOWIN]) {   // every block leaves
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.is[I_GRID_LATE] = 1;
+        return;
+    }
+    const Window w = loadWindow(table, o.full, a.N);
+    const int KE = ellWidth(a.K), cap = win16Lds(a.N);
+    const int n = row ? c.cnt[i] : 0;
+    const double diag = row ? c.diag[i] : 1.0, b = row ? c.b[i] : 0.0;
+    const bool lv = row && live(a, i);
+    double x = lv ? c.x[i] : 0.0;   // slots beyond the live count do not take part
+    const double invd = (diag != 0.0) ? 1.0 / diag : 1.0;
+    double* const part0 = o.part;
+    double* const part1 = o.part + 2 * (size_t)gridDim.x;
+    unsigned epoch = 0;
+    double r = 0.0, s2[2], s1[1];
+    auto residual = [&]() {   // b - A x of the published x (c.x)
+        auto xOf = [&](int j) { return loadAgent(c.x + j); };
+        return b - rowPublished<double, L>(c, c.val, w, win, cap, n, KE, i, diag * x, xOf);
+    };
+    bool ok = true;
+    if (o.asmRed != nullptr) {
+        r = row ? c.r[i] : 0.0;
+        sumLeft<2>(o.asmRed, o.asmBlocks, s2);
+    } else {
+        if (own) storeAgent(c.x + i, x);
+        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        if (ok) {
+            r = residual();
+            publishSums<2>(part0, own ? b * b : 0.0, own ? r * r : 0.0);
+            ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+            sumPublished<2>(part0, s2);
+        }
+    }
+    const double bn2 = s2[0];
+    double rn2 = s2[1];
+    const double thr = fmax(o.tol * o.tol * bn2, DBL_MIN);   // kCgStartFinish
+    int done = 0, it = 0;
+    if (!isfinite(bn2) || !isfinite(rn2)) done = 5;
+    else if (bn2 == 0.0) done = 2;
+    else if (rn2 < thr) done = 1;
+    if (done == 2) x = 0.0;
+    double p = invd * r, z = p, absNew = 0.0, beta = 0.0;
+    double* pOld = c.p;    // p of the iteration before, published
+    double* pNew = o.p2;
+    if (ok && !done) {
+        if (own) storeAgent(c.z + i, z);
+        publishSums<2>(part1, own ? r * p : 0.0, 0.0);
+        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        sumPublished<2>(part1, s2);
+        absNew = s2[0];
+    }
+    for (bool first = true; ok && !done; first = false) {
+        // q = A p, p formed from the published z and the last p
+        auto pOf = [&](int j) {
+            const double zj = loadAgent(c.z + j);
+            return first ? zj : zj + beta * loadAgent(pOld + j);
+        };
+        const double q = rowPublished<double, L>(c, c.val, w, win, cap, n, KE, i, diag * p, pOf);
+        if (own) storeAgent(pNew + i, p);
+        publishSums<1>(part0, own ? p * q : 0.0, 0.0);
+        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        sumPublished<1>(part0, s1);
+        const double alpha = absNew / s1[0];
+        x += alpha * p;
+        r = r - alpha * q;
+        z = invd * r;
+        if (own) storeAgent(c.z + i, z);
+        publishSums<2>(part1, own ? r * r : 0.0, own ? r * z : 0.0);
+        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        sumPublished<2>(part1, s2);
+        rn2 = s2[0];   // kCgBeta
+        if (rn2 < thr) done = 1;
+        else if (!isfinite(rn2)) done = 5;
+        else {
+            const double absOld = absNew;
+            absNew = s2[1];
+            beta = absNew / absOld;
+            if (++it >= o.maxIt) done = 3;
+        }
+        p = z + beta * p;
+        double* const t = pOld;
+        pOld = pNew;
+        pNew = t;
+    }
+    if (ok) {   // the true residual of the result
+        if (own) storeAgent(c.x + i, x);
+        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        if (ok) {
+            const double tr = residual();
+            if (own) c.r[i] = tr;
+            publishSums<2>(part0, own ? tr * tr : 0.0, own ? b * b : 0.0);
+            ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+            sumPublished<2>(part0, s2);
+        }
+    }
+    if (own && lv) a.D[DPRESS][i] = (x < 0) ? 0.0 : x;   // setZeroOnNegativePressure
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.ds[S_RHSN2] = bn2;
+        a.ds[S_RN2] = rn2;
+        a.ds[S_TRUE_RN2] = s2[0];
+        a.ds[S_BN2] = s2[1];
+        a.is[I_CG_ITER] = it;
+        a.is[I_CG_DONE] = done;
+    }
+    leaveGrid(o.bar);
+}
+
+// solveMixed (Jacobi preconditioner) in one launch: the refinement loop on
+// the FP64 true residual around the FP32 PCG, and the pressure.
+template <int L, int BT>
+__global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaunch o) {
+    double* const win64 = reinterpret_cast<double*>(oneLaunchLds);
+    float* const win = reinterpret_cast<float*>(oneLaunchLds);
+    const int i = blockIdx.x * (BT / L) + threadIdx.x / L;
+    const bool row = i < a.N;
+    const bool own = row && groupLaneId<L>() == 0;
+    const int* const table = c.win + (size_t)(blockIdx.x * (BT / L) / kB) * kWinStride;
+    if (!o.full && a.is[I_NOWIN]) {   // every block leaves
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.is[I_GRID_LATE] = 1;
+        return;
+    }
+    const Window w = loadWindow(table, o.full, a.N);
+    const int KE = ellWidth(a.K), cap = win16Lds(a.N);
+    const int n = row ? c.cnt[i] : 0;
+    const double diag = row ? c.diag[i] : 1.0, b = row ? c.b[i] : 0.0;
+    const float diag32 = row ? c.diag32[i] : 1.0f, invd = row ? c.invd32[i] : 1.0f;
+    const bool lv = row && live(a, i);
+    double x = lv ? c.x[i] : 0.0;
+    double* const part0 = o.part;
+    double* const part1 = o.part + 2 * (size_t)gridDim.x;
+    float* const p2 = reinterpret_cast<float*>(o.p2);
+    unsigned epoch = 0;
+    int total = 0, outer = 0, done = 0;
+    double rn2 = 0.0, bn2 = 0.0, s2[2], s1[1];
+    bool ok = true;
+    for (;;) {
+        double r64;
+        if (outer == 0 && o.asmRed != nullptr) {
+            r64 = row ? c.r[i] : 0.0;
+            sumLeft<2>(o.asmRed, o.asmBlocks, s2);
+        } else {
+            if (own) storeAgent(c.x + i, x);
+            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            auto xOf = [&](int j) { return loadAgent(c.x + j); };
+            r64 = b - rowPublished<double, L>(c, c.val, w, win64, cap, n, KE, i, diag * x, xOf);
+            publishSums<2>(part0, own ? r64 * r64 : 0.0, own ? b * b : 0.0);
+            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            sumPublished<2>(part0, s2);
+        }
+        if (own) c.r[i] = r64;
+        rn2 = s2[0];
+        bn2 = s2[1];
+        if (!isfinite(rn2) || !isfinite(bn2)) break;
+        if (bn2 == 0.0) {   // zero right-hand side: x = 0, as the FP64 path
+            x = 0.0;
+            break;
+        }
+        if (rn2 < o.tol * o.tol * bn2 || outer >= o.maxOuter || total >= o.maxIt) break;
+        outer++;
+        // kMxInit
+        float r = (float)r64, z = invd * r, p = z;
+        double d = 0.0;
+        if (own) storeAgent(c.fz + i, z);
+        publishSums<2>(part1, own ? (double)r * (double)z : 0.0, own ? (double)r * (double)r : 0.0);
+        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        sumPublished<2>(part1, s2);
+        double absNew = s2[0];
+        const double in2 = s2[1];
+        const double thr = fmax(fmax(o.tolIn * o.tolIn * in2, 0.25 * o.tol * o.tol * bn2), DBL_MIN);   // kMxInitFinish
+        done = (in2 == 0.0) ? 2 : (isfinite(in2) && isfinite(absNew)) ? 0 : 5;
+        int it = 0;
+        double beta = 0.0;
+        float* pOld = c.fp;
+        float* pNew = p2;
+        for (bool first = true; !done; first = false) {
+            const float beta32 = (float)beta;
+            auto pOf = [&](int j) {
+                const float zj = loadAgent(c.fz + j);
+                return first ? zj : zj + beta32 * loadAgent(pOld + j);
+            };
+            const float q = (float)rowPublished<float, L>(c, c.val32, w, win, 2 * cap, n, KE, i,
+                                                          (double)(diag32 * p), pOf);
+            if (own) storeAgent(pNew + i, p);
+            publishSums<1>(part0, own ? (double)p * (double)q : 0.0, 0.0);
+            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            sumPublished<1>(part0, s1);
+            const float alpha = (float)(absNew / s1[0]);
+            d += (double)alpha * (double)p;
+            r = r - alpha * q;
+            z = invd * r;
+            if (own) storeAgent(c.fz + i, z);
+            publishSums<2>(part1, own ? (double)r * (double)r : 0.0, own ? (double)r * (double)z : 0.0);
+            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            sumPublished<2>(part1, s2);
+            if (s2[0] < thr) done = 1;
+            else if (!isfinite(s2[0])) done = 5;
+            else {
+                const double absOld = absNew;
+                absNew = s2[1];
+                beta = absNew / absOld;
+                if (++it >= o.maxIt) done = 3;
+            }
+            p = z + (float)beta * p;
+            float* const t = pOld;
+            pOld = pNew;
+            pNew = t;
+        }
+        if (!ok) break;
+        total += it + 1;
+        if (lv) x += d;   // kMxApply
+        if (done == 5) break;
+    }
+    if (own) c.x[i] = x;
+    if (own && lv) a.D[DPRESS][i] = (x < 0) ? 0.0 : x;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.ds[S_TRUE_RN2] = rn2;
+        a.ds[S_BN2] = bn2;
+        a.is[I_CG_ITER] = total;
+        a.is[I_CG_OUTER] = outer;
+        a.is[I_CG_DONE] = done;
+    }
+    leaveGrid(o.bar);
+}
+
 // ------------------------------------- flexible CG with the learned operator
 // Inner solve of the mixed path with z = M r (M from the learned operator):
 // p_{k+1} = z_{k+1} - (z_{k+1} . q_k) / (p_k . q_k) p_k, q_k = A p_k.
@@ -1304,6 +1859,7 @@ static CgPtrs cgPtrs(Ctx* ctx) {
     c.lc8 = ctx->aLc8;
     c.lcEsc = ctx->aLcEsc;
     c.win = ctx->winValid ? ctx->aWin : nullptr;
+    c.lc16 = ctx->aLc16;
     return c;
 }
 
@@ -1321,11 +1877,20 @@ static int ensureMixed(Ctx* ctx) {
     return MPS_OK;
 }
 
-static int ensureWindows(Ctx* ctx) {
-    if (ctx->aLc8) return MPS_OK;
-    MPS_HIP(hipMalloc(&ctx->aLc8, (size_t)ellWidth(ctx->K) * ellRows(ctx->N)));
-    MPS_HIP(hipMalloc(&ctx->aLcEsc, sizeof(unsigned short) * (size_t)kLcEsc * ellRows(ctx->N)));
-    MPS_HIP(hipMalloc(&ctx->aWin, sizeof(int) * (size_t)kWinStride * gridFor(ctx->N, kB)));
+// a periodic domain's window is the whole vector
+static bool periodicCtx(const Ctx* ctx) { return ctx->P.domain_type_bc == 1; }
+// rows few enough for a solve in one launch, whose 16-bit window indices the
+// assembly writes then
+static bool oneLaunchRows(const Ctx* ctx) { return ctx->N <= (periodicCtx(ctx) ? kFullMax : kOneLaunchMax); }
+
+static int ensureWindows(Ctx* ctx, bool bytes) {
+    if (!ctx->aWin) MPS_HIP(hipMalloc(&ctx->aWin, sizeof(int) * (size_t)kWinStride * gridFor(ctx->N, kB)));
+    if (bytes && !ctx->aLc8) {
+        MPS_HIP(hipMalloc(&ctx->aLc8, (size_t)ellWidth(ctx->K) * ellRows(ctx->N)));
+        MPS_HIP(hipMalloc(&ctx->aLcEsc, sizeof(unsigned short) * (size_t)kLcEsc * ellRows(ctx->N)));
+    }
+    if (oneLaunchRows(ctx) && !ctx->aLc16)
+        MPS_HIP(hipMalloc(&ctx->aLc16, sizeof(unsigned short) * (size_t)ellWidth(ctx->K) * ellRows(ctx->N)));
     return MPS_OK;
 }
 
@@ -1354,8 +1919,7 @@ int ppeAssemble(Ctx* ctx) {
     // I_NESC counts the escaped columns; the entry count is summed from the
     // row counts when asked for (reduceCounts), not by one same-address
     // atomic per wavefront here
-    MPS_HIP(hipMemsetAsync(ctx->is + I_NESC, 0, sizeof(int), ctx->stream));
-    MPS_HIP(hipMemsetAsync(ctx->is + I_NLCESC, 0, sizeof(int), ctx->stream));
+    MPS_HIP(hipMemsetAsync(ctx->is + I_NESC, 0, 3 * sizeof(int), ctx->stream));   // and I_NLCESC, I_NOWIN
     // the CG solve's first true residual comes out of the assembly (with the
     // learned warm start it is the residual the warm start corrects)
     const bool res = !bicg;
@@ -1363,14 +1927,18 @@ int ppeAssemble(Ctx* ctx) {
     double* invd64 = (res && !mixed) ? ctx->cgInvD : nullptr;
     const int bFirst = mixed ? 0 : 1;
     // the CG solves' LDS windows (ppe_window scalar)
+    // and those of a solve in one launch, whatever the scalar says
     const bool wins = !bicg && ctx->ppeWindow;
-    if (wins) {
-        int rc = ensureWindows(ctx);
+    const bool wins16 = !bicg && oneLaunchRows(ctx);
+    if (wins || wins16) {
+        int rc = ensureWindows(ctx, wins);
         if (rc) return rc;
     }
     unsigned char* lc8 = wins ? ctx->aLc8 : nullptr;
     unsigned short* lcEsc = wins ? ctx->aLcEsc : nullptr;
-    int* win = wins ? ctx->aWin : nullptr;
+    int* win = wins || wins16 ? ctx->aWin : nullptr;
+    unsigned short* lc16 = wins16 ? ctx->aLc16 : nullptr;
+    ctx->win16Valid = wins16;
     // Several lanes per row where one lane per row leaves the chip idle (a
     // row's ~120 entries one after the other take ~180 us whatever the count).
     // Us with one lane / 4 / 16 lanes and the window kernel: 178 / 70 / 33 at
@@ -1379,11 +1947,11 @@ int ppeAssemble(Ctx* ctx) {
     const int lanes = ctx->N <= 8192 ? 16 : (ctx->N <= 65536 ? 4 : 0);
     if (lanes != 0) {
         ctx->asmBlocks = gridFor(ctx->N, kB / lanes);
-        if (wins) hipLaunchKernelGGL(kPpeWindow, dim3(g), dim3(kB), 0, ctx->stream, a, win);
+        if (win) hipLaunchKernelGGL(kPpeWindow, dim3(g), dim3(kB), 0, ctx->stream, a, win);
 #define ASMG(L, TT, R, LL)                                                                                     \
     hipLaunchKernelGGL((kPpeAssembleGroup<L, TT, R, LL>), dim3(ctx->asmBlocks), dim3(kB), 0, ctx->stream, a,   \
                        ctx->aVal, ctx->aCol, ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->D[DPPEB], v32, d32, i32,   \
-                       invd64, x, ctx->cgR, bFirst, lc8, lcEsc, win)
+                       invd64, x, ctx->cgR, bFirst, lc8, lcEsc, win, lc16)
 #define ASMGL(L, TT, R)                        \
     do {                                       \
         if (lanes == 16) ASMG(L, TT, R, 16);   \
@@ -1410,20 +1978,26 @@ int ppeAssemble(Ctx* ctx) {
         return MPS_OK;
     }
     ctx->asmBlocks = g;
-#define ASM(L, TT, R)                                                                                          \
-    hipLaunchKernelGGL((kPpeAssemble<L, TT, R>), dim3(g), dim3(kB), 0, ctx->stream, a, ctx->aVal, ctx->aCol,   \
+#define ASM(L, TT, R, W)                                                                                          \
+    hipLaunchKernelGGL((kPpeAssemble<L, TT, R, W>), dim3(g), dim3(kB), 0, ctx->stream, a, ctx->aVal, ctx->aCol,   \
                        ctx->aEsc, ctx->aCnt, ctx->aDiag, ctx->D[DPPEB], v32, d32, i32, invd64, x, ctx->cgR, bFirst, \
-                       lc8, lcEsc, win)
-    if (res) {
+                       lc8, lcEsc, win, lc16)
+    if (res && wins16) {
         if (ctx->listValid) {
-            if (T) ASM(true, true, true); else ASM(true, false, true);
+            if (T) ASM(true, true, true, true); else ASM(true, false, true, true);
         } else {
-            if (T) ASM(false, true, true); else ASM(false, false, true);
+            if (T) ASM(false, true, true, true); else ASM(false, false, true, true);
+        }
+    } else if (res) {
+        if (ctx->listValid) {
+            if (T) ASM(true, true, true, false); else ASM(true, false, true, false);
+        } else {
+            if (T) ASM(false, true, true, false); else ASM(false, false, true, false);
         }
     } else if (ctx->listValid) {
-        if (T) ASM(true, true, false); else ASM(true, false, false);
+        if (T) ASM(true, true, false, false); else ASM(true, false, false, false);
     } else {
-        if (T) ASM(false, true, false); else ASM(false, false, false);
+        if (T) ASM(false, true, false, false); else ASM(false, false, false, false);
     }
 #undef ASM
     MPS_HIP(hipGetLastError());
@@ -1728,11 +2302,95 @@ static int solveBicgstab(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int 
     return MPS_OK;
 }
 
+// The kernel, threads and rows per block of a solve in one launch (kernel null: too many rows).
+struct OneLaunchKind {
+    const void* kernel;
+    int threads, rows;
+};
+static OneLaunchKind oneLaunchKind(int N, bool mixed) {
+    if (N <= 16384) return {mixed ? (const void*)kMxOneLaunch<16, 1024> : (const void*)kCgOneLaunch<16, 1024>, 1024, 64};
+    if (N <= 65536) return {mixed ? (const void*)kMxOneLaunch<4, 1024> : (const void*)kCgOneLaunch<4, 1024>, 1024, 256};
+    if (N <= kOneLaunchMax) return {mixed ? (const void*)kMxOneLaunch<2, 512> : (const void*)kCgOneLaunch<2, 512>, 512, 256};
+    return {nullptr, 0, 0};
+}
+
+// Whether the CG solve of the last assembly runs in one launch: it left the
+// 16-bit window indices, and the device holds every block of the grid at once
+// (asked of the runtime for the kernel, once per context).  Not while SpMV
+// launches are timed one by one.
+static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
+    *fits = false;
+    if (ctx->profile || !ctx->win16Valid) return MPS_OK;
+    const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
+    if (!k.kernel) return MPS_OK;
+    const int nb = gridFor(ctx->N, k.rows);
+    const size_t lds = sizeof(double) * (size_t)win16Lds(ctx->N);
+    if (ctx->oneLaunchFits[mixed] < 0) {
+        int cus = 0, perCu = 0;
+        MPS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->dev));
+        MPS_HIP(hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        MPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k.kernel, k.threads, lds));
+        ctx->oneLaunchFits[mixed] = nb <= perCu * cus ? 1 : 0;
+    }
+    if (!ctx->oneLaunchFits[mixed]) return MPS_OK;
+    if (!ctx->gridBar) {
+        const size_t bytes = sizeof(unsigned) * (kGridBars + 1) * kBarStride;
+        MPS_HIP(hipMalloc(&ctx->gridBar, bytes));
+        MPS_HIP(hipMemsetAsync(ctx->gridBar, 0, bytes, ctx->stream));
+        MPS_HIP(hipMalloc(&ctx->gridPart, sizeof(double) * 4 * (size_t)nb));
+        MPS_HIP(hipMalloc(&ctx->gridP2, sizeof(double) * (size_t)ctx->N));
+    }
+    *fits = true;
+    return MPS_OK;
+}
+
+// *solved: false when a block has no window or a grid barrier gave up; the guess and the system are
+// still valid then and the solve goes on in pieces.
+static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c, double tol, double tolIn, int maxIt,
+                           int maxOuter, bool* solved) {
+    const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
+    const bool fresh = ctx->r0Fresh && ctx->r0FreshMixed == mixed;
+    ctx->r0Fresh = false;
+    OneLaunch o;
+    o.bar = ctx->gridBar;
+    o.part = ctx->gridPart;
+    o.p2 = ctx->gridP2;
+    o.asmRed = fresh ? ctx->asmRed : nullptr;
+    o.asmBlocks = ctx->asmBlocks;
+    o.full = periodicCtx(ctx) ? 1 : 0;
+    o.tol = tol;
+    o.tolIn = tolIn;
+    o.maxIt = maxIt;
+    o.maxOuter = maxOuter;
+    KArgs ka = a;
+    CgPtrs kc = c;
+    kc.win = ctx->aWin;
+    void* args[] = {&ka, &kc, &o};
+    MPS_HIP(hipLaunchKernel(k.kernel, dim3(gridFor(ctx->N, k.rows)), dim3(k.threads), args,
+                            sizeof(double) * (size_t)win16Lds(ctx->N), ctx->stream));
+    const int rc = readStatus(ctx, nullptr, 0);
+    if (rc) return rc;
+    *solved = ctx->hostInts[I_GRID_LATE] == 0;
+    if (!*solved) MPS_HIP(hipMemsetAsync(ctx->is + I_GRID_LATE, 0, sizeof(int), ctx->stream));
+    return MPS_OK;
+}
+
 // Eigen-semantics Jacobi-PCG in FP64 (solveConjugateGradient, src/MpsPressure.cpp:424-445)
-static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batch) {
+static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batch, bool* oneLaunch) {
     hipStream_t s = ctx->stream;
     const double tol = ctx->P.solver_tol > 0 ? ctx->P.solver_tol : DBL_EPSILON;
     const int maxIt = ctx->P.solver_max_iter > 0 ? ctx->P.solver_max_iter : 2 * ctx->nLiveHost;
+    int rcL;
+    if ((rcL = oneLaunchFits(ctx, false, oneLaunch))) return rcL;
+    if (*oneLaunch && (rcL = launchOneLaunch(ctx, false, a, c, tol, 0.0, maxIt, 0, oneLaunch))) return rcL;
+    if (*oneLaunch) {
+        ctx->lastCgIters = ctx->hostInts[I_CG_ITER];
+        ctx->lastDone = ctx->hostInts[I_CG_DONE];
+        ctx->solverIter = ctx->hostInts[I_CG_ITER];
+        ctx->outerIter = 1;
+        ctx->solverErr = ctx->hostScalars[S_RHSN2] > 0 ? sqrt(ctx->hostScalars[S_RN2] / ctx->hostScalars[S_RHSN2]) : 0.0;
+        return MPS_OK;
+    }
     // r = b - A x, 1 / diag and the partials may come from the assembly
     const bool fresh = ctx->r0Fresh && !ctx->r0FreshMixed;
     if (!fresh) hipLaunchKernelGGL(kCgStart, dim3(nb), dim3(kB), 0, s, a, c);
@@ -1779,7 +2437,7 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
 
 // Mixed precision: FP64 iterative refinement on the true residual around an
 // FP32 Jacobi-PCG (FP64 dot products).  Stops when |b - A x| < tol |b| in FP64.
-static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batch) {
+static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batch, bool* oneLaunch) {
     constexpr int kMaxOuter = 30;
     // A refinement pass with the learned preconditioner ends after this many
     // iterations: an operator that neither converges nor breaks down (a
@@ -1801,6 +2459,17 @@ static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int bat
     int total = 0, outer = 0, rc;
     double prevRn2 = 0.0;
     ctx->lastDone = 0;
+    if (!useM) {
+        if ((rc = oneLaunchFits(ctx, true, oneLaunch))) return rc;
+        if (*oneLaunch && (rc = launchOneLaunch(ctx, true, a, c, tol, tolIn, maxIt, kMaxOuter, oneLaunch))) return rc;
+        if (*oneLaunch) {
+            ctx->solverIter = ctx->hostInts[I_CG_ITER];
+            ctx->outerIter = ctx->hostInts[I_CG_OUTER];
+            ctx->lastDone = ctx->hostInts[I_CG_DONE];
+            ctx->solverErr = ctx->hostScalars[S_BN2] > 0 ? sqrt(ctx->hostScalars[S_TRUE_RN2] / ctx->hostScalars[S_BN2]) : 0.0;
+            return MPS_OK;
+        }
+    }
     // when profiling, the entry count (for the SpMV bytes) is summed on the
     // device and comes with the next status read
     if (ctx->profile && (rc = launchCountToScalar(ctx, ctx->aCnt, ctx->N, S_NNZ))) return rc;
@@ -1967,19 +2636,21 @@ int ppeSolve(Ctx* ctx) {
         if ((rc = gnnForward(ctx))) return rc;
         if ((rc = gnnWarmStart(ctx))) return rc;
     }
+    // a solve in one launch ends with its true residual and the pressure
+    bool oneLaunch = false;
     if (bicg) rc = solveBicgstab(ctx, a, c, nb, batch);
-    else rc = mixed ? solveMixed(ctx, a, c, nb, batch) : solveFp64(ctx, a, c, nb, batch);
+    else rc = mixed ? solveMixed(ctx, a, c, nb, batch, &oneLaunch) : solveFp64(ctx, a, c, nb, batch, &oneLaunch);
     if (rc) return rc;
-    if (!mixed) {   // the mixed path ends on a fresh true residual already
+    if (!mixed && !oneLaunch) {   // the mixed path ends on a fresh true residual already
         hipLaunchKernelGGL(kTrueResidual, dim3(nb), dim3(kB), 0, s, a, c);
         hipLaunchKernelGGL(kTrueResidualFinish, dim3(1), dim3(1024), 0, s, a, nb);
     }
-    hipLaunchKernelGGL(kPressFromX, dim3(nb), dim3(kB), 0, s, a, c.x);
+    if (!oneLaunch) hipLaunchKernelGGL(kPressFromX, dim3(nb), dim3(kB), 0, s, a, c.x);
     MPS_HIP(hipEventRecord(ctx->ev1, s));
     // the mixed path's last status read already holds the final true
     // residual; the other paths read the one computed above.  The solve's
     // time is read from its events when asked for (ppeSolveMs).
-    if (!mixed && (rc = readStatus(ctx, nullptr, 0))) return rc;
+    if (!mixed && !oneLaunch && (rc = readStatus(ctx, nullptr, 0))) return rc;
     MPS_HIP(hipGetLastError());
     ctx->ppeMsPending = true;
     const double* hs = ctx->hostScalars;
