@@ -326,25 +326,32 @@ __global__ __launch_bounds__(256) void kGnnMessage(int n, const int* gcol, const
 }
 
 // -------------------------------------------------------------------- head
+// Thread = (node, every kHeadLanes-th edge): the edges' couplings do not
+// depend on each other (one thread per node: 57 us at 71,463 nodes, now 40).
+constexpr int kHeadLanes = 4;
+
 __global__ __launch_bounds__(256) void kGnnHead(int n, const int* gcol, const int* gcnt, const float4* ge,
                                                 const unsigned short* AB, const unsigned short* h, const float* th,
                                                 const float* da, const float* ainv, float* cs, float* dsi, float* uo,
                                                 float* so) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int l = threadIdx.x % kHeadLanes;
+    const int i = blockIdx.x * (256 / kHeadLanes) + threadIdx.x / kHeadLanes;
     if (i >= n) return;
     float pa[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) pa[q] = fromBf16(AB[(size_t)i * 32 + q]) + th[gnn::oP + q];
-    float u = th[gnn::oBd];
+    if (l == 0) {
+        float u = th[gnn::oBd];
 #pragma unroll
-    for (int ch = 0; ch < H; ch++) u += th[gnn::oVd + ch] * fromBf16(h[(size_t)i * H + ch]);
-    const float s = expf(fminf(fmaxf(u, -3.f), 3.f));
-    uo[i] = u;
-    so[i] = s;
-    dsi[i] = s * ainv[i];
+        for (int ch = 0; ch < H; ch++) u += th[gnn::oVd + ch] * fromBf16(h[(size_t)i * H + ch]);
+        const float s = expf(fminf(fmaxf(u, -3.f), 3.f));
+        uo[i] = u;
+        so[i] = s;
+        dsi[i] = s * ainv[i];
+    }
     const float dai = da[i];
     const int cnt = gcnt[i];
-    for (int e = 0; e < cnt; e++) {
+    for (int e = l; e < cnt; e += kHeadLanes) {
         const size_t o = (size_t)e * n + i;
         const int j = gcol[o];
         const float4 ef = ge[o];
@@ -360,16 +367,30 @@ __global__ __launch_bounds__(256) void kGnnHead(int n, const int* gcol, const in
     }
 }
 
-// z = M r (FP32)
-__global__ void kGnnApply(int n, const int* gcol, const int* gcnt, const float* cs, const float* dsi, const float* r,
-                          float* z) {
+// z = M r (FP32); eight edges' gathers in flight (one after the other: 16 us
+// at 71,463 nodes, now 6)
+__global__ void kGnnApply(int n, const int* __restrict__ gcol, const int* __restrict__ gcnt,
+                          const float* __restrict__ cs, const float* __restrict__ dsi, const float* __restrict__ r,
+                          float* __restrict__ z) {
+    constexpr int B = 8;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float acc = dsi[i] * r[i];
     const int cnt = gcnt[i];
-    for (int e = 0; e < cnt; e++) {
-        const size_t o = (size_t)e * n + i;
-        acc += cs[o] * r[gcol[o]];
+    for (int e0 = 0; e0 < cnt; e0 += B) {
+        int j[B];
+        float c[B], v[B];
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+            const size_t o = (size_t)min(e0 + q, cnt - 1) * n + i;
+            j[q] = gcol[o];
+            c[q] = cs[o];
+        }
+#pragma unroll
+        for (int q = 0; q < B; q++) v[q] = r[j[q]];
+#pragma unroll
+        for (int q = 0; q < B; q++)
+            if (e0 + q < cnt) acc += c[q] * v[q];
     }
     z[i] = acc;
 }
@@ -381,98 +402,113 @@ __global__ void kGnnAddFloat(KArgs a, const float* z, double* x) {
 }
 
 // ------------------------------------------------------------------ backward
-// Node terms of the operator and the diagonal head; initialises dh.
-__global__ void kGnnBwdNode(int n, const float* gz, const float* r, const float* ainv, const float* s, const float* u,
-                            const unsigned short* h, const float* th, float* dh, float* grad) {
-    __shared__ float red[H + 1];
-    if (threadIdx.x <= H) red[threadIdx.x] = 0.f;
-    __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
+constexpr int kEdgeBatch = 4;
+constexpr int kBwdBlocks = 1024;   // about what the chip holds at once: the sums stay in registers over a block's nodes
+
+// Node terms of the operator and the diagonal head; initialises dh.  Thread =
+// (node, channel), so that a channel's sum needs no atomic per node (with
+// them, a wavefront's 64 on one LDS word: 72 us at 71,463 nodes, now 28).
+__global__ __launch_bounds__(256) void kGnnBwdNode(int n, const float* __restrict__ gz, const float* __restrict__ r,
+                                                   const float* __restrict__ ainv, const float* __restrict__ s,
+                                                   const float* __restrict__ u, const unsigned short* __restrict__ h,
+                                                   const float* __restrict__ th, float* __restrict__ dh,
+                                                   float* grad) {
+    __shared__ float sh[4][H + 1];
+    const int ch = threadIdx.x % H, half = (threadIdx.x & 63) / H;
+    const float vd = th[gnn::oVd + ch];
+    float gv = 0.f, gd = 0.f;
+    for (int i = blockIdx.x * (256 / H) + threadIdx.x / H; i < n; i += gridDim.x * (256 / H)) {
         const float ds = gz[i] * r[i] * ainv[i];
         const float du = (u[i] > -3.f && u[i] < 3.f) ? ds * s[i] : 0.f;
-#pragma unroll
-        for (int ch = 0; ch < H; ch++) {
-            dh[(size_t)i * H + ch] = du * th[gnn::oVd + ch];
-            atomicAdd(&red[ch], du * fromBf16(h[(size_t)i * H + ch]));
-        }
-        atomicAdd(&red[H], du);
+        dh[(size_t)i * H + ch] = du * vd;
+        gv += du * fromBf16(h[(size_t)i * H + ch]);
+        gd += du;
+    }
+    gv += __shfl_xor(gv, H, 64);
+    gd += __shfl_xor(gd, H, 64);
+    if (half == 0) {
+        sh[threadIdx.x >> 6][ch] = gv;
+        if (ch == 0) sh[threadIdx.x >> 6][H] = gd;
     }
     __syncthreads();
-    if (threadIdx.x < H) atomicAdd(&grad[gnn::oVd + threadIdx.x], red[threadIdx.x]);
-    if (threadIdx.x == H) atomicAdd(&grad[gnn::oBd], red[H]);
+    if (threadIdx.x <= H) {
+        const float t = (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
+        atomicAdd(threadIdx.x < H ? &grad[gnn::oVd + threadIdx.x] : &grad[gnn::oBd], t);
+    }
 }
 
-// Edge head, row side: dPA_i and the v, Pe, p gradients.  Thread = (node, q).
-__global__ __launch_bounds__(256) void kGnnBwdHeadI(int n, const int* gcol, const int* gcnt, const float4* ge,
-                                                    const unsigned short* AB, const float* th, const float* da,
-                                                    const float* gz, const float* r, float* dAB, float* grad) {
-    __shared__ float red[Q * 6];
-    for (int k = threadIdx.x; k < Q * 6; k += blockDim.x) red[k] = 0.f;
-    __syncthreads();
-    const int q = threadIdx.x & (Q - 1);
-    const int i = blockIdx.x * (blockDim.x / Q) + threadIdx.x / Q;
-    float dPA = 0.f, dv = 0.f, dp = 0.f, dpe0 = 0.f, dpe1 = 0.f, dpe2 = 0.f, dpe3 = 0.f;
-    if (i < n) {
-        const float* pe = th + gnn::oPe + q * 4;
-        const float pa = fromBf16(AB[(size_t)i * 32 + q]) + th[gnn::oP + q];
-        const float vq = th[gnn::oV + q];
-        const float gi = gz[i] * da[i];
-        const int cnt = gcnt[i];
-        for (int e = 0; e < cnt; e++) {
-            const size_t o = (size_t)e * n + i;
-            const int j = gcol[o];
-            const float4 ef = ge[o];
-            const float tp = pa + fromBf16(AB[(size_t)j * 32 + Q + q]) + pe[0] * ef.x + pe[1] * ef.y + pe[2] * ef.z +
-                             pe[3] * ef.w;
-            const float dc = gi * r[j] * da[j];
-            dv += dc * relu(tp);
-            if (tp > 0.f) {
-                const float dt = dc * vq;
-                dPA += dt;
-                dp += dt;
-                dpe0 += dt * ef.x; dpe1 += dt * ef.y; dpe2 += dt * ef.z; dpe3 += dt * ef.w;
+// Edge head.  Row side: dPA_m over the edges m <- j, and the v, Pe, p
+// gradients; column side: dPB_m over the edges j <- m, visited from m's own
+// list (the reS graph is symmetric; e_mj = -e_jm in position, same w).
+// Thread = (node m, q), both sides from one pass over the list, kEdgeBatch
+// edges in flight (two kernels, an edge after the other, LDS atomics for the
+// sums: 155 + 86 us at 71,463 nodes, now 71).
+__global__ __launch_bounds__(256) void kGnnBwdHead(int n, const int* __restrict__ gcol, const int* __restrict__ gcnt,
+                                                   const float4* __restrict__ ge,
+                                                   const unsigned short* __restrict__ AB,
+                                                   const float* __restrict__ th, const float* __restrict__ da,
+                                                   const float* __restrict__ gz, const float* __restrict__ r,
+                                                   float* __restrict__ dAB, float* grad) {
+    constexpr int B = kEdgeBatch;
+    __shared__ float sh[4][Q * 6];
+    const int q = threadIdx.x % Q;
+    const float4 pe = *reinterpret_cast<const float4*>(th + gnn::oPe + q * 4);
+    const float pq = th[gnn::oP + q], vq = th[gnn::oV + q];
+    float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // v, p, Pe
+    for (int m = blockIdx.x * (256 / Q) + threadIdx.x / Q; m < n; m += gridDim.x * (256 / Q)) {
+        const float pa = fromBf16(AB[(size_t)m * 32 + q]) + pq, pb = fromBf16(AB[(size_t)m * 32 + Q + q]) + pq;
+        const float dm = da[m], gi = gz[m] * dm, rm = r[m] * dm;
+        const int cnt = gcnt[m];
+        float dPA = 0.f, dPB = 0.f;
+        for (int e0 = 0; e0 < cnt; e0 += B) {
+            int j[B];
+            float4 f[B];
+            float A[B], Bj[B], rj[B], dj[B], gj[B];
+#pragma unroll
+            for (int k = 0; k < B; k++) {   // past the end: the last edge again, not used
+                const size_t o = (size_t)min(e0 + k, cnt - 1) * n + m;
+                j[k] = gcol[o];
+                f[k] = ge[o];
+            }
+#pragma unroll
+            for (int k = 0; k < B; k++) {
+                A[k] = fromBf16(AB[(size_t)j[k] * 32 + q]);
+                Bj[k] = fromBf16(AB[(size_t)j[k] * 32 + Q + q]);
+                rj[k] = r[j[k]];
+                dj[k] = da[j[k]];
+                gj[k] = gz[j[k]];
+            }
+#pragma unroll
+            for (int k = 0; k < B; k++) {
+                if (e0 + k >= cnt) break;
+                const float tr = pa + Bj[k] + pe.x * f[k].x + pe.y * f[k].y + pe.z * f[k].z + pe.w * f[k].w;
+                const float dc = gi * rj[k] * dj[k];
+                t[0] += dc * relu(tr);
+                if (tr > 0.f) {
+                    const float dt = dc * vq;
+                    dPA += dt;
+                    t[1] += dt;
+                    t[2] += dt * f[k].x; t[3] += dt * f[k].y; t[4] += dt * f[k].z; t[5] += dt * f[k].w;
+                }
+                const float tc = A[k] + pb - pe.x * f[k].x - pe.y * f[k].y - pe.z * f[k].z + pe.w * f[k].w;
+                if (tc > 0.f) dPB += gj[k] * dj[k] * rm * vq;
             }
         }
-        dAB[(size_t)i * 32 + q] = dPA;
+        dAB[(size_t)m * 32 + q] = dPA;
+        dAB[(size_t)m * 32 + Q + q] = dPB;
     }
-    atomicAdd(&red[q], dv);
-    atomicAdd(&red[Q + q], dp);
-    atomicAdd(&red[2 * Q + q * 4], dpe0);
-    atomicAdd(&red[2 * Q + q * 4 + 1], dpe1);
-    atomicAdd(&red[2 * Q + q * 4 + 2], dpe2);
-    atomicAdd(&red[2 * Q + q * 4 + 3], dpe3);
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        t[k] += __shfl_xor(t[k], 16, 64);
+        t[k] += __shfl_xor(t[k], 32, 64);
+        if ((threadIdx.x & 63) < Q) sh[threadIdx.x >> 6][k < 2 ? k * Q + q : 2 * Q + q * 4 + k - 2] = t[k];
+    }
     __syncthreads();
-    for (int k = threadIdx.x; k < Q * 6; k += blockDim.x) {
-        if (k < Q) atomicAdd(&grad[gnn::oV + k], red[k]);
-        else if (k < 2 * Q) atomicAdd(&grad[gnn::oP + k - Q], red[k]);
-        else atomicAdd(&grad[gnn::oPe + k - 2 * Q], red[k]);
+    const int k = threadIdx.x;
+    if (k < Q * 6) {
+        const float g = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+        atomicAdd(&grad[k < Q ? gnn::oV + k : k < 2 * Q ? gnn::oP + k - Q : gnn::oPe + k - 2 * Q], g);
     }
-}
-
-// Edge head, column side: dPB_j = sum over edges i <- j, visited from j's
-// own list (the reS graph is symmetric; e_ij = -e_ji in position, same w).
-__global__ __launch_bounds__(256) void kGnnBwdHeadJ(int n, const int* gcol, const int* gcnt, const float4* ge,
-                                                    const unsigned short* AB, const float* th, const float* da,
-                                                    const float* gz, const float* r, float* dAB) {
-    const int q = threadIdx.x & (Q - 1);
-    const int j = blockIdx.x * (blockDim.x / Q) + threadIdx.x / Q;
-    if (j >= n) return;
-    const float* pe = th + gnn::oPe + q * 4;
-    const float pb = fromBf16(AB[(size_t)j * 32 + Q + q]) + th[gnn::oP + q];
-    const float vq = th[gnn::oV + q];
-    const float rj = r[j] * da[j];
-    const int cnt = gcnt[j];
-    float acc = 0.f;
-    for (int e = 0; e < cnt; e++) {
-        const size_t o = (size_t)e * n + j;
-        const int i = gcol[o];
-        const float4 ef = ge[o];
-        const float tp = fromBf16(AB[(size_t)i * 32 + q]) + pb - pe[0] * ef.x - pe[1] * ef.y - pe[2] * ef.z +
-                         pe[3] * ef.w;
-        if (tp > 0.f) acc += gz[i] * da[i] * rj * vq;
-    }
-    dAB[(size_t)j * 32 + Q + q] = acc;
 }
 
 // dA = dh * [a > 0]
@@ -483,117 +519,157 @@ __global__ void kGnnMask(int n, const float* dh, const unsigned short* a, float*
 }
 
 // Messages, column side: dG_j = sum over edges i <- j of om_ij dm_i [q_ij > 0]
-// and the E, c gradients.  Thread = (node, 8-channel group).
-__global__ __launch_bounds__(256) void kGnnBwdMessage(int n, const int* gcol, const int* gcnt, const float4* ge,
-                                                      const float* gw, const float* wsum, const unsigned short* G,
-                                                      const float* E, const float* cb, const float* dm, float* dG,
-                                                      float* gE, float* gc) {
-    __shared__ float red[H * 5];
-    for (int k = threadIdx.x; k < H * 5; k += blockDim.x) red[k] = 0.f;
-    __syncthreads();
-    const int grp = threadIdx.x & 3;
-    const int j = blockIdx.x * (blockDim.x / 4) + threadIdx.x / 4;
-    float acc[8], pE[8][4], pc[8];
+// and the E, c gradients.  Thread = (node, 8-channel group); bound by the
+// loads per edge (a node's lanes repeat the edge's own) and the chain list
+// entry -> gathered row, so two edges are loaded together, as many as the
+// registers hold.  The E, c sums stay in registers over a block's nodes and
+// go through shuffles.  One edge after the other and the sums added to LDS by
+// every thread: 242 us at 71,463 nodes; 4 channels and four edges: 83; this: 75.
+__global__ __launch_bounds__(256) void kGnnBwdMessage(int n, const int* __restrict__ gcol, const int* __restrict__ gcnt,
+                                                      const float4* __restrict__ ge, const float* __restrict__ gw,
+                                                      const float* __restrict__ wsum,
+                                                      const unsigned short* __restrict__ G,
+                                                      const float* __restrict__ E, const float* __restrict__ cb,
+                                                      const float* __restrict__ dm, float* __restrict__ dG, float* gE,
+                                                      float* gc) {
+    constexpr int C = 8, GR = H / C, B = 2;
+    __shared__ float sh[4][H * 5];
+    const int grp = threadIdx.x % GR, c0 = grp * C;
+    float Er[C][4], cr[C], pE[C][4], pc[C];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        acc[k] = 0.f; pc[k] = 0.f;
-        pE[k][0] = pE[k][1] = pE[k][2] = pE[k][3] = 0.f;
+    for (int k = 0; k < C; k++) {
+        const float4 e4 = reinterpret_cast<const float4*>(E)[c0 + k];
+        Er[k][0] = e4.x; Er[k][1] = e4.y; Er[k][2] = e4.z; Er[k][3] = e4.w;
+        cr[k] = cb[c0 + k];
+        pc[k] = pE[k][0] = pE[k][1] = pE[k][2] = pE[k][3] = 0.f;
     }
-    if (j < n) {
-        float g[8];
+    for (int j = blockIdx.x * (256 / GR) + threadIdx.x / GR; j < n; j += gridDim.x * (256 / GR)) {
+        float acc[C], g[C];
+        const uint4 gv = *reinterpret_cast<const uint4*>(G + (size_t)j * H + c0);
+        const unsigned gw4[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
-        for (int k = 0; k < 8; k++) g[k] = fromBf16(G[(size_t)j * H + grp * 8 + k]);
+        for (int k = 0; k < C; k++)
+            g[k] = __uint_as_float((k & 1) ? (gw4[k >> 1] & 0xFFFF0000u) : (gw4[k >> 1] << 16));
+#pragma unroll
+        for (int k = 0; k < C; k++) acc[k] = 0.f;
         const int cnt = gcnt[j];
-        for (int e = 0; e < cnt; e++) {
-            const size_t o = (size_t)e * n + j;
-            const int i = gcol[o];
-            const float4 f = ge[o];
-            const float ex = -f.x, ey = -f.y, ez = -f.z, ew = f.w;
-            const float ws = wsum[i];
-            const float om = ws > 0.f ? gw[o] / ws : 0.f;
+        for (int e0 = 0; e0 < cnt; e0 += B) {
+            int i[B];
+            float4 f[B], d[B][2];
+            float w[B], ws[B];
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int ch = grp * 8 + k;
-                const float q = g[k] + E[ch * 4] * ex + E[ch * 4 + 1] * ey + E[ch * 4 + 2] * ez + E[ch * 4 + 3] * ew + cb[ch];
-                if (q > 0.f) {
-                    const float dq = om * dm[(size_t)i * H + ch];
+            for (int q = 0; q < B; q++) {   // past the end: the last edge again, with weight 0
+                const size_t o = (size_t)min(e0 + q, cnt - 1) * n + j;
+                i[q] = gcol[o];
+                f[q] = ge[o];
+                w[q] = gw[o];
+            }
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                ws[q] = wsum[i[q]];
+                d[q][0] = *reinterpret_cast<const float4*>(dm + (size_t)i[q] * H + c0);
+                d[q][1] = *reinterpret_cast<const float4*>(dm + (size_t)i[q] * H + c0 + 4);
+            }
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                if (e0 + q >= cnt) break;
+                const float ex = -f[q].x, ey = -f[q].y, ez = -f[q].z, ew = f[q].w;
+                const float om = ws[q] > 0.f ? w[q] / ws[q] : 0.f;
+                const float dv[C] = {d[q][0].x, d[q][0].y, d[q][0].z, d[q][0].w, d[q][1].x, d[q][1].y, d[q][1].z, d[q][1].w};
+#pragma unroll
+                for (int k = 0; k < C; k++) {
+                    const float t = g[k] + Er[k][0] * ex + Er[k][1] * ey + Er[k][2] * ez + Er[k][3] * ew + cr[k];
+                    const float dq = t > 0.f ? om * dv[k] : 0.f;
                     acc[k] += dq;
                     pc[k] += dq;
                     pE[k][0] += dq * ex; pE[k][1] += dq * ey; pE[k][2] += dq * ez; pE[k][3] += dq * ew;
                 }
             }
         }
-#pragma unroll
-        for (int k = 0; k < 8; k++) dG[(size_t)j * H + grp * 8 + k] = acc[k];
+        *reinterpret_cast<float4*>(dG + (size_t)j * H + c0) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        *reinterpret_cast<float4*>(dG + (size_t)j * H + c0 + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
     }
+    // over the wave's nodes (lanes of the same channel group), then its four waves
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int ch = grp * 8 + k;
-        atomicAdd(&red[ch], pc[k]);
-        atomicAdd(&red[H + ch * 4], pE[k][0]);
-        atomicAdd(&red[H + ch * 4 + 1], pE[k][1]);
-        atomicAdd(&red[H + ch * 4 + 2], pE[k][2]);
-        atomicAdd(&red[H + ch * 4 + 3], pE[k][3]);
+    for (int k = 0; k < C; k++) {
+#pragma unroll
+        for (int m = GR; m < 64; m <<= 1) {
+            pc[k] += __shfl_xor(pc[k], m, 64);
+#pragma unroll
+            for (int x = 0; x < 4; x++) pE[k][x] += __shfl_xor(pE[k][x], m, 64);
+        }
+        if ((threadIdx.x & 63) < GR) {
+            float* const t = sh[threadIdx.x >> 6];
+            t[c0 + k] = pc[k];
+#pragma unroll
+            for (int x = 0; x < 4; x++) t[H + (c0 + k) * 4 + x] = pE[k][x];
+        }
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < H * 5; k += blockDim.x) {
-        if (k < H) atomicAdd(&gc[k], red[k]);
-        else atomicAdd(&gE[k - H], red[k]);
+    for (int k = threadIdx.x; k < H * 5; k += 256) {
+        const float t = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+        if (k < H) atomicAdd(&gc[k], t);
+        else atomicAdd(&gE[k - H], t);
     }
 }
 
 // Weight gradients gW[o][k] += sum_i dY[i][o] X[i][k] (X = [X1 | X2]) and
-// gb[o] += sum_i dY[i][o].  Blocks take 32-node tiles through LDS.
-template <int O, int K, typename XT>
-__global__ __launch_bounds__(256) void kGnnWGrad(int n, int nodesPerBlock, const float* dY, const XT* X1, const XT* X2,
-                                                 float* gW, float* gb) {
-    __shared__ float sY[32][O];
-    __shared__ float sX[32][K];
-    constexpr int NP = O * K + O;
-    constexpr int PER = (NP + 255) / 256;
-    float acc[PER];
+// gb[o] += sum_i dY[i][o], FP32.  The sum over the nodes is a contraction:
+// v_mfma_f32_32x32x2_f32 takes two nodes at a time with lane l supplying
+// dY[i + l / 32][l % 32] and X[i + l / 32][l % 32] (one coalesced load each)
+// and receiving gW[8 (v / 4) + 4 (l / 32) + v % 4][l % 32], v = 0 .. 15.  The
+// kernel reads dY and X once (18 MB for 71,463 nodes and K = 64); kWGradBlocks
+// blocks, one per CU, keep enough loads in flight and few enough atomic sums.
+// With a 32-node tile in LDS, dot products per thread and a block per 2,048
+// nodes it took 591 us at that size (K = 32: 255), now 24 (19).
+constexpr int kWGradBlocks = 256;
+
+template <int K, typename XT>
+__global__ __launch_bounds__(256) void kGnnWGrad(int n, int nodesPerBlock, const float* __restrict__ dY,
+                                                 const XT* __restrict__ X1, const XT* __restrict__ X2, float* gW,
+                                                 float* gb) {
+    typedef float F16 __attribute__((ext_vector_type(16)));
+    constexpr int T = K > 32 ? 2 : 1;   // 32-column tiles
+    constexpr int B = 8;                // node pairs in flight
+    constexpr int ROW = K == 4 ? 4 : 32;
+    __shared__ float sh[4][32 * K + 32];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ch = lane & 31, half = lane >> 5;
+    F16 acc[T];
 #pragma unroll
-    for (int p = 0; p < PER; p++) acc[p] = 0.f;
-    const int start = blockIdx.x * nodesPerBlock;
-    const int stop = min(n, start + nodesPerBlock);
-    for (int t0 = start; t0 < stop; t0 += 32) {
-        __syncthreads();
-        for (int k = threadIdx.x; k < 32 * O; k += 256) {
-            const int r = k / O, c = k % O, i = t0 + r;
-            sY[r][c] = (i < stop) ? dY[(size_t)i * O + c] : 0.f;
-        }
-        for (int k = threadIdx.x; k < 32 * K; k += 256) {
-            const int r = k / K, c = k % K, i = t0 + r;
-            float v = 0.f;
-            if (i < stop) {
-                if (K == 4) v = reinterpret_cast<const float*>(X1)[(size_t)i * 4 + c];
-                else if (c < 32) v = (float)X1[(size_t)i * 32 + c];
-                else v = (float)X2[(size_t)i * 32 + c - 32];
-            }
-            sX[r][c] = v;
-        }
-        __syncthreads();
+    for (int t = 0; t < T; t++)
 #pragma unroll
-        for (int p = 0; p < PER; p++) {
-            const int idx = threadIdx.x + p * 256;
-            if (idx < O * K) {
-                const int o = idx / K, k = idx % K;
-                float s = 0.f;
-                for (int r = 0; r < 32; r++) s += sY[r][o] * sX[r][k];
-                acc[p] += s;
-            } else if (idx < NP) {
-                const int o = idx - O * K;
-                float s = 0.f;
-                for (int r = 0; r < 32; r++) s += sY[r][o];
-                acc[p] += s;
-            }
+        for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+    float ys = 0.f;
+    const int start = blockIdx.x * nodesPerBlock, stop = min(n, start + nodesPerBlock);
+    for (int i0 = start + 2 * B * w; i0 < stop; i0 += 4 * 2 * B) {
+        float y[B], x[T][B];
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+            const int i = i0 + 2 * q + half;
+            const bool in = i < stop;
+            y[q] = in ? dY[(size_t)i * 32 + ch] : 0.f;
+            x[0][q] = in && ch < ROW ? (float)X1[(size_t)i * ROW + ch] : 0.f;
+            if constexpr (T == 2) x[1][q] = in ? (float)X2[(size_t)i * 32 + ch] : 0.f;
+        }
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+            ys += y[q];
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[q], x[t][q], acc[t], 0, 0, 0);
         }
     }
+    ys += __shfl_xor(ys, 32, 64);
 #pragma unroll
-    for (int p = 0; p < PER; p++) {
-        const int idx = threadIdx.x + p * 256;
-        if (idx < O * K) atomicAdd(&gW[idx], acc[p]);
-        else if (idx < NP && gb) atomicAdd(&gb[idx - O * K], acc[p]);
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            if (K >= 32 || ch < K) sh[w][(8 * (v / 4) + 4 * half + v % 4) * K + 32 * t + ch] = acc[t][v];
+    if (half == 0) sh[w][32 * K + ch] = ys;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 32 * K + 32; k += 256) {
+        const float g = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+        if (k < 32 * K) atomicAdd(&gW[k], g);
+        else if (gb) atomicAdd(&gb[k - 32 * K], g);
     }
 }
 
@@ -877,7 +953,7 @@ int gnnForward(Ctx* ctx) {
     e2.out = g->AB;
     hipLaunchKernelGGL((kGnnGemm<32, 32, GM_STORE, unsigned short>), dim3(gg), dim3(256), 0, s, n, g->Hs[gnn::L],
                        g->Hs[gnn::L], g->wb + gnn::wPab, e2);
-    hipLaunchKernelGGL(kGnnHead, dim3(gb), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge, g->AB, g->Hs[gnn::L], g->theta,
+    hipLaunchKernelGGL(kGnnHead, dim3((n * kHeadLanes + 255) / 256), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge, g->AB, g->Hs[gnn::L], g->theta,
                        g->da, g->ainv, g->cs, g->dsi, g->u, g->s);
     MPS_HIP(hipGetLastError());
     g->ready = true;
@@ -888,20 +964,18 @@ int gnnForward(Ctx* ctx) {
 int gnnBackward(Ctx* ctx) {
     Gnn* g = ctx->gnn;
     hipStream_t s = ctx->stream;
-    const int n = ctx->N, gb = g256(n), gg = (n + 63) / 64;
-    const int npb = 2048, wg = (n + npb - 1) / npb;
+    const int n = ctx->N, gg = (n + 63) / 64;
+    // nodes per block of the weight gradients: whole rounds of its four waves
+    const int npb = ((n + kWGradBlocks - 1) / kWGradBlocks + 63) / 64 * 64, wg = (n + npb - 1) / npb;
     float* gr = g->grad;
     MPS_HIP(hipMemsetAsync(gr, 0, sizeof(float) * gnn::NPARAM, s));
-    hipLaunchKernelGGL(kGnnBwdNode, dim3(gb), dim3(256), 0, s, n, g->gz, g->rv, g->ainv, g->s, g->u, g->Hs[gnn::L],
+    hipLaunchKernelGGL(kGnnBwdNode, dim3(min((n + 7) / 8, kBwdBlocks)), dim3(256), 0, s, n, g->gz, g->rv, g->ainv, g->s, g->u, g->Hs[gnn::L],
                        g->theta, g->dh, gr);
-    const int hb = (n + 15) / 16;
-    hipLaunchKernelGGL(kGnnBwdHeadI, dim3(hb), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge, g->AB, g->theta, g->da,
-                       g->gz, g->rv, g->dX, gr);
-    hipLaunchKernelGGL(kGnnBwdHeadJ, dim3(hb), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge, g->AB, g->theta, g->da,
-                       g->gz, g->rv, g->dX);
+    hipLaunchKernelGGL(kGnnBwdHead, dim3(min((n + 15) / 16, kBwdBlocks)), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge,
+                       g->AB, g->theta, g->da, g->gz, g->rv, g->dX, gr);
     // [Pa; Pb] gradients (Pa and Pb are contiguous: one [32][32] block) and
     // dh += dAB [Pa; Pb]
-    hipLaunchKernelGGL((kGnnWGrad<32, 32, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
+    hipLaunchKernelGGL((kGnnWGrad<32, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
                        reinterpret_cast<const Bf16In*>(g->Hs[gnn::L]), reinterpret_cast<const Bf16In*>(g->Hs[gnn::L]),
                        gr + gnn::oPa, nullptr);
     GemmEpi ea{};
@@ -911,7 +985,7 @@ int gnnBackward(Ctx* ctx) {
     for (int l = gnn::L - 1; l >= 0; l--) {
         const size_t tot = (size_t)n * H;
         hipLaunchKernelGGL(kGnnMask, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, g->dh, g->As[l], g->dX);
-        hipLaunchKernelGGL((kGnnWGrad<32, 64, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
+        hipLaunchKernelGGL((kGnnWGrad<64, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
                            reinterpret_cast<const Bf16In*>(g->Hs[l]), reinterpret_cast<const Bf16In*>(g->Ms[l]),
                            gr + gnn::oU(l), gr + gnn::oD(l));
         GemmEpi es{};
@@ -920,11 +994,11 @@ int gnnBackward(Ctx* ctx) {
         hipLaunchKernelGGL((kGnnGemm<32, 64, GM_SPLIT, float>), dim3(gg), dim3(256), 0, s, n, g->dX, g->dX,
                            g->wb + gnn::wUt(l), es);
         // dG into dX, E and c gradients
-        const int mb = (n + 63) / 64;
+        const int mb = min((n + 63) / 64, kBwdBlocks);
         hipLaunchKernelGGL(kGnnBwdMessage, dim3(mb), dim3(256), 0, s, n, g->gcol, g->gcnt, g->ge, g->gw, g->wsum,
                            g->Gs[l], g->theta + gnn::oE(l), g->theta + gnn::oC(l), g->dm, g->dX, gr + gnn::oE(l),
                            gr + gnn::oC(l));
-        hipLaunchKernelGGL((kGnnWGrad<32, 32, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
+        hipLaunchKernelGGL((kGnnWGrad<32, Bf16In>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
                            reinterpret_cast<const Bf16In*>(g->Hs[l]), reinterpret_cast<const Bf16In*>(g->Hs[l]),
                            gr + gnn::oB(l), nullptr);
         GemmEpi eb{};
@@ -935,7 +1009,7 @@ int gnnBackward(Ctx* ctx) {
     // encoder
     const size_t tot = (size_t)n * H;
     hipLaunchKernelGGL(kGnnMask, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, g->dh, g->pre0, g->dX);
-    hipLaunchKernelGGL((kGnnWGrad<32, 4, float>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
+    hipLaunchKernelGGL((kGnnWGrad<4, float>), dim3(wg), dim3(256), 0, s, n, npb, g->dX,
                        reinterpret_cast<const float*>(g->feat), reinterpret_cast<const float*>(g->feat),
                        gr + gnn::oW0, gr + gnn::ob0);
     MPS_HIP(hipGetLastError());

@@ -1929,7 +1929,8 @@ int ppeAssemble(Ctx* ctx) {
     // the CG solves' LDS windows (ppe_window scalar)
     // and those of a solve in one launch, whatever the scalar says
     const bool wins = !bicg && ctx->ppeWindow;
-    const bool wins16 = !bicg && oneLaunchRows(ctx);
+    // (the learned preconditioner's solve runs in pieces)
+    const bool wins16 = !bicg && oneLaunchRows(ctx) && !(mixed && ctx->P.learned_mode == 2 && ctx->gnn != nullptr);
     if (wins || wins16) {
         int rc = ensureWindows(ctx, wins);
         if (rc) return rc;
