@@ -504,6 +504,7 @@ int mps_create(mps_ctx** out, const mps_params* p, int n, int device) {
     MPS_HIP(hipMalloc(&ctx->is, sizeof(int) * NIS));
     ctx->redCap = std::max(kRedBlocks, gridFor(n, 256));
     MPS_HIP(hipMalloc(&ctx->red, sizeof(double) * (3 * ctx->redCap + 16)));
+    MPS_HIP(hipMalloc(&ctx->cgSums, sizeof(double) * 2 * kRedBlocks));
     MPS_HIP(hipMalloc(&ctx->asmRed, sizeof(double) * 2 * (size_t)std::max(kRedBlocks, gridFor(n, 16))));
     if (p->fluid_type == 1) {   // granular phase: carried per-step fields, bed-level grid
         for (int q = 0; q < kNNCarriedCount; q++) MPS_HIP(hipMalloc(&ctx->DaltNN[q], nd));
@@ -549,7 +550,7 @@ int mps_destroy(mps_ctx* ctx) {
                     ctx->aDiag32, ctx->cgR, ctx->cgP,
                     ctx->cgZ, ctx->cgQ, ctx->cgInvD, ctx->cgX, ctx->fR, ctx->fP, ctx->fZ, ctx->fQ, ctx->fX,
                     ctx->bcgR0, ctx->bcgY, ctx->bcgS, ctx->bcgT, ctx->patchList, ctx->fixList, ctx->V4, ctx->nbrMaskS, ctx->nbrS, ctx->nbrCntS,
-                    ctx->ds, ctx->is, ctx->red, ctx->asmRed, ctx->gridBar, ctx->gridPart, ctx->gridP2, ctx->red64, ctx->IaltPtype, ctx->bedKeys, ctx->bedIdx};
+                    ctx->ds, ctx->is, ctx->red, ctx->asmRed, ctx->cgSums, ctx->gridBar, ctx->gridPart, ctx->gridP2, ctx->red64, ctx->IaltPtype, ctx->bedKeys, ctx->bedIdx};
     for (void* b : bufs)
         if (b) hipFree(b);
     freeSlot(ctx->extraMesh[0]);

@@ -259,6 +259,7 @@ struct Ctx {
     double* gridP2 = nullptr;
     int oneLaunchFits[2] = {-1, -1};
     int asmBlocks = 0;           // blocks (partials) of the last assembly
+    double* cgSums = nullptr;    // block sums of a CG iteration's vector update (kRedBlocks pairs)
     double* asmRed = nullptr;    // block partials of the assembly's first residual (no other kernel writes them)
     unsigned long long* red64 = nullptr;   // result of reduceCounts (allocated on first use)
     // solver kind of the last PPE assembly (MPS_SOLVER_* / precision), -1 when

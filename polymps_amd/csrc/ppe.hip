@@ -1116,50 +1116,118 @@ __global__ void kCgAlpha(KArgs a, int nb) {
         a.ds[S_ALPHA] = a.ds[S_ABSNEW] / s0;
     }
 }
-// x += alpha p; r -= alpha q; z = invd r; partials |r|^2, r.z
-__global__ void kCgUpdate(KArgs a, CgPtrs c) {
+// The vectors of a Jacobi-PCG in FP64 (solveFp64) or FP32 (solveMixed; the
+// correction fd is FP64).
+template <class T>
+struct CgVecs {
+    double* x;
+    T *p, *r, *q, *z;
+    const T* invd;
+};
+template <class T>
+__device__ __forceinline__ CgVecs<T> cgVecs(const CgPtrs& c) {
+    if constexpr (sizeof(T) == 8) return {c.x, c.p, c.r, c.q, c.z, c.invd};
+    else return {c.fd, c.fp, c.fr, c.fq, c.fz, c.invd32};
+}
+
+// The two vector kernels of an iteration add the block sums they need
+// themselves, every block all of them, instead of waiting for a one-block
+// kernel each: 4.4 us and a launch gap twice per iteration (216,000 rows: 66
+// us of kernels per iteration, now 62, in three launches instead of five).  They
+// run on at most kVecBlocks blocks, so the
+// second's sums are few; the SpMV leaves one pair per 256 rows, which the
+// first adds up to kSumBlocks of them (every block reads them all: at 2,048
+// that takes what kCgAlpha takes).
+constexpr int kVecBlocks = kRedBlocks;
+constexpr int kSumBlocks = 1536;
+
+// x += alpha p; r -= alpha q; z = invd r; partials |r|^2, r.z in sums.  SUM:
+// alpha from the SpMV's partials, else from kCgAlpha.
+template <class T, bool SUM>
+__global__ __launch_bounds__(256) void kCgUpdate(KArgs a, CgPtrs c, int nb, double* sums) {
     if (a.is[I_CG_DONE]) return;
-    const int i = slotId();
-    const double alpha = a.ds[S_ALPHA];
+    const CgVecs<T> v = cgVecs<T>(c);
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    const double absNew = a.ds[S_ABSNEW];   // written by kCgP
+    double al;
+    if constexpr (SUM) {
+        double pap, unused;
+        finishPartials(a.red, nb, pap, unused);
+        al = absNew / pap;
+        if (first) {
+            a.ds[S_PAP] = pap;
+            a.ds[S_ALPHA] = al;
+        }
+    } else {
+        al = a.ds[S_ALPHA];
+    }
+    if (first) a.ds[S_ABSOLD] = absNew;
+    const T alpha = (T)al;
     double s0 = 0, s1 = 0;
-    if (i < a.N) {
-        c.x[i] += alpha * c.p[i];
-        const double r = c.r[i] - alpha * c.q[i];
-        c.r[i] = r;
-        const double z = c.invd[i] * r;
-        c.z[i] = z;
-        s0 = r * r;
-        s1 = r * z;
+    const int step = gridDim.x * blockDim.x;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.N; i += 2 * step) {   // two rows in flight
+        const int k[2] = {i, i + step < a.N ? i + step : i};
+        double x[2];
+        T p[2], r[2], q[2], iv[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            x[e] = v.x[k[e]];
+            p[e] = v.p[k[e]];
+            r[e] = v.r[k[e]];
+            q[e] = v.q[k[e]];
+            iv[e] = v.invd[k[e]];
+        }
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            if (e == 1 && i + step >= a.N) break;
+            v.x[k[e]] = x[e] + (double)alpha * (double)p[e];
+            const T rn = r[e] - alpha * q[e];
+            v.r[k[e]] = rn;
+            const T z = iv[e] * rn;
+            v.z[k[e]] = z;
+            s0 += (double)rn * (double)rn;
+            s1 += (double)rn * (double)z;
+        }
     }
-    writePartials(a, s0, s1);
+    KArgs o = a;
+    o.red = sums;
+    writePartials(o, s0, s1);
 }
-__global__ void kCgBeta(KArgs a, int nb, int maxIt) {
-    if (a.is[I_CG_DONE]) return;
+// The end of an iteration from kCgUpdate's sums, and p = z + beta p.  The
+// flag is read once per block: the first block may raise it meanwhile (a
+// block that sees it leaves p as it is, which nothing reads any more).
+template <class T>
+__global__ __launch_bounds__(256) void kCgP(KArgs a, CgPtrs c, int nb, const double* sums, int maxIt) {
+    __shared__ int done;
+    if (threadIdx.x == 0) done = a.is[I_CG_DONE];
+    __syncthreads();
+    if (done) return;
     double rn2, rz;
-    finishPartials(a.red, nb, rn2, rz);
-    if (threadIdx.x != 0) return;
-    a.ds[S_RN2] = rn2;
-    if (rn2 < a.ds[S_THR]) {
-        a.is[I_CG_DONE] = 1;
-        return;
+    finishPartials(sums, nb, rn2, rz);
+    const int end = rn2 < a.ds[S_THR] ? 1 : !isfinite(rn2) ? 5 : 0;
+    const double beta = rz / a.ds[S_ABSOLD];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.ds[S_RN2] = rn2;
+        if (end) {
+            a.is[I_CG_DONE] = end;
+        } else {
+            a.ds[S_ABSNEW] = rz;
+            a.ds[S_BETA] = beta;
+            const int it = a.is[I_CG_ITER] + 1;
+            a.is[I_CG_ITER] = it;
+            if (it >= maxIt) a.is[I_CG_DONE] = 3;
+        }
     }
-    if (!isfinite(rn2)) {
-        a.is[I_CG_DONE] = 5;
-        return;
+    if (end) return;
+    const CgVecs<T> v = cgVecs<T>(c);
+    const T bt = (T)beta;
+    const int step = gridDim.x * blockDim.x;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.N; i += 2 * step) {
+        const int j = i + step < a.N ? i + step : i;
+        const T z0 = v.z[i], p0 = v.p[i], z1 = v.z[j], p1 = v.p[j];
+        v.p[i] = z0 + bt * p0;
+        if (j != i) v.p[j] = z1 + bt * p1;
     }
-    const double absOld = a.ds[S_ABSNEW];
-    a.ds[S_ABSOLD] = absOld;
-    a.ds[S_ABSNEW] = rz;
-    a.ds[S_BETA] = rz / absOld;
-    const int it = a.is[I_CG_ITER] + 1;
-    a.is[I_CG_ITER] = it;
-    if (it >= maxIt) a.is[I_CG_DONE] = 3;
-}
-// p = z + beta p
-__global__ void kCgP(KArgs a, CgPtrs c) {
-    if (a.is[I_CG_DONE]) return;
-    const int i = slotId();
-    if (i < a.N) c.p[i] = c.z[i] + a.ds[S_BETA] * c.p[i];
 }
 
 // true residual r = b - M x in FP64 (kept in c.r); partials |r|^2, |b|^2
@@ -1237,23 +1305,8 @@ __global__ __launch_bounds__(256) void kMxSpmv(KArgs a, CgPtrs c) {
     }
     writePartials(a, s0, 0.0);
 }
-__global__ void kMxUpdate(KArgs a, CgPtrs c) {
-    if (a.is[I_CG_DONE]) return;
-    const int i = slotId();
-    const float alpha = (float)a.ds[S_ALPHA];
-    double s0 = 0, s1 = 0;
-    if (i < a.N) {
-        c.fd[i] += (double)alpha * (double)c.fp[i];
-        const float r = c.fr[i] - alpha * c.fq[i];
-        c.fr[i] = r;
-        const float z = c.invd32[i] * r;
-        c.fz[i] = z;
-        s0 = (double)r * (double)r;
-        s1 = (double)r * (double)z;
-    }
-    writePartials(a, s0, s1);
-}
-__global__ void kMxP(KArgs a, CgPtrs c) {
+// p = z + beta p of the flexible CG (learned operator)
+__global__ void kFcgP(KArgs a, CgPtrs c) {
     if (a.is[I_CG_DONE]) return;
     const int i = slotId();
     if (i < a.N) c.fp[i] = c.fz[i] + (float)a.ds[S_BETA] * c.fp[i];
@@ -1613,7 +1666,7 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
         publishSums<2>(part1, own ? r * r : 0.0, own ? r * z : 0.0);
         if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
         sumPublished<2>(part1, s2);
-        rn2 = s2[0];   // kCgBeta
+        rn2 = s2[0];   // kCgP
         if (rn2 < thr) done = 1;
         else if (!isfinite(rn2)) done = 5;
         else {
@@ -2376,6 +2429,20 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
     return MPS_OK;
 }
 
+// what follows an iteration's SpMV (nb blocks' p.q in a.red)
+template <class T>
+static void launchCgVectors(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int maxIt) {
+    hipStream_t s = ctx->stream;
+    const int vb = std::min(nb, kVecBlocks);
+    if (nb <= kSumBlocks) {
+        hipLaunchKernelGGL((kCgUpdate<T, true>), dim3(vb), dim3(kB), 0, s, a, c, nb, ctx->cgSums);
+    } else {
+        hipLaunchKernelGGL(kCgAlpha, dim3(1), dim3(1024), 0, s, a, nb);
+        hipLaunchKernelGGL((kCgUpdate<T, false>), dim3(vb), dim3(kB), 0, s, a, c, nb, ctx->cgSums);
+    }
+    hipLaunchKernelGGL(kCgP<T>, dim3(vb), dim3(kB), 0, s, a, c, vb, ctx->cgSums, maxIt);
+}
+
 // Eigen-semantics Jacobi-PCG in FP64 (solveConjugateGradient, src/MpsPressure.cpp:424-445)
 static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batch, bool* oneLaunch) {
     hipStream_t s = ctx->stream;
@@ -2413,10 +2480,7 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
     for (int launched = 0, b = firstBatch(ctx->lastCgIters, batch); !done; launched += b, b = batch) {
         for (int q = 0; q < b; q++) {
             timedSpmv(ctx, kCgSpmv, a, c, nb, q);
-            hipLaunchKernelGGL(kCgAlpha, dim3(1), dim3(1024), 0, s, a, nb);
-            hipLaunchKernelGGL(kCgUpdate, dim3(nb), dim3(kB), 0, s, a, c);
-            hipLaunchKernelGGL(kCgBeta, dim3(1), dim3(1024), 0, s, a, nb, maxIt);
-            hipLaunchKernelGGL(kCgP, dim3(nb), dim3(kB), 0, s, a, c);
+            launchCgVectors<double>(ctx, a, c, nb, maxIt);
         }
         int rc = readStatus(ctx, &times, b);
         if (rc) return rc;
@@ -2518,17 +2582,16 @@ static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int bat
         for (int launched = 0, bq = bq0; !done; launched += bq, bq = batch) {
             for (int q = 0; q < bq; q++) {
                 timedSpmv(ctx, kMxSpmv, a, c, nb, q);
-                hipLaunchKernelGGL(kCgAlpha, dim3(1), dim3(1024), 0, s, a, nb);
                 if (useM) {
+                    hipLaunchKernelGGL(kCgAlpha, dim3(1), dim3(1024), 0, s, a, nb);
                     hipLaunchKernelGGL(kFcgUpdate, dim3(nb), dim3(kB), 0, s, a, c);
                     gnnApply32(ctx, c.fr, c.fz);
                     hipLaunchKernelGGL(kFcgDots, dim3(nb), dim3(kB), 0, s, a, c);
                     hipLaunchKernelGGL(kFcgBeta, dim3(1), dim3(1024), 0, s, a, nb, std::min(maxIt, kLearnedPassMax));
+                    hipLaunchKernelGGL(kFcgP, dim3(nb), dim3(kB), 0, s, a, c);
                 } else {
-                    hipLaunchKernelGGL(kMxUpdate, dim3(nb), dim3(kB), 0, s, a, c);
-                    hipLaunchKernelGGL(kCgBeta, dim3(1), dim3(1024), 0, s, a, nb, maxIt);
+                    launchCgVectors<float>(ctx, a, c, nb, maxIt);
                 }
-                hipLaunchKernelGGL(kMxP, dim3(nb), dim3(kB), 0, s, a, c);
             }
             if ((rc = readStatus(ctx, &times, bq))) return rc;
             done = ctx->hostInts[I_CG_DONE];

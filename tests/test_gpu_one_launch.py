@@ -96,3 +96,11 @@ def test_wide_windows(built, shape, precision):
     w = _block(*shape, thin=300)
     g = _check(w, precision)
     assert g.scalar("ppe_window_blocks") < (len(w.types) + 255) // 256
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(64, 64, 64), (96, 64, 64), (97, 64, 64)])
+def test_pieces(built, shape, precision):
+    """Larger systems: the vector kernels take one row per thread up to 262,144
+    rows and several above, and add the SpMV's sums themselves up to 393,216."""
+    _check(_block(*shape), precision)
