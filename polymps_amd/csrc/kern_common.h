@@ -285,13 +285,6 @@ __device__ __forceinline__ void listNbrsQ(const KArgs& a, const int* nbr, const 
     listNbrsX(a, nbr, cnt, i, [](int) { return NoExtra{}; }, [&](int j, const double4& q, NoExtra) { g(j, q); });
 }
 
-// The large-radius list with a second packed per-slot array: g(j, q, v)
-// receives P4[j] and V[j], both gathered in the batch.
-template <class G>
-__device__ __forceinline__ void listNbrsQV(const KArgs& a, const double4* __restrict__ V, int i, G&& g) {
-    listNbrsX(a, a.nbr, a.nbrCnt, i, [&](int j) { return V[j]; }, g);
-}
-
 // Particle type from the w component of P4: its low 10 bits, sign-extended
 // (types in [-512, 511]); bits 10 and up hold the flags of update_bc.
 __device__ __forceinline__ int p4Type(double w) { return ((((int)w) & 1023) ^ 512) - 512; }
@@ -312,22 +305,6 @@ template <bool LIST, class F>
 __device__ __forceinline__ void forNbrsPosS(const KArgs& a, int i, double x, double y, double z, F&& f) {
     if (LIST) listNbrsQ(a, a.nbrS, a.nbrCntS, i, [&](int j, const double4& q) { f(j, q.x, q.y, q.z); });
     else walkCellsPos(a, i, x, y, z, f);
-}
-
-// Small-radius neighbours with one more per-slot FP64 value S[j]:
-// f(j, xj, yj, zj, sOf), sOf() returning S[j].  With the list S[j] is
-// gathered in the batch (every entry is a valid slot); a walk reads it only
-// when sOf is called.
-template <bool LIST, class F>
-__device__ __forceinline__ void forNbrsPosSX(const KArgs& a, int i, double x, double y, double z,
-                                             const double* __restrict__ S, F&& f) {
-    if (LIST) {
-        listNbrsX(a, a.nbrS, a.nbrCntS, i, [&](int j) { return S[j]; },
-                  [&](int j, const double4& q, double s) { f(j, q.x, q.y, q.z, [s]() { return s; }); });
-    } else {
-        walkCellsPos(a, i, x, y, z,
-                     [&](int j, double xj, double yj, double zj) { f(j, xj, yj, zj, [S, j]() { return S[j]; }); });
-    }
 }
 
 // The same with the neighbour's particle type, f(j, xj, yj, zj, tj).
