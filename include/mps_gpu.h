@@ -126,7 +126,9 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * used from the next assembly; read-only "ppe_window_blocks": blocks of the
  * last assembly served from a window, "window_escapes": window index
  * escapes of the last assembly, the rows' absolute indices next to their
- * one-byte steps) "ppe_warm_start" (initial guess of each
+ * one-byte steps) "grid_spin" (set only, [1, 2^20], default 65536: polls
+ * before a grid barrier of a solve in one launch gives up and the solve runs
+ * in pieces) "ppe_warm_start" (initial guess of each
  * pressure solve: 0 previous solution, 1 / 2 / 3 linear / quadratic / cubic
  * extrapolation of the last solutions) "mesh_bvh" (closest-point search: -1 BVH for
  * meshes above 64 faces, 0 brute force, 1 BVH; both give the same result). */

@@ -824,6 +824,13 @@ int mps_set_scalar(mps_ctx* ctx, const char* name, double value) {
         ctx->timeCurrent = value;
     } else if (s == "solver_failures") {
         ctx->solverFailures = (long)value;
+    } else if (s == "grid_spin") {
+        // polls before a grid barrier of a solve in one launch gives up and the solve runs in pieces
+        if (!(value >= 1.0 && value <= (double)(1 << 20))) {
+            ctx->err = "grid_spin must be in [1, 2^20]";
+            return MPS_E_ARG;
+        }
+        ctx->gridSpin = (int)value;
     } else if (s == "profile") {
         ctx->profile = value != 0.0;
         ctx->spmvMsTotal = 0.0;

@@ -1347,13 +1347,12 @@ __global__ void kMxApply(KArgs a, CgPtrs c) {
 // The grid is no larger than what the device holds (asked of the runtime), so
 // on a device of its own every block is running when it waits.  Where other
 // work keeps blocks out (another context's solve in one launch, at worst,
-// waiting for the same CUs), the wait ends after kSpinMax polls, every block
+// waiting for the same CUs), the wait ends after Ctx::gridSpin polls, every block
 // leaves, and the solve is repeated in pieces.  (A cooperative launch would
 // settle this in the runtime, at the price of draining the stream before and
 // after it: 40-60 us per solve.)
 constexpr int kGridBars = 9;            // counters: eight groups of blocks, the root (one cache line each)
 constexpr int kBarStride = 32;          // unsigned per cache line
-constexpr int kSpinMax = 1 << 16;       // polls (of about 0.7 us) before a barrier gives up
 
 template <class T>
 __device__ __forceinline__ T loadAgent(const T* p) {
@@ -1369,7 +1368,7 @@ __device__ __forceinline__ void storeAgent(T* p, T v) {
 // group counts at the root, which all poll: 256 blocks on one counter take
 // 3.7 us.  The threads' agent-scope stores have completed when it is counted.
 // false: a block did not arrive in time, every block leaves.
-__device__ __forceinline__ bool gridBarrier(unsigned* bar, unsigned epoch, int* lateFlag) {
+__device__ __forceinline__ bool gridBarrier(unsigned* bar, unsigned epoch, int spinMax, int* lateFlag) {
     __shared__ int late;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // the wave's own stores
     __syncthreads();
@@ -1380,8 +1379,8 @@ __device__ __forceinline__ bool gridBarrier(unsigned* bar, unsigned epoch, int* 
             epoch * size)
             __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         int spin = 0;
-        while (loadAgent(root) < epoch * groups && ++spin < kSpinMax) __builtin_amdgcn_s_sleep(1);
-        late = spin >= kSpinMax ? 1 : 0;
+        while (loadAgent(root) < epoch * groups && ++spin < spinMax) __builtin_amdgcn_s_sleep(1);
+        late = spin >= spinMax ? 1 : 0;
         if (late) atomicOr(lateFlag, 1);
     }
     __syncthreads();
@@ -1582,6 +1581,7 @@ struct OneLaunch {
     const double* asmRed;   // the assembly's sums (null: the first residual is computed here)
     int asmBlocks;
     int full;            // windows: the whole vector (periodic domains)
+    int spin;            // polls before a barrier gives up
     double tol, tolIn;
     int maxIt, maxOuter;
 };
@@ -1621,11 +1621,11 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
         sumLeft<2>(o.asmRed, o.asmBlocks, s2);
     } else {
         if (own) storeAgent(c.x + i, x);
-        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE);
         if (ok) {
             r = residual();
             publishSums<2>(part0, own ? b * b : 0.0, own ? r * r : 0.0);
-            ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+            ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE);
             sumPublished<2>(part0, s2);
         }
     }
@@ -1643,7 +1643,7 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
     if (ok && !done) {
         if (own) storeAgent(c.z + i, z);
         publishSums<2>(part1, own ? r * p : 0.0, 0.0);
-        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE);
         sumPublished<2>(part1, s2);
         absNew = s2[0];
     }
@@ -1656,7 +1656,7 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
         const double q = rowPublished<double, L>(c, c.val, w, win, cap, n, KE, i, diag * p, pOf);
         if (own) storeAgent(pNew + i, p);
         publishSums<1>(part0, own ? p * q : 0.0, 0.0);
-        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
         sumPublished<1>(part0, s1);
         const double alpha = absNew / s1[0];
         x += alpha * p;
@@ -1664,7 +1664,7 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
         z = invd * r;
         if (own) storeAgent(c.z + i, z);
         publishSums<2>(part1, own ? r * r : 0.0, own ? r * z : 0.0);
-        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
         sumPublished<2>(part1, s2);
         rn2 = s2[0];   // kCgP
         if (rn2 < thr) done = 1;
@@ -1682,12 +1682,12 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
     }
     if (ok) {   // the true residual of the result
         if (own) storeAgent(c.x + i, x);
-        ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+        ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE);
         if (ok) {
             const double tr = residual();
             if (own) c.r[i] = tr;
             publishSums<2>(part0, own ? tr * tr : 0.0, own ? b * b : 0.0);
-            ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE);
+            ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE);
             sumPublished<2>(part0, s2);
         }
     }
@@ -1738,11 +1738,11 @@ __global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaun
             sumLeft<2>(o.asmRed, o.asmBlocks, s2);
         } else {
             if (own) storeAgent(c.x + i, x);
-            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
             auto xOf = [&](int j) { return loadAgent(c.x + j); };
             r64 = b - rowPublished<double, L>(c, c.val, w, win64, cap, n, KE, i, diag * x, xOf);
             publishSums<2>(part0, own ? r64 * r64 : 0.0, own ? b * b : 0.0);
-            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
             sumPublished<2>(part0, s2);
         }
         if (own) c.r[i] = r64;
@@ -1760,7 +1760,7 @@ __global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaun
         double d = 0.0;
         if (own) storeAgent(c.fz + i, z);
         publishSums<2>(part1, own ? (double)r * (double)z : 0.0, own ? (double)r * (double)r : 0.0);
-        if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+        if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
         sumPublished<2>(part1, s2);
         double absNew = s2[0];
         const double in2 = s2[1];
@@ -1780,7 +1780,7 @@ __global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaun
                                                           (double)(diag32 * p), pOf);
             if (own) storeAgent(pNew + i, p);
             publishSums<1>(part0, own ? (double)p * (double)q : 0.0, 0.0);
-            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
             sumPublished<1>(part0, s1);
             const float alpha = (float)(absNew / s1[0]);
             d += (double)alpha * (double)p;
@@ -1788,7 +1788,7 @@ __global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaun
             z = invd * r;
             if (own) storeAgent(c.fz + i, z);
             publishSums<2>(part1, own ? (double)r * (double)r : 0.0, own ? (double)r * (double)z : 0.0);
-            if (!(ok = gridBarrier(o.bar, ++epoch, a.is + I_GRID_LATE))) break;
+            if (!(ok = gridBarrier(o.bar, ++epoch, o.spin, a.is + I_GRID_LATE))) break;
             sumPublished<2>(part1, s2);
             if (s2[0] < thr) done = 1;
             else if (!isfinite(s2[0])) done = 5;
@@ -2412,6 +2412,7 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
     o.asmRed = fresh ? ctx->asmRed : nullptr;
     o.asmBlocks = ctx->asmBlocks;
     o.full = periodicCtx(ctx) ? 1 : 0;
+    o.spin = ctx->gridSpin;
     o.tol = tol;
     o.tolIn = tolIn;
     o.maxIt = maxIt;

@@ -104,3 +104,26 @@ def test_pieces(built, shape, precision):
     """Larger systems: the vector kernels take one row per thread up to 262,144
     rows and several above, and add the SpMV's sums themselves up to 393,216."""
     _check(_block(*shape), precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(24, 6, 12), (64, 32, 32), (64, 41, 25)])
+def test_blocks_that_do_not_meet(built, shape, precision):
+    """A wait of one poll: blocks give up at their first barriers, all leave,
+    and the solve runs in pieces with the same answer; the counters are at
+    zero for the next solve, which meets again."""
+    w = _block(*shape)
+    w.params.precision_mode = precision
+    w.params.ppe_transpose = 0
+    print(f"one poll {w.n} precision {precision}", flush=True)
+    g = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh, device=0)
+    g.call("init")
+    guess = 0.9 * g.get("press") + 1e-3 * configs.splitmix64_uniform(5, w.n)
+    x0, it0, _ = _solve(g, guess, False)
+    g.set_scalar("grid_spin", 1)
+    x1, it1, res1 = _solve(g, guess, False)
+    assert abs(it1 - it0) <= 1 and res1 <= 1.01e-8
+    assert _residual(g.ppe_matrix(), g.get("ppe_b"), x1) <= 1.01e-8
+    g.set_scalar("grid_spin", 65536)
+    x2, it2, _ = _solve(g, guess, False)
+    assert it2 == it0 and np.array_equal(x0, x2)
