@@ -844,48 +844,60 @@ static std::vector<float> initParams(unsigned long long seed) {
     return th;
 }
 
-int gnnEnsure(Ctx* ctx) {
-    if (ctx->gnn) return MPS_OK;
+// The operator's buffers and initial parameters: all or none, so that a call
+// after a failed allocation starts again.
+static int gnnCreate(Ctx* ctx) {
     Gnn* g = new Gnn();
     ctx->gnn = g;
     const size_t n = ctx->N;
     g->N = ctx->N;
-    MPS_HIP(hipMalloc(&g->theta, sizeof(float) * gnn::NPARAM));
-    MPS_HIP(hipMalloc(&g->grad, sizeof(float) * gnn::NPARAM));
-    MPS_HIP(hipMalloc(&g->adamM, sizeof(float) * gnn::NPARAM));
-    MPS_HIP(hipMalloc(&g->adamV, sizeof(float) * gnn::NPARAM));
-    MPS_HIP(hipMalloc(&g->wb, sizeof(unsigned short) * gnn::NWB));
-    MPS_HIP(hipMalloc(&g->gcol, sizeof(int) * KE * n));
-    MPS_HIP(hipMalloc(&g->gcnt, sizeof(int) * n));
-    MPS_HIP(hipMalloc(&g->ge, sizeof(float4) * KE * n));
-    MPS_HIP(hipMalloc(&g->gw, sizeof(float) * KE * n));
-    MPS_HIP(hipMalloc(&g->wsum, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->feat, sizeof(float4) * n));
-    MPS_HIP(hipMalloc(&g->da, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->ainv, sizeof(float) * n));
-    for (int l = 0; l <= gnn::L; l++) MPS_HIP(hipMalloc(&g->Hs[l], sizeof(unsigned short) * H * n));
+    int rc = MPS_OK;
+    auto make = [&](auto** p, size_t count) {
+        if (!rc) rc = ensureBuffer(ctx, p, count);
+    };
+    make(&g->theta, gnn::NPARAM);
+    make(&g->grad, gnn::NPARAM);
+    make(&g->adamM, gnn::NPARAM);
+    make(&g->adamV, gnn::NPARAM);
+    make(&g->wb, gnn::NWB);
+    make(&g->gcol, KE * n);
+    make(&g->gcnt, n);
+    make(&g->ge, KE * n);
+    make(&g->gw, KE * n);
+    make(&g->wsum, n);
+    make(&g->feat, n);
+    make(&g->da, n);
+    make(&g->ainv, n);
+    for (int l = 0; l <= gnn::L; l++) make(&g->Hs[l], H * n);
     for (int l = 0; l < gnn::L; l++) {
-        MPS_HIP(hipMalloc(&g->Gs[l], sizeof(unsigned short) * H * n));
-        MPS_HIP(hipMalloc(&g->Ms[l], sizeof(unsigned short) * H * n));
-        MPS_HIP(hipMalloc(&g->As[l], sizeof(unsigned short) * H * n));
+        make(&g->Gs[l], H * n);
+        make(&g->Ms[l], H * n);
+        make(&g->As[l], H * n);
     }
-    MPS_HIP(hipMalloc(&g->pre0, sizeof(unsigned short) * H * n));
-    MPS_HIP(hipMalloc(&g->AB, sizeof(unsigned short) * 32 * n));
-    MPS_HIP(hipMalloc(&g->u, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->s, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->cs, sizeof(float) * KE * n));
-    MPS_HIP(hipMalloc(&g->dsi, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->gz, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->rv, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->dh, sizeof(float) * H * n));
-    MPS_HIP(hipMalloc(&g->dX, sizeof(float) * H * n));
-    MPS_HIP(hipMalloc(&g->dm, sizeof(float) * H * n));
-    MPS_HIP(hipMalloc(&g->zt, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&g->dv1, sizeof(double) * n));
-    MPS_HIP(hipMalloc(&g->dv2, sizeof(double) * n));
-    MPS_HIP(hipMalloc(&g->dv3, sizeof(double) * n));
-    MPS_HIP(hipMalloc(&g->acc, sizeof(double) * 4));
-    return gnnSetParams(ctx, nullptr, 0);
+    make(&g->pre0, H * n);
+    make(&g->AB, 32 * n);
+    make(&g->u, n);
+    make(&g->s, n);
+    make(&g->cs, KE * n);
+    make(&g->dsi, n);
+    make(&g->gz, n);
+    make(&g->rv, n);
+    make(&g->dh, H * n);
+    make(&g->dX, H * n);
+    make(&g->dm, H * n);
+    make(&g->zt, n);
+    make(&g->dv1, n);
+    make(&g->dv2, n);
+    make(&g->dv3, n);
+    make(&g->acc, 4);
+    return rc ? rc : gnnSetParams(ctx, nullptr, 0);
+}
+
+int gnnEnsure(Ctx* ctx) {
+    if (ctx->gnn) return MPS_OK;
+    const int rc = gnnCreate(ctx);
+    if (rc) gnnFree(ctx);
+    return rc;
 }
 
 // Install parameters (nullptr: the seeded initial values) and reset Adam.

@@ -302,6 +302,22 @@ struct Ctx {
         }                                                                               \
     } while (0)
 
+// A buffer made at first use.  Each pointer asks for itself: after a call
+// whose allocation failed, the next one makes what is missing.
+template <class T>
+int ensureBuffer(Ctx* ctx, T** p, size_t count) {
+    if (*p) return MPS_OK;
+    T* made = nullptr;
+    const hipError_t e = hipMalloc(&made, sizeof(T) * count);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not by the next call
+        ctx->err = "hipMalloc of " + std::to_string(sizeof(T) * count) + " bytes: " + hipGetErrorString(e);
+        return MPS_E_HIP;
+    }
+    *p = made;
+    return MPS_OK;
+}
+
 inline int gridFor(int n, int block) { return (n + block - 1) / block; }
 
 // launchers (defined in the .hip translation units)

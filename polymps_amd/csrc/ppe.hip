@@ -1917,17 +1917,12 @@ static CgPtrs cgPtrs(Ctx* ctx) {
 }
 
 static int ensureMixed(Ctx* ctx) {
-    if (ctx->aVal32) return MPS_OK;
     const size_t n = ctx->N;
-    MPS_HIP(hipMalloc(&ctx->aVal32, sizeof(float) * (size_t)ellWidth(ctx->K) * ellRows(n)));
-    MPS_HIP(hipMalloc(&ctx->aDiagInv32, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->aDiag32, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->fR, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->fP, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->fZ, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->fQ, sizeof(float) * n));
-    MPS_HIP(hipMalloc(&ctx->fX, sizeof(double) * n));
-    return MPS_OK;
+    int rc;
+    if ((rc = ensureBuffer(ctx, &ctx->aVal32, (size_t)ellWidth(ctx->K) * ellRows(n)))) return rc;
+    for (float** v : {&ctx->aDiagInv32, &ctx->aDiag32, &ctx->fR, &ctx->fP, &ctx->fZ, &ctx->fQ})
+        if ((rc = ensureBuffer(ctx, v, n))) return rc;
+    return ensureBuffer(ctx, &ctx->fX, n);
 }
 
 // a periodic domain's window is the whole vector
@@ -1937,14 +1932,12 @@ static bool periodicCtx(const Ctx* ctx) { return ctx->P.domain_type_bc == 1; }
 static bool oneLaunchRows(const Ctx* ctx) { return ctx->N <= (periodicCtx(ctx) ? kFullMax : kOneLaunchMax); }
 
 static int ensureWindows(Ctx* ctx, bool bytes) {
-    if (!ctx->aWin) MPS_HIP(hipMalloc(&ctx->aWin, sizeof(int) * (size_t)kWinStride * gridFor(ctx->N, kB)));
-    if (bytes && !ctx->aLc8) {
-        MPS_HIP(hipMalloc(&ctx->aLc8, (size_t)ellWidth(ctx->K) * ellRows(ctx->N)));
-        MPS_HIP(hipMalloc(&ctx->aLcEsc, sizeof(unsigned short) * (size_t)kLcEsc * ellRows(ctx->N)));
-    }
-    if (oneLaunchRows(ctx) && !ctx->aLc16)
-        MPS_HIP(hipMalloc(&ctx->aLc16, sizeof(unsigned short) * (size_t)ellWidth(ctx->K) * ellRows(ctx->N)));
-    return MPS_OK;
+    const size_t entries = (size_t)ellWidth(ctx->K) * ellRows(ctx->N);
+    int rc = ensureBuffer(ctx, &ctx->aWin, (size_t)kWinStride * gridFor(ctx->N, kB));
+    if (!rc && bytes) rc = ensureBuffer(ctx, &ctx->aLc8, entries);
+    if (!rc && bytes) rc = ensureBuffer(ctx, &ctx->aLcEsc, (size_t)kLcEsc * ellRows(ctx->N));
+    if (!rc && oneLaunchRows(ctx)) rc = ensureBuffer(ctx, &ctx->aLc16, entries);
+    return rc;
 }
 
 // The solver kind an assembly prepares: FP64 CG, mixed CG (FP32 values as
@@ -2307,12 +2300,9 @@ __global__ void kBcgCheck(KArgs a, int nb, int maxIt) {
 }
 
 static int ensureBicgstab(Ctx* ctx) {
-    if (ctx->bcgR0) return MPS_OK;
-    const size_t bytes = sizeof(double) * (size_t)ctx->N;
-    MPS_HIP(hipMalloc(&ctx->bcgR0, bytes));
-    MPS_HIP(hipMalloc(&ctx->bcgY, bytes));
-    MPS_HIP(hipMalloc(&ctx->bcgS, bytes));
-    MPS_HIP(hipMalloc(&ctx->bcgT, bytes));
+    int rc;
+    for (double** v : {&ctx->bcgR0, &ctx->bcgY, &ctx->bcgS, &ctx->bcgT})
+        if ((rc = ensureBuffer(ctx, v, (size_t)ctx->N))) return rc;
     return MPS_OK;
 }
 
@@ -2387,12 +2377,17 @@ static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
         ctx->oneLaunchFits[mixed] = nb <= perCu * cus ? 1 : 0;
     }
     if (!ctx->oneLaunchFits[mixed]) return MPS_OK;
-    if (!ctx->gridBar) {
-        const size_t bytes = sizeof(unsigned) * (kGridBars + 1) * kBarStride;
-        MPS_HIP(hipMalloc(&ctx->gridBar, bytes));
-        MPS_HIP(hipMemsetAsync(ctx->gridBar, 0, bytes, ctx->stream));
-        MPS_HIP(hipMalloc(&ctx->gridPart, sizeof(double) * 4 * (size_t)nb));
-        MPS_HIP(hipMalloc(&ctx->gridP2, sizeof(double) * (size_t)ctx->N));
+    int rc;
+    if ((rc = ensureBuffer(ctx, &ctx->gridPart, 4 * (size_t)nb))) return rc;
+    if ((rc = ensureBuffer(ctx, &ctx->gridP2, (size_t)ctx->N))) return rc;
+    if (!ctx->gridBar) {   // the counters: kept only once they are zero
+        const size_t count = (kGridBars + 1) * kBarStride;
+        unsigned* bar = nullptr;
+        if ((rc = ensureBuffer(ctx, &bar, count))) return rc;
+        const hipError_t e = hipMemsetAsync(bar, 0, sizeof(unsigned) * count, ctx->stream);
+        if (e != hipSuccess) (void)hipFree(bar);
+        MPS_HIP(e);
+        ctx->gridBar = bar;
     }
     *fits = true;
     return MPS_OK;

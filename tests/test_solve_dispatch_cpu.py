@@ -1,0 +1,119 @@
+"""Host side of the pressure solve without a GPU: what it allocates and which
+kernels it launches, on a runtime that only notes both (host_runtime.cpp).
+
+Each case runs in a process of its own, which loads that runtime in the place
+of the real one before the library.
+"""
+import ctypes
+import re
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+# ------------------------------------------------------- in the child process
+class Runtime:
+    def __init__(self, path):
+        self.dll = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.dll.test_launched.restype = ctypes.c_char_p
+        self.dll.test_allocations.restype = ctypes.c_long
+        self.dll.test_live.restype = ctypes.c_long
+        self.dll.test_status_bytes.argtypes = [ctypes.c_size_t]
+        self.dll.test_fail_allocation.argtypes = [ctypes.c_long]
+        text = (ROOT / "polymps_amd" / "csrc" / "mps_internal.h").read_text()
+        names = re.sub(r"//.*", "", re.search(r"enum IScalar \{(.*?)\}", text, re.S).group(1))
+        self.slots = {s.strip(): k for k, s in enumerate(names.split(","))}
+        self.dll.test_status_bytes(4 * self.slots["NIS"])
+
+    def status(self, **ints):
+        self.dll.test_status_clear()
+        for name, v in ints.items():
+            self.dll.test_status_int(self.slots[name], v)
+
+    def launches(self):
+        out = self.dll.test_launched().decode().split()
+        self.dll.test_forget_launches()
+        return out
+
+
+def _sim(nx=12, ny=6, nz=6, solver=0, precision=0):
+    from polymps_amd import configs
+    from polymps_amd.lib import Simulation
+    l0 = 0.6 / nx
+    b = (nx * l0, ny * l0, nz * l0)
+    w = configs.dam3d_inc(l0=l0, tank=(1.61, b[1], 2.0 * b[2]), block=b)
+    w.params.solver_type, w.params.precision_mode = solver, precision
+    return Simulation(w.params, w.types, w.pos, w.vel)
+
+
+def _solve(g):
+    g.call("ppe_assemble")
+    g.call("ppe_solve")
+
+
+def allocations(rt, solver, precision, learned):
+    """Whichever of its allocations fails, a solve reports it, and the next
+    one makes every buffer that is missing."""
+    from polymps_amd.lib import MpsError
+    rt.status(I_CG_DONE=1)
+
+    def run(g):
+        if learned:
+            g.gnn_init(0)
+            g.set_scalar("learned_mode", 1)
+        _solve(g)
+
+    def made(fail):
+        g = _sim(solver=solver, precision=precision)
+        live, before = rt.dll.test_live(), rt.dll.test_allocations()
+        rt.dll.test_fail_allocation(fail)
+        failed = False
+        try:
+            run(g)
+        except MpsError as e:
+            assert "out of memory" in str(e), e
+            failed = True
+        rt.dll.test_fail_allocation(0)
+        run(g)
+        n = rt.dll.test_live() - live
+        calls = rt.dll.test_allocations() - before
+        g.close()
+        return n, calls, failed
+
+    clean, calls, failed = made(0)
+    assert clean > 0 and not failed
+    for k in range(1, calls + 1):
+        n, _, failed = made(k)
+        assert failed, k
+        assert n == clean, f"allocation {k} of {calls} failed: {n} buffers afterwards, {clean} without a failure"
+    assert rt.dll.test_live() == 0
+
+
+# ------------------------------------------------------------------ the tests
+@pytest.fixture(scope="module")
+def runtime(built, tmp_path_factory):
+    out = tmp_path_factory.mktemp("runtime") / "libamdhip64.so.7"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(ROOT / "tests" / "host_runtime.cpp"), "-Wl,-soname,libamdhip64.so.7",
+                    f"-Wl,--version-script={ROOT / 'tests' / 'host_runtime.map'}", "-o", str(out)], check=True)
+    return out
+
+
+def _child(runtime, case, *args):
+    res = subprocess.run([sys.executable, __file__, str(runtime), case, *map(str, args)], capture_output=True,
+                         text=True, timeout=300, cwd=ROOT)
+    assert res.returncode == 0, (res.stdout + res.stderr)[-3000:]
+
+
+@pytest.mark.parametrize("solver,precision,learned", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
+def test_allocation_failures(runtime, solver, precision, learned):
+    _child(runtime, "allocations", solver, precision, learned)
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, str(ROOT))
+    globals()[sys.argv[2]](Runtime(sys.argv[1]), *map(int, sys.argv[3:]))
