@@ -2371,10 +2371,11 @@ static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
     const size_t lds = sizeof(double) * (size_t)win16Lds(ctx->N);
     if (ctx->oneLaunchFits[mixed] < 0) {
         int cus = 0, perCu = 0;
-        MPS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->dev));
-        MPS_HIP(hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        MPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k.kernel, k.threads, lds));
-        ctx->oneLaunchFits[mixed] = nb <= perCu * cus ? 1 : 0;
+        hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->dev);
+        if (e == hipSuccess) e = hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k.kernel, k.threads, lds);
+        if (e != hipSuccess) (void)hipGetLastError();   // refused (LDS size): the pieces need no such thing
+        ctx->oneLaunchFits[mixed] = e == hipSuccess && nb <= perCu * cus ? 1 : 0;
     }
     if (!ctx->oneLaunchFits[mixed]) return MPS_OK;
     int rc;

@@ -93,6 +93,20 @@ def allocations(rt, solver, precision, learned):
     assert rt.dll.test_live() == 0
 
 
+def attributes(rt, precision):
+    """A device that refuses the kernel's LDS size gets the solve in pieces."""
+    rt.status(I_CG_DONE=1)
+    names = ("kCgOneLaunch", "kMxOneLaunch")
+    for refuse in (0, 1):
+        rt.dll.test_refuse_attributes(refuse)
+        g = _sim(precision=precision)
+        rt.launches()
+        _solve(g)
+        one = [k for k in rt.launches() if k.startswith(names)]
+        assert len(one) == (0 if refuse else 1), one
+        g.close()
+
+
 # ------------------------------------------------------------------ the tests
 @pytest.fixture(scope="module")
 def runtime(built, tmp_path_factory):
@@ -112,6 +126,11 @@ def _child(runtime, case, *args):
 @pytest.mark.parametrize("solver,precision,learned", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
 def test_allocation_failures(runtime, solver, precision, learned):
     _child(runtime, "allocations", solver, precision, learned)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_refused_kernel_attributes(runtime, precision):
+    _child(runtime, "attributes", precision)
 
 
 if __name__ == "__main__":
