@@ -94,7 +94,9 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * "iterations" "ppe_ms" "true_residual" "fallback" "outer_iterations"
  * "solver_failed" (last pressure solve: 0 converged, 1 stopped above the
  * tolerance, 2 non-finite residual) "solver_failures" (failed solves since
- * the count was last set; settable)
+ * the count was last set; settable) "solve_path" (how the last pressure solve
+ * ran: 0 launched in pieces, 1 in one launch, 2 in pieces because a block of
+ * the matrix has no 16-bit window, 3 in pieces because a grid barrier gave up)
  * "list_max" "list_capacity" "capacity" "nnz" "list_start" (1 when the last
  * step built a list at its start positions) "spmv_ms_total"
  * "spmv_launches" "spmv_bytes_total" (with "profile" on: the time, count and

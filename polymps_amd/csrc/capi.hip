@@ -770,6 +770,7 @@ int mps_get_scalar(mps_ctx* ctx, const char* name, double* out) {
         if (rc2) return rc2;
     }
     else if (s == "solver_failed") *out = ctx->solverFailed;
+    else if (s == "solve_path") *out = ctx->solvePath;
     else if (s == "cfl_visc") {
         const int rc2 = granularCflVisc(ctx, out);
         if (rc2) return rc2;

@@ -56,8 +56,16 @@ enum DScalar { S_VELMAX, S_ABSNEW, S_ABSOLD, S_RHSN2, S_THR, S_RN2, S_ALPHA, S_B
 enum IScalar { I_NLIVE, I_OUTCNT, I_OVERFLOW, I_CG_ITER, I_CG_OUTER, I_CG_DONE, I_COMPACT_OVF,
                I_NESC, I_NLCESC, I_NOWIN,   // zeroed together by each assembly; I_NOWIN: no solve in one launch
                I_BCG_RESTART, I_BCG_RESTARTS, I_REBUILD, I_PATCHCNT, I_FIXCNT,
-               I_GRID_LATE,   // a solve in one launch left without a result
+               I_GRID_LATE,   // a grid barrier of a solve in one launch gave up
                NIS };
+
+// how a pressure solve ran
+enum SolvePath {
+    SOLVE_PIECES,       // launched in pieces
+    SOLVE_ONE_LAUNCH,   // in one launch
+    SOLVE_NO_WINDOW,    // in pieces, as a block of the matrix has no 16-bit window
+    SOLVE_LATE,         // in pieces, after a grid barrier gave up
+};
 
 constexpr int kWallTable = 50;
 // escaped (non-delta) columns per PPE row: the first entry and stencil-row
@@ -259,6 +267,7 @@ struct Ctx {
     double* gridPart = nullptr;
     double* gridP2 = nullptr;
     int oneLaunchFits[2] = {-1, -1};
+    SolvePath solvePath = SOLVE_PIECES;   // of the last pressure solve (solve_path scalar)
     int asmBlocks = 0;           // blocks (partials) of the last assembly
     double* cgSums = nullptr;    // block sums of a CG iteration's vector update (kRedBlocks pairs)
     double* asmRed = nullptr;    // block partials of the assembly's first residual (no other kernel writes them)

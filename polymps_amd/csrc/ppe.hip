@@ -1596,10 +1596,7 @@ __global__ __launch_bounds__(BT, 4) void kCgOneLaunch(KArgs a, CgPtrs c, OneLaun
     const bool row = i < a.N;
     const bool own = row && groupLaneId<L>() == 0;   // the row's lane that stores and counts
     const int* const table = c.win + (size_t)(blockIdx.x * (BT / L) / kB) * kWinStride;
-    if (!o.full && a.is[I_NOWIN]) {   // every block leaves
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.is[I_GRID_LATE] = 1;
-        return;
-    }
+    if (!o.full && a.is[I_NOWIN]) return;   // every block leaves (launchOneLaunch reads the flag)
     const Window w = loadWindow(table, o.full, a.N);
     const int KE = ellWidth(a.K), cap = win16Lds(a.N);
     const int n = row ? c.cnt[i] : 0;
@@ -1713,10 +1710,7 @@ __global__ __launch_bounds__(BT, 4) void kMxOneLaunch(KArgs a, CgPtrs c, OneLaun
     const bool row = i < a.N;
     const bool own = row && groupLaneId<L>() == 0;
     const int* const table = c.win + (size_t)(blockIdx.x * (BT / L) / kB) * kWinStride;
-    if (!o.full && a.is[I_NOWIN]) {   // every block leaves
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.is[I_GRID_LATE] = 1;
-        return;
-    }
+    if (!o.full && a.is[I_NOWIN]) return;   // every block leaves (launchOneLaunch reads the flag)
     const Window w = loadWindow(table, o.full, a.N);
     const int KE = ellWidth(a.K), cap = win16Lds(a.N);
     const int n = row ? c.cnt[i] : 0;
@@ -2394,8 +2388,9 @@ static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
     return MPS_OK;
 }
 
-// *solved: false when a block has no window or a grid barrier gave up; the guess and the system are
-// still valid then and the solve goes on in pieces.
+// *solved: false when a block has no window or a grid barrier gave up
+// (ctx->solvePath says which); the guess and the system are still valid then
+// and the solve goes on in pieces.
 static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c, double tol, double tolIn, int maxIt,
                            int maxOuter, bool* solved) {
     const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
@@ -2421,8 +2416,11 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
                             sizeof(double) * (size_t)win16Lds(ctx->N), ctx->stream));
     const int rc = readStatus(ctx, nullptr, 0);
     if (rc) return rc;
-    *solved = ctx->hostInts[I_GRID_LATE] == 0;
-    if (!*solved) MPS_HIP(hipMemsetAsync(ctx->is + I_GRID_LATE, 0, sizeof(int), ctx->stream));
+    ctx->solvePath = !o.full && ctx->hostInts[I_NOWIN] ? SOLVE_NO_WINDOW
+                     : ctx->hostInts[I_GRID_LATE]      ? SOLVE_LATE
+                                                       : SOLVE_ONE_LAUNCH;
+    if (ctx->solvePath == SOLVE_LATE) MPS_HIP(hipMemsetAsync(ctx->is + I_GRID_LATE, 0, sizeof(int), ctx->stream));
+    *solved = ctx->solvePath == SOLVE_ONE_LAUNCH;
     return MPS_OK;
 }
 
@@ -2691,6 +2689,7 @@ int ppeSolve(Ctx* ctx) {
     }
     MPS_HIP(hipEventRecord(ctx->ev0, s));
     ctx->fallbackUsed = 0;
+    ctx->solvePath = SOLVE_PIECES;
     int rc;
     if (ctx->P.learned_mode >= 1) {
         // learned operator for this matrix, then x += M (b - A x)

@@ -16,6 +16,8 @@ from polymps_amd.lib import Simulation
 
 pytestmark = pytest.mark.gpu
 
+PIECES, ONE_LAUNCH, NO_WINDOW, LATE = range(4)   # solve_path
+
 
 def _block(nx, ny, nz, thin=0):
     l0 = 0.6 / nx
@@ -39,6 +41,35 @@ def _solve(g, guess, pieces):
     return g.get("ppe_x"), int(g.scalar("solver_iter")), g.scalar("true_residual")
 
 
+def _widest_window(g):
+    """Slots of the widest window: per 256-row block the union of its rows'
+    stencil rows, in the slot order of the buckets (every row has entries)."""
+    p, pos = g.params, g.get("pos").reshape(-1, 3)
+    nb = np.array([p.num_buckets_x, p.num_buckets_y, p.num_buckets_z])
+    c = np.floor((pos - np.array(p.domain_min)) * p.inv_bucket_side + 1e-8).astype(int)
+    key = (c[:, 2] * nb[1] + c[:, 1]) * nb[0] + c[:, 0]
+    order = np.argsort(key, kind="stable")
+    c = c[order]
+    start = np.searchsorted(key[order], np.arange(nb.prod() + 1))
+    widest = 0
+    for a in range(0, len(c), 256):
+        s = []
+        for dz in (-1, 0, 1):
+            for dy in (-1, 0, 1):
+                q = c[a:a + 256] + [0, dy, dz]
+                q = q[((q >= 0) & (q < nb)).all(axis=1)]
+                if len(q):
+                    row = (q[:, 2] * nb[1] + q[:, 1]) * nb[0]
+                    s.append((start[row + np.maximum(q[:, 0] - 1, 0)].min(),
+                              start[row + np.minimum(q[:, 0] + 1, nb[0] - 1) + 1].max()))
+        size, last = 0, 0
+        for lo, hi in sorted(s):
+            size += max(0, hi - max(lo, last))
+            last = max(last, hi)
+        widest = max(widest, size)
+    return widest
+
+
 def _residual(m, b, x):
     rp, cols, vals = m
     rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
@@ -46,7 +77,7 @@ def _residual(m, b, x):
     return np.linalg.norm(r) / np.linalg.norm(b)
 
 
-def _check(w, precision):
+def _check(w, precision, path=ONE_LAUNCH):
     w.params.precision_mode = precision
     w.params.ppe_transpose = 0
     w.params.solver_tol = 1e-8
@@ -55,16 +86,19 @@ def _check(w, precision):
     g.call("init")
     guess = 0.9 * g.get("press") + 1e-3 * configs.splitmix64_uniform(5, n)
     x0, it0, res0 = _solve(g, guess, True)
+    assert g.scalar("solve_path") == PIECES
     x1, it1, res1 = _solve(g, guess, False)
+    assert g.scalar("solve_path") == path
     m, b = g.ppe_matrix(), g.get("ppe_b")
     print(f"one launch {n} precision {precision}: {it0} and {it1} iterations, residuals {res0:.2e} {res1:.2e}", flush=True)
     assert it0 > 0 and abs(it1 - it0) <= 1 + it0 // 50
     # FP64 stops on the recurrence's residual, which drifts from the true one
     # by a few roundings of x per iteration: a hundredth of 1e-8 covers it
-    assert res1 <= 1.01e-8
     # the reported residual is the matrix's, up to the rounding of its sums
     # (120 products of up to |a||x| ~ |b| each, eps 2.2e-16, against 1e-8)
-    assert abs(_residual(m, b, x1) - res1) <= 1e-3 * res1 + 1e-13
+    for x, res in ((x0, res0), (x1, res1)):
+        assert res <= 1.01e-8
+        assert abs(_residual(m, b, x) - res) <= 1e-3 * res + 1e-13
     press = g.get("press")
     assert np.array_equal(press, np.where(x1 < 0, 0.0, x1))
     # a second solve from the same guess gives the same bits: sums in a fixed order
@@ -77,7 +111,8 @@ def _check(w, precision):
 @pytest.mark.parametrize("shape", [(7, 5, 3), (32, 16, 32), (32, 27, 19), (64, 32, 32), (64, 41, 25), (64, 64, 32),
                                    (76, 69, 25)])
 def test_sizes(built, shape, precision):
-    _check(_block(*shape), precision)
+    w = _block(*shape)
+    _check(w, precision, ONE_LAUNCH if w.n <= 131072 else PIECES)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -94,8 +129,9 @@ def test_wide_windows(built, shape, precision):
     65,536 rows such a window is staged in parts (three in FP64, two in FP32
     here), above the solve goes back to pieces."""
     w = _block(*shape, thin=300)
-    g = _check(w, precision)
-    assert g.scalar("ppe_window_blocks") < (len(w.types) + 255) // 256
+    small = len(w.types) <= 65536
+    g = _check(w, precision, ONE_LAUNCH if small else NO_WINDOW)
+    assert _widest_window(g) > (16384 if small else 9216)   # slots of the LDS
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -103,7 +139,7 @@ def test_wide_windows(built, shape, precision):
 def test_pieces(built, shape, precision):
     """Larger systems: the vector kernels take one row per thread up to 262,144
     rows and several above, and add the SpMV's sums themselves up to 393,216."""
-    _check(_block(*shape), precision)
+    _check(_block(*shape), precision, PIECES)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -120,10 +156,13 @@ def test_blocks_that_do_not_meet(built, shape, precision):
     g.call("init")
     guess = 0.9 * g.get("press") + 1e-3 * configs.splitmix64_uniform(5, w.n)
     x0, it0, _ = _solve(g, guess, False)
+    assert g.scalar("solve_path") == ONE_LAUNCH
     g.set_scalar("grid_spin", 1)
     x1, it1, res1 = _solve(g, guess, False)
+    assert g.scalar("solve_path") == LATE
     assert abs(it1 - it0) <= 1 and res1 <= 1.01e-8
     assert _residual(g.ppe_matrix(), g.get("ppe_b"), x1) <= 1.01e-8
     g.set_scalar("grid_spin", 65536)
     x2, it2, _ = _solve(g, guess, False)
+    assert g.scalar("solve_path") == ONE_LAUNCH
     assert it2 == it0 and np.array_equal(x0, x2)

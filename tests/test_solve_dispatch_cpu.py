@@ -93,16 +93,43 @@ def allocations(rt, solver, precision, learned):
     assert rt.dll.test_live() == 0
 
 
+ONE_LAUNCH = ("kCgOneLaunch", "kMxOneLaunch")
+
+
+def path(rt, precision):
+    """solve_path says what was launched: the one launch alone, or the pieces
+    after it and why, or the pieces alone."""
+    g = _sim(precision=precision)
+    if precision:
+        # a mixed solve in pieces reads |r|^2 and |b|^2 as 0 here and ends before its first pass
+        pieces = "kTrueResidualFinish"
+    else:
+        pieces = "kCgSpmv"
+    for ints, want in ((dict(), 1), (dict(I_NOWIN=1), 2), (dict(I_GRID_LATE=1), 3), (dict(), 1)):
+        rt.status(I_CG_DONE=1, **ints)
+        rt.launches()
+        _solve(g)
+        got = rt.launches()
+        assert any(k.startswith(ONE_LAUNCH) for k in got)
+        assert any(k == pieces for k in got) == (want != 1), (want, got)
+        assert g.scalar("solve_path") == want
+    g.close()
+    rt.status(I_CG_DONE=1)
+    g = _sim(solver=1)
+    _solve(g)
+    assert g.scalar("solve_path") == 0
+    g.close()
+
+
 def attributes(rt, precision):
     """A device that refuses the kernel's LDS size gets the solve in pieces."""
     rt.status(I_CG_DONE=1)
-    names = ("kCgOneLaunch", "kMxOneLaunch")
     for refuse in (0, 1):
         rt.dll.test_refuse_attributes(refuse)
         g = _sim(precision=precision)
         rt.launches()
         _solve(g)
-        one = [k for k in rt.launches() if k.startswith(names)]
+        one = [k for k in rt.launches() if k.startswith(ONE_LAUNCH)]
         assert len(one) == (0 if refuse else 1), one
         g.close()
 
@@ -126,6 +153,11 @@ def _child(runtime, case, *args):
 @pytest.mark.parametrize("solver,precision,learned", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
 def test_allocation_failures(runtime, solver, precision, learned):
     _child(runtime, "allocations", solver, precision, learned)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_solve_path(runtime, precision):
+    _child(runtime, "path", precision)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
