@@ -2395,7 +2395,6 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
                            int maxOuter, bool* solved) {
     const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
     const bool fresh = ctx->r0Fresh && ctx->r0FreshMixed == mixed;
-    ctx->r0Fresh = false;
     OneLaunch o;
     o.bar = ctx->gridBar;
     o.part = ctx->gridPart;
@@ -2419,6 +2418,8 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
     ctx->solvePath = !o.full && ctx->hostInts[I_NOWIN] ? SOLVE_NO_WINDOW
                      : ctx->hostInts[I_GRID_LATE]      ? SOLVE_LATE
                                                        : SOLVE_ONE_LAUNCH;
+    // without a window the launch has touched nothing: the assembly's residual serves the pieces
+    if (ctx->solvePath != SOLVE_NO_WINDOW) ctx->r0Fresh = false;
     if (ctx->solvePath == SOLVE_LATE) MPS_HIP(hipMemsetAsync(ctx->is + I_GRID_LATE, 0, sizeof(int), ctx->stream));
     *solved = ctx->solvePath == SOLVE_ONE_LAUNCH;
     return MPS_OK;

@@ -113,6 +113,9 @@ def path(rt, precision):
         assert any(k.startswith(ONE_LAUNCH) for k in got)
         assert any(k == pieces for k in got) == (want != 1), (want, got)
         assert g.scalar("solve_path") == want
+        # the assembly's residual serves the pieces unless blocks may have moved the guess
+        first = "kTrueResidual" if precision else "kCgStart"
+        assert got.count(first) == (1 if want == 3 else 0)
     g.close()
     rt.status(I_CG_DONE=1)
     g = _sim(solver=1)
