@@ -101,7 +101,7 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * step built a list at its start positions) "spmv_ms_total"
  * "spmv_launches" "spmv_bytes_total" (with "profile" on: the time, count and
  * algorithmic bytes of the timed SpMV launches, every eighth launch of a
- * batch) "list_skin" (skin of the last step's
+ * batch; a solve in one launch has none) "list_skin" (skin of the last step's
  * kept neighbour list, in l0; 0: built after the prediction) "list_rebuilt"
  * (1 when the last step rebuilt its list after the prediction)
  * "list_entries" "list_entries_small" (entries of the current neighbour
@@ -114,7 +114,8 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * the largest one-step displacement, in [2, 10], default 3) "mask_words" (candidate
  * window per stencil row in 32-slot words, at most the allocated width;
  * particles with a longer row are listed by a direct walk, same results)
- * "profile" (nonzero: time every eighth SpMV launch with HIP events, counters reset)
+ * "profile" (nonzero: time every eighth SpMV launch with HIP events, counters
+ * reset; results do not change)
  * "precision_mode" (MPS_PREC_*, used from the next PPE assembly)
  * "learned_mode" (0 off, 1 learned warm start, 2 warm start + learned
  * flexible-CG preconditioner) "learned_stall_ratio" (in (0, 1), default
@@ -128,7 +129,10 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * used from the next assembly; read-only "ppe_window_blocks": blocks of the
  * last assembly served from a window, "window_escapes": window index
  * escapes of the last assembly, the rows' absolute indices next to their
- * one-byte steps) "grid_spin" (set only, [1, 2^20], default 65536: polls
+ * one-byte steps) "one_launch" (1 default: CG solves of up
+ * to 131,072 rows, 16,384 in a periodic domain, run in one launch, from the
+ * next assembly on; 0: always in pieces; the two round differently)
+ * "grid_spin" (set only, [1, 2^20], default 65536: polls
  * before a grid barrier of a solve in one launch gives up and the solve runs
  * in pieces) "ppe_warm_start" (initial guess of each
  * pressure solve: 0 previous solution, 1 / 2 / 3 linear / quadratic / cubic

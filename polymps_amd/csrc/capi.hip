@@ -770,6 +770,7 @@ int mps_get_scalar(mps_ctx* ctx, const char* name, double* out) {
         if (rc2) return rc2;
     }
     else if (s == "solver_failed") *out = ctx->solverFailed;
+    else if (s == "one_launch") *out = ctx->oneLaunch ? 1.0 : 0.0;
     else if (s == "solve_path") *out = ctx->solvePath;
     else if (s == "cfl_visc") {
         const int rc2 = granularCflVisc(ctx, out);
@@ -876,6 +877,14 @@ int mps_set_scalar(mps_ctx* ctx, const char* name, double value) {
             return MPS_E_ARG;
         }
         ctx->ppeWindow = value != 0.0;
+    } else if (s == "one_launch") {
+        // CG solves of small systems in one launch (1, default, from the next
+        // assembly on) or always in pieces (0)
+        if (!(value == 0.0 || value == 1.0)) {
+            ctx->err = "one_launch must be 0 or 1";
+            return MPS_E_ARG;
+        }
+        ctx->oneLaunch = value != 0.0;
     } else if (s == "mask_words") {
         // candidate window of a stencil row in 32-slot words (at most the
         // allocated width); rows beyond it are listed by a direct walk

@@ -262,6 +262,7 @@ struct Ctx {
     bool r0FreshMixed = false;   // ... in the mixed solve's partial order (else the FP64 CG's, with 1/diag)
     // solves in one launch (allocated on first use): barrier counters,
     // block sums, the second search direction; whether the device holds the grid (per precision)
+    bool oneLaunch = true;       // one_launch scalar
     int gridSpin = 1 << 16;      // polls (of about 0.7 us) before a grid barrier gives up (grid_spin scalar)
     unsigned* gridBar = nullptr;
     double* gridPart = nullptr;

@@ -1925,12 +1925,12 @@ static bool periodicCtx(const Ctx* ctx) { return ctx->P.domain_type_bc == 1; }
 // assembly writes then
 static bool oneLaunchRows(const Ctx* ctx) { return ctx->N <= (periodicCtx(ctx) ? kFullMax : kOneLaunchMax); }
 
-static int ensureWindows(Ctx* ctx, bool bytes) {
+static int ensureWindows(Ctx* ctx, bool bytes, bool index16) {
     const size_t entries = (size_t)ellWidth(ctx->K) * ellRows(ctx->N);
     int rc = ensureBuffer(ctx, &ctx->aWin, (size_t)kWinStride * gridFor(ctx->N, kB));
     if (!rc && bytes) rc = ensureBuffer(ctx, &ctx->aLc8, entries);
     if (!rc && bytes) rc = ensureBuffer(ctx, &ctx->aLcEsc, (size_t)kLcEsc * ellRows(ctx->N));
-    if (!rc && oneLaunchRows(ctx)) rc = ensureBuffer(ctx, &ctx->aLc16, entries);
+    if (!rc && index16) rc = ensureBuffer(ctx, &ctx->aLc16, entries);
     return rc;
 }
 
@@ -1970,9 +1970,9 @@ int ppeAssemble(Ctx* ctx) {
     // and those of a solve in one launch, whatever the scalar says
     const bool wins = !bicg && ctx->ppeWindow;
     // (the learned preconditioner's solve runs in pieces)
-    const bool wins16 = !bicg && oneLaunchRows(ctx) && !(mixed && ctx->P.learned_mode == 2 && ctx->gnn != nullptr);
+    const bool wins16 = !bicg && ctx->oneLaunch && oneLaunchRows(ctx) && !(mixed && ctx->P.learned_mode == 2 && ctx->gnn != nullptr);
     if (wins || wins16) {
-        int rc = ensureWindows(ctx, wins);
+        int rc = ensureWindows(ctx, wins, wins16);
         if (rc) return rc;
     }
     unsigned char* lc8 = wins ? ctx->aLc8 : nullptr;
@@ -2354,11 +2354,10 @@ static OneLaunchKind oneLaunchKind(int N, bool mixed) {
 
 // Whether the CG solve of the last assembly runs in one launch: it left the
 // 16-bit window indices, and the device holds every block of the grid at once
-// (asked of the runtime for the kernel, once per context).  Not while SpMV
-// launches are timed one by one.
+// (asked of the runtime for the kernel, once per context).
 static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
     *fits = false;
-    if (ctx->profile || !ctx->win16Valid) return MPS_OK;
+    if (!ctx->oneLaunch || !ctx->win16Valid) return MPS_OK;
     const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
     if (!k.kernel) return MPS_OK;
     const int nb = gridFor(ctx->N, k.rows);

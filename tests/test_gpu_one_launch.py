@@ -2,8 +2,7 @@
 
 Up to 131,072 rows (16,384 in a periodic domain) the CG runs as one launch
 whose blocks meet at grid barriers; the pieces still serve larger systems,
-timed SpMV launches (the profile scalar) and systems whose blocks have no
-16-bit window.  The sizes lie on both sides of the lines between the kinds.
+the one_launch scalar at 0 and systems whose blocks have no 16-bit window.  The sizes lie on both sides of the lines between the kinds.
 Both solves stop by the same test on the same residual, so they take the same
 number of iterations up to the rounding of the sums, and the answer is judged
 by its residual on the assembled matrix.
@@ -34,7 +33,7 @@ def _block(nx, ny, nz, thin=0):
 
 
 def _solve(g, guess, pieces):
-    g.set_scalar("profile", 1 if pieces else 0)
+    g.set_scalar("one_launch", 0 if pieces else 1)
     g.set("ppe_x", guess)
     g.call("ppe_assemble")
     g.call("ppe_solve")
@@ -113,6 +112,28 @@ def _check(w, precision, path=ONE_LAUNCH):
 def test_sizes(built, shape, precision):
     w = _block(*shape)
     _check(w, precision, ONE_LAUNCH if w.n <= 131072 else PIECES)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_profile_changes_no_result(built, precision):
+    """Timing does not choose the solver: same path, same bits."""
+    w = _block(32, 16, 16)
+    w.params.precision_mode = precision
+    print(f"profile {w.n} precision {precision}", flush=True)
+    g = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh, device=0)
+    g.call("init")
+    guess = 0.9 * g.get("press")
+    x0, it0, _ = _solve(g, guess, False)
+    g.set_scalar("profile", 1)
+    x1, it1, _ = _solve(g, guess, False)
+    assert g.scalar("solve_path") == ONE_LAUNCH and g.scalar("spmv_launches") == 0
+    assert it0 == it1 and np.array_equal(x0, x1)
+    # the pieces are timed, with the same bits too
+    p0, _, _ = _solve(g, guess, True)
+    assert g.scalar("solve_path") == PIECES and g.scalar("spmv_launches") > 0
+    g.set_scalar("profile", 0)
+    p1, _, _ = _solve(g, guess, True)
+    assert np.array_equal(p0, p1)
 
 
 @pytest.mark.parametrize("precision", [0, 1])

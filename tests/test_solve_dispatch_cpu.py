@@ -124,6 +124,37 @@ def path(rt, precision):
     g.close()
 
 
+def switches(rt, precision):
+    """one_launch chooses the solver and the memory of its windows; profile does not."""
+    from polymps_amd.lib import MpsError
+    rt.status(I_CG_DONE=1)
+    g = _sim(precision=precision)
+    live = rt.dll.test_live()
+    g.set_scalar("ppe_window", 0)
+    g.set_scalar("one_launch", 0)
+    for profile in (0, 1):
+        g.set_scalar("profile", profile)
+        rt.launches()
+        _solve(g)
+        assert not any(k.startswith(ONE_LAUNCH) for k in rt.launches())
+        assert g.scalar("solve_path") == 0 and g.scalar("one_launch") == 0
+    # neither windows nor the buffers of a solve in one launch (a mixed solve makes its eight, profile the entry sum)
+    assert rt.dll.test_live() - live == (9 if precision else 1)
+    g.set_scalar("one_launch", 1)
+    for profile in (0, 1):
+        g.set_scalar("profile", profile)
+        rt.launches()
+        _solve(g)
+        assert sum(k.startswith(ONE_LAUNCH) for k in rt.launches()) == 1
+        assert g.scalar("solve_path") == 1
+    try:
+        g.set_scalar("one_launch", 2)
+        raise AssertionError("one_launch 2 was accepted")
+    except MpsError:
+        pass
+    g.close()
+
+
 def attributes(rt, precision):
     """A device that refuses the kernel's LDS size gets the solve in pieces."""
     rt.status(I_CG_DONE=1)
@@ -161,6 +192,11 @@ def test_allocation_failures(runtime, solver, precision, learned):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_solve_path(runtime, precision):
     _child(runtime, "path", precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_switches(runtime, precision):
+    _child(runtime, "switches", precision)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
