@@ -96,7 +96,9 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * tolerance, 2 non-finite residual) "solver_failures" (failed solves since
  * the count was last set; settable) "solve_path" (how the last pressure solve
  * ran: 0 launched in pieces, 1 in one launch, 2 in pieces because a block of
- * the matrix has no 16-bit window, 3 in pieces because a grid barrier gave up)
+ * the matrix has no 16-bit window, 3 in pieces because a grid barrier gave up,
+ * 4 in pieces because one did not long ago) "solve_repeats" (solves repeated in
+ * pieces after a barrier gave up)
  * "list_max" "list_capacity" "capacity" "nnz" "list_start" (1 when the last
  * step built a list at its start positions) "spmv_ms_total"
  * "spmv_launches" "spmv_bytes_total" (with "profile" on: the time, count and
@@ -132,9 +134,10 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * one-byte steps) "one_launch" (1 default: CG solves of up
  * to 131,072 rows, 16,384 in a periodic domain, run in one launch, from the
  * next assembly on; 0: always in pieces; the two round differently)
- * "grid_spin" (set only, [1, 2^20], default 65536: polls
- * before a grid barrier of a solve in one launch gives up and the solve runs
- * in pieces) "ppe_warm_start" (initial guess of each
+ * "grid_spin" ([1, 2^20], default 4096: polls of about 0.3 us before a grid
+ * barrier of a solve in one launch gives up, as where another context keeps
+ * its blocks out; that solve and the next 4, 8, ... 1,024 run in pieces;
+ * setting it makes the next solve try again) "ppe_warm_start" (initial guess of each
  * pressure solve: 0 previous solution, 1 / 2 / 3 linear / quadratic / cubic
  * extrapolation of the last solutions) "mesh_bvh" (closest-point search: -1 BVH for
  * meshes above 64 faces, 0 brute force, 1 BVH; both give the same result). */

@@ -772,6 +772,8 @@ int mps_get_scalar(mps_ctx* ctx, const char* name, double* out) {
     else if (s == "solver_failed") *out = ctx->solverFailed;
     else if (s == "one_launch") *out = ctx->oneLaunch ? 1.0 : 0.0;
     else if (s == "solve_path") *out = ctx->solvePath;
+    else if (s == "solve_repeats") *out = (double)ctx->solveRepeats;
+    else if (s == "grid_spin") *out = ctx->gridSpin;
     else if (s == "cfl_visc") {
         const int rc2 = granularCflVisc(ctx, out);
         if (rc2) return rc2;
@@ -833,6 +835,7 @@ int mps_set_scalar(mps_ctx* ctx, const char* name, double value) {
             return MPS_E_ARG;
         }
         ctx->gridSpin = (int)value;
+        ctx->lateRow = ctx->lateSkip = 0;   // another patience: the next solve tries again
     } else if (s == "profile") {
         ctx->profile = value != 0.0;
         ctx->spmvMsTotal = 0.0;

@@ -65,6 +65,7 @@ enum SolvePath {
     SOLVE_ONE_LAUNCH,   // in one launch
     SOLVE_NO_WINDOW,    // in pieces, as a block of the matrix has no 16-bit window
     SOLVE_LATE,         // in pieces, after a grid barrier gave up
+    SOLVE_BACKOFF,      // in pieces, as an earlier solve's barrier gave up (Ctx::lateSkip)
 };
 
 constexpr int kWallTable = 50;
@@ -263,7 +264,10 @@ struct Ctx {
     // solves in one launch (allocated on first use): barrier counters,
     // block sums, the second search direction; whether the device holds the grid (per precision)
     bool oneLaunch = true;       // one_launch scalar
-    int gridSpin = 1 << 16;      // polls (of about 0.7 us) before a grid barrier gives up (grid_spin scalar)
+    int gridSpin = 1 << 12;      // polls before a grid barrier gives up (grid_spin scalar)
+    int lateRow = 0;             // give-ups without a solve in one launch between them
+    int lateSkip = 0;            // solves still to run in pieces after the last one
+    long solveRepeats = 0;       // solves repeated in pieces after a give-up
     unsigned* gridBar = nullptr;
     double* gridPart = nullptr;
     double* gridP2 = nullptr;

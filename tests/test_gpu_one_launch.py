@@ -15,7 +15,7 @@ from polymps_amd.lib import Simulation
 
 pytestmark = pytest.mark.gpu
 
-PIECES, ONE_LAUNCH, NO_WINDOW, LATE = range(4)   # solve_path
+PIECES, ONE_LAUNCH, NO_WINDOW, LATE, BACKOFF = range(5)   # solve_path
 
 
 def _block(nx, ny, nz, thin=0):
@@ -167,8 +167,8 @@ def test_pieces(built, shape, precision):
 @pytest.mark.parametrize("shape", [(24, 6, 12), (64, 32, 32), (64, 41, 25)])
 def test_blocks_that_do_not_meet(built, shape, precision):
     """A wait of one poll: blocks give up at their first barriers, all leave,
-    and the solve runs in pieces with the same answer; the counters are at
-    zero for the next solve, which meets again."""
+    and the solve runs in pieces with the same answer, as does the next one;
+    the counters are at zero for the next launch, which meets again."""
     w = _block(*shape)
     w.params.precision_mode = precision
     w.params.ppe_transpose = 0
@@ -180,7 +180,12 @@ def test_blocks_that_do_not_meet(built, shape, precision):
     assert g.scalar("solve_path") == ONE_LAUNCH
     g.set_scalar("grid_spin", 1)
     x1, it1, res1 = _solve(g, guess, False)
-    assert g.scalar("solve_path") == LATE
+    assert g.scalar("solve_path") == LATE and g.scalar("solve_repeats") == 1
+    x3, _, _ = _solve(g, guess, False)
+    assert g.scalar("solve_path") == BACKOFF and g.scalar("solve_repeats") == 1
+    # by other kernels than a retry, from the residual the assembly left: the same system and
+    # guess, both answers at a residual of 1e-8
+    assert _residual(g.ppe_matrix(), g.get("ppe_b"), x3) <= 1.01e-8
     assert abs(it1 - it0) <= 1 and res1 <= 1.01e-8
     assert _residual(g.ppe_matrix(), g.get("ppe_b"), x1) <= 1.01e-8
     g.set_scalar("grid_spin", 65536)

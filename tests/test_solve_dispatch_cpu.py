@@ -107,6 +107,7 @@ def path(rt, precision):
         pieces = "kCgSpmv"
     for ints, want in ((dict(), 1), (dict(I_NOWIN=1), 2), (dict(I_GRID_LATE=1), 3), (dict(), 1)):
         rt.status(I_CG_DONE=1, **ints)
+        g.set_scalar("grid_spin", 4096)   # tries again after a give-up
         rt.launches()
         _solve(g)
         got = rt.launches()
@@ -121,6 +122,49 @@ def path(rt, precision):
     g = _sim(solver=1)
     _solve(g)
     assert g.scalar("solve_path") == 0
+    g.close()
+
+
+def backoff(rt, precision):
+    """After a barrier gave up the next solves run in pieces without a try, 4
+    of them, then twice as many each time; a solve in one launch starts over."""
+    g = _sim(precision=precision)
+    assert g.scalar("grid_spin") == 4096
+    paths = []
+
+    def solves(n):
+        for _ in range(n):
+            rt.launches()
+            _solve(g)
+            paths.append(int(g.scalar("solve_path")))
+            tried = any(k.startswith(ONE_LAUNCH) for k in rt.launches())
+            assert tried == (paths[-1] != 4)
+
+    rt.status(I_CG_DONE=1, I_GRID_LATE=1)
+    solves(1 + 4 + 1 + 8 + 1 + 16 + 1)
+    assert paths == [3] + 4 * [4] + [3] + 8 * [4] + [3] + 16 * [4] + [3]
+    assert g.scalar("solve_repeats") == 4
+    rt.status(I_CG_DONE=1)
+    paths.clear()
+    solves(32 + 2)
+    assert paths == 32 * [4] + [1, 1]
+    rt.status(I_CG_DONE=1, I_GRID_LATE=1)
+    paths.clear()
+    solves(6)
+    assert paths == [3, 4, 4, 4, 4, 3]
+    rt.status(I_CG_DONE=1)
+    g.set_scalar("grid_spin", 100)
+    paths.clear()
+    solves(1)
+    assert paths == [1] and g.scalar("grid_spin") == 100
+    # the longest wait
+    rt.status(I_CG_DONE=1, I_GRID_LATE=1)
+    paths.clear()
+    while paths.count(3) < 12:
+        solves(1)
+    late = [k for k, p in enumerate(paths) if p == 3]
+    gaps = [b - a - 1 for a, b in zip(late, late[1:])]
+    assert gaps == [4, 8, 16, 32, 64, 128, 256, 512, 1024, 1024, 1024]
     g.close()
 
 
@@ -192,6 +236,11 @@ def test_allocation_failures(runtime, solver, precision, learned):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_solve_path(runtime, precision):
     _child(runtime, "path", precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_backoff(runtime, precision):
+    _child(runtime, "backoff", precision)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
