@@ -264,6 +264,7 @@ struct Ctx {
     // solves in one launch (allocated on first use): barrier counters,
     // block sums, the second search direction; whether the device holds the grid (per precision)
     bool oneLaunch = true;       // one_launch scalar
+    bool noWindow = false;       // the last solve had a block without a 16-bit window: look before launching
     int gridSpin = 1 << 12;      // polls before a grid barrier gives up (grid_spin scalar)
     int lateRow = 0;             // give-ups without a solve in one launch between them
     int lateSkip = 0;            // solves still to run in pieces after the last one

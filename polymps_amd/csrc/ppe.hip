@@ -1046,10 +1046,16 @@ __global__ void kCgStart(KArgs a, CgPtrs c) {
     writePartials(a, s0, s1);
 }
 
-__global__ void kCgStartFinish(KArgs a, int nb, double tol) {
+// noWin: the solve goes on in pieces for want of a window only; where every
+// block has one after all, the queue ends here (flag 6)
+__global__ void kCgStartFinish(KArgs a, int nb, double tol, int noWin) {
     double bn2, rn2;
     finishPartials(a.red, nb, bn2, rn2);
     if (threadIdx.x != 0) return;
+    if (noWin && a.is[I_NOWIN] == 0) {
+        a.is[I_CG_DONE] = 6;
+        return;
+    }
     a.ds[S_RHSN2] = bn2;
     a.ds[S_RN2] = rn2;
     a.is[I_CG_ITER] = 0;
@@ -2360,8 +2366,16 @@ static OneLaunchKind oneLaunchKind(int N, bool mixed) {
 // Whether the CG solve of the last assembly runs in one launch: it left the
 // 16-bit window indices, and the device holds every block of the grid at once
 // (asked of the runtime for the kernel, once per context).
-static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
+//
+// *probe: after a solve that found a block without a window the pieces are
+// queued first and the flag is read with their first status; a launch comes
+// only where it is down again (a developed flow keeps such blocks for
+// thousands of steps, and a launch that leaves at once costs its status read:
+// 0.515 against 0.48 ms per solve of 83,204 rows).  Either way the matrix
+// alone decides which of the two solves it.
+static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits, bool* probe) {
     *fits = false;
+    *probe = false;
     if (!ctx->oneLaunch || !ctx->win16Valid) return MPS_OK;
     const OneLaunchKind k = oneLaunchKind(ctx->N, mixed);
     if (!k.kernel) return MPS_OK;
@@ -2393,7 +2407,9 @@ static int oneLaunchFits(Ctx* ctx, bool mixed, bool* fits) {
         ctx->solvePath = SOLVE_BACKOFF;
         return MPS_OK;
     }
-    *fits = true;
+    *probe = ctx->noWindow && !periodicCtx(ctx);
+    if (*probe) ctx->solvePath = SOLVE_NO_WINDOW;
+    *fits = !*probe;
     return MPS_OK;
 }
 
@@ -2428,7 +2444,8 @@ static int launchOneLaunch(Ctx* ctx, bool mixed, const KArgs& a, const CgPtrs& c
                      : ctx->hostInts[I_GRID_LATE]      ? SOLVE_LATE
                                                        : SOLVE_ONE_LAUNCH;
     // without a window the launch has touched nothing: the assembly's residual serves the pieces
-    if (ctx->solvePath != SOLVE_NO_WINDOW) ctx->r0Fresh = false;
+    ctx->noWindow = ctx->solvePath == SOLVE_NO_WINDOW;
+    if (!ctx->noWindow) ctx->r0Fresh = false;
     if (ctx->solvePath == SOLVE_LATE) {
         ctx->solveRepeats++;
         ctx->lateSkip = 4 << ctx->lateRow;
@@ -2460,7 +2477,8 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
     const double tol = ctx->P.solver_tol > 0 ? ctx->P.solver_tol : DBL_EPSILON;
     const int maxIt = ctx->P.solver_max_iter > 0 ? ctx->P.solver_max_iter : 2 * ctx->nLiveHost;
     int rcL;
-    if ((rcL = oneLaunchFits(ctx, false, oneLaunch))) return rcL;
+    bool probe = false;
+    if ((rcL = oneLaunchFits(ctx, false, oneLaunch, &probe))) return rcL;
     if (*oneLaunch && (rcL = launchOneLaunch(ctx, false, a, c, tol, 0.0, maxIt, 0, oneLaunch))) return rcL;
     if (*oneLaunch) {
         ctx->lastCgIters = ctx->hostInts[I_CG_ITER];
@@ -2476,7 +2494,7 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
     ctx->r0Fresh = false;
     KArgs a0 = a;
     if (fresh) a0.red = ctx->asmRed;
-    hipLaunchKernelGGL(kCgStartFinish, dim3(1), dim3(1024), 0, s, a0, fresh ? ctx->asmBlocks : nb, tol);
+    hipLaunchKernelGGL(kCgStartFinish, dim3(1), dim3(1024), 0, s, a0, fresh ? ctx->asmBlocks : nb, tol, probe ? 1 : 0);
     hipLaunchKernelGGL(kCgZeroX, dim3(nb), dim3(kB), 0, s, a, c.x);
     hipLaunchKernelGGL(kCgInitP, dim3(nb), dim3(kB), 0, s, a, c);
     hipLaunchKernelGGL(kCgInitPFinish, dim3(1), dim3(1024), 0, s, a, nb);
@@ -2497,6 +2515,11 @@ static int solveFp64(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int batc
         if (rc) return rc;
         done = ctx->hostInts[I_CG_DONE];
         iters = ctx->hostInts[I_CG_ITER];
+        if (probe && done == 6) {   // every block has a window again
+            ctx->noWindow = false;
+            ctx->r0Fresh = fresh;
+            return solveFp64(ctx, a, c, nb, batch, oneLaunch);
+        }
         if (launched > 4 * maxIt + 64) break;   // the device flag ends every batch; this only bounds the host loop
     }
     ctx->lastCgIters = iters;
@@ -2535,8 +2558,9 @@ static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int bat
     int total = 0, outer = 0, rc;
     double prevRn2 = 0.0;
     ctx->lastDone = 0;
+    bool probe = false;
     if (!useM) {
-        if ((rc = oneLaunchFits(ctx, true, oneLaunch))) return rc;
+        if ((rc = oneLaunchFits(ctx, true, oneLaunch, &probe))) return rc;
         if (*oneLaunch && (rc = launchOneLaunch(ctx, true, a, c, tol, tolIn, maxIt, kMaxOuter, oneLaunch))) return rc;
         if (*oneLaunch) {
             ctx->solverIter = ctx->hostInts[I_CG_ITER];
@@ -2559,6 +2583,11 @@ static int solveMixed(Ctx* ctx, const KArgs& a, const CgPtrs& c, int nb, int bat
         if (fresh) a0.red = ctx->asmRed;
         hipLaunchKernelGGL(kTrueResidualFinish, dim3(1), dim3(1024), 0, s, a0, fresh ? ctx->asmBlocks : nb);
         if ((rc = readStatus(ctx, nullptr, 0))) return rc;
+        if (probe && outer == 0 && !ctx->hostInts[I_NOWIN]) {   // every block has a window again
+            ctx->noWindow = false;
+            ctx->r0Fresh = fresh;
+            return solveMixed(ctx, a, c, nb, batch, oneLaunch);
+        }
         const double rn2 = ctx->hostScalars[S_TRUE_RN2], bn2 = ctx->hostScalars[S_BN2];
         if (!std::isfinite(rn2) || !std::isfinite(bn2)) break;   // reported by ppeSolve
         if (bn2 == 0.0) {   // zero right-hand side: x = 0, as the FP64 path

@@ -7,6 +7,8 @@ Both solves stop by the same test on the same residual, so they take the same
 number of iterations up to the rounding of the sums, and the answer is judged
 by its residual on the assembled matrix.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -153,6 +155,36 @@ def test_wide_windows(built, shape, precision):
     small = len(w.types) <= 65536
     g = _check(w, precision, ONE_LAUNCH if small else NO_WINDOW)
     assert _widest_window(g) > (16384 if small else 9216)   # slots of the LDS
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_windows_come_back(built, precision):
+    """A context that solved without windows solves the next system as a new
+    context does, in one launch and to the same bits."""
+    wide, narrow = _block(300, 80, 6, thin=300), _block(301, 80, 3)
+    l0 = wide.params.part_dist
+    narrow.pos = narrow.pos * (l0 / (0.6 / 301))   # the lattice of the wide block
+    n = wide.n
+    assert n == narrow.n
+    wide.params.precision_mode = precision
+    wide.params.ppe_transpose = 0
+    print(f"windows come back {n} precision {precision}", flush=True)
+    a = Simulation(wide.params, wide.types, wide.pos, wide.vel, mesh=wide.mesh, device=0)
+    b = Simulation(a.params, wide.types, narrow.pos, wide.vel, mesh=wide.mesh, device=0)
+    a.call("init")
+    assert a.scalar("solve_path") == NO_WINDOW
+    _solve(a, a.get("press"), False)
+    assert a.scalar("solve_path") == NO_WINDOW
+    zero = np.zeros(n)
+    args = [np.ascontiguousarray(v) for v in (wide.types, narrow.pos, wide.vel, zero, zero)]
+    a._check(a._lib.mps_upload_state(a._h, *[v.ctypes.data_as(ctypes.c_void_p) for v in args]))
+    for g in (a, b):
+        g.set("ppe_x", zero)
+        g.call("init")
+        assert g.scalar("solve_path") == ONE_LAUNCH
+    for f in ("press", "ppe_x", "ppe_b"):
+        assert np.array_equal(a.get(f), b.get(f)), f
+    assert a.scalar("solver_iter") == b.scalar("solver_iter") > 0
 
 
 @pytest.mark.parametrize("precision", [0, 1])

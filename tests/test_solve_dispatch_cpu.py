@@ -105,7 +105,7 @@ def path(rt, precision):
         pieces = "kTrueResidualFinish"
     else:
         pieces = "kCgSpmv"
-    for ints, want in ((dict(), 1), (dict(I_NOWIN=1), 2), (dict(I_GRID_LATE=1), 3), (dict(), 1)):
+    for ints, want in ((dict(), 1), (dict(I_GRID_LATE=1), 3), (dict(), 1), (dict(I_NOWIN=1), 2)):
         rt.status(I_CG_DONE=1, **ints)
         g.set_scalar("grid_spin", 4096)   # tries again after a give-up
         rt.launches()
@@ -165,6 +165,34 @@ def backoff(rt, precision):
     late = [k for k, p in enumerate(paths) if p == 3]
     gaps = [b - a - 1 for a, b in zip(late, late[1:])]
     assert gaps == [4, 8, 16, 32, 64, 128, 256, 512, 1024, 1024, 1024]
+    g.close()
+
+
+def no_window(rt, precision):
+    """After a launch that left for want of a window the pieces come first,
+    until the assembly's flag is down again."""
+    g = _sim(precision=precision)
+    # what kCgStartFinish sets where it finds the flag down
+    down = dict(I_CG_DONE=1 if precision else 6)
+    up = dict(I_CG_DONE=1, I_NOWIN=1)
+    for ints, want, tries in ((up, 2, 1), (up, 2, 0), (up, 2, 0), (down, 1, 1), (down, 1, 1), (up, 2, 1), (up, 2, 0)):
+        rt.status(**ints)
+        rt.launches()
+        _solve(g)
+        got = rt.launches()
+        assert g.scalar("solve_path") == want
+        assert sum(k.startswith(ONE_LAUNCH) for k in got) == tries
+        # the assembly's residual serves whichever solves the system
+        assert ("kTrueResidual" if precision else "kCgStart") not in got
+    # a guess that moved after the assembly: its residual is computed for the pieces, and by the launch itself
+    rt.status(**down)
+    g.call("ppe_assemble")
+    g.set_scalar("solver_failures", 0)
+    rt.launches()
+    g.call("ppe_solve")
+    got = rt.launches()
+    assert g.scalar("solve_path") == 1
+    assert got.count("kTrueResidual" if precision else "kCgStart") == 1
     g.close()
 
 
@@ -241,6 +269,11 @@ def test_solve_path(runtime, precision):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_backoff(runtime, precision):
     _child(runtime, "backoff", precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_no_window(runtime, precision):
+    _child(runtime, "no_window", precision)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
