@@ -278,16 +278,30 @@ __device__ __forceinline__ void listOfParticle(const KArgs& a, int i, int* nbr, 
     if (nbrS != nullptr) cntS[i] = cs;
 }
 
-// Lists of the particles whose candidate rows overflowed the mask windows,
-// one wavefront each: few particles, which one lane apiece would walk ~1,400
-// candidates of 27 buckets one by one.  nbrS null: the large list only.
-constexpr int kQueueBlocks = 1024;   // blocks of a launch over a queue of unknown length
+// Lists of n queued particles.  Few of them (the 216,000-particle dam break
+// queues some hundred per step) get a wavefront each: one lane apiece would
+// walk ~1,400 candidates of 27 buckets one by one.  A long queue fills the
+// chip with eight lanes each.  Us per build with every particle queued and 1
+// / 8 / 64 lanes: 466 / 153 / 138 at 13,824 particles, 486 / 211 / 226 at
+// 44,100, 792 / 590 / 793 at 216,000, 5,686 / 5,256 / 7,700 at 1.73M (1,024
+// blocks instead of 4,096: 5,501 with eight).  nbrS null: the large list only.
+constexpr int kQueueBlocks = 4096;   // blocks of a launch over a queue of unknown length
+constexpr int kQueueLong = 16384;
+__device__ __forceinline__ void listsOfQueue(const KArgs& a, const int* queue, int n, int* nbr, int* cnt, int* nbrS,
+                                             int* cntS, double r2, double r2s) {
+    if (n <= kQueueLong)
+        for (int t = groupSlot<64>(); t < n; t += gridDim.x * (blockDim.x / 64))
+            listOfParticle<64>(a, queue[t], nbr, cnt, nbrS, cntS, r2, r2s);
+    else
+        for (int t = groupSlot<8>(); t < n; t += gridDim.x * (blockDim.x / 8))
+            listOfParticle<8>(a, queue[t], nbr, cnt, nbrS, cntS, r2, r2s);
+}
+
+// Lists of the particles whose candidate rows overflowed the mask windows.
 __global__ __launch_bounds__(256) void kFixList(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS,
                                                 const int* fixList, double r2, double r2s, const int* gate) {
     if (gate != nullptr && *gate == 0) return;
-    const int n = a.is[I_FIXCNT];
-    for (int t = groupSlot<64>(); t < n; t += gridDim.x * (blockDim.x / 64))
-        listOfParticle<64>(a, fixList[t], nbr, cnt, nbrS, cntS, r2, r2s);
+    listsOfQueue(a, fixList, a.is[I_FIXCNT], nbr, cnt, nbrS, cntS, r2, r2s);
 }
 
 // Lists of every particle by group walks (L lanes per particle), with the
@@ -2448,15 +2462,12 @@ __global__ __launch_bounds__(256) void kListRefresh(KArgs a, int* patch, double 
 }
 
 // The list of each queued particle from its own stencil walk, in walk order
-// (the order of kBuildList + kMaskToList), one wavefront per particle: of the
-// 216,000-particle dam break's a few hundred change their stencil centre in a
-// step (one lane each: 206 us per launch).
+// (the order of kBuildList + kMaskToList): those that changed their stencil
+// centre in the prediction.
 __global__ __launch_bounds__(256) void kPatchList(KArgs a, int* nbr, int* cnt, int* nbrS, int* cntS, const int* patch,
                                                   double r2, double r2s) {
     if (a.is[I_REBUILD]) return;   // the whole list was rebuilt
-    const int n = a.is[I_PATCHCNT];
-    for (int t = groupSlot<64>(); t < n; t += gridDim.x * (blockDim.x / 64))
-        listOfParticle<64>(a, patch[t], nbr, cnt, nbrS, cntS, r2, r2s);
+    listsOfQueue(a, patch, a.is[I_PATCHCNT], nbr, cnt, nbrS, cntS, r2, r2s);
 }
 
 // Drops from a kept row the entries that lie outside the list radius at the

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from polymps_amd import configs
+from polymps_amd.lib import Simulation
 from tests.parity_util import check, new_pair
 
 pytestmark = pytest.mark.gpu
@@ -61,6 +62,31 @@ def test_polygon_wall_operators(built, shape):
     both("wall_viscosity", "wall_viscosity", ["acc", "force_wall"])
     both("collision", "collision", ["vel"])
     assert np.any(g.get("vel") != w.vel)   # some pairs collided
+
+
+@pytest.mark.parametrize("shape", [(7, 5, 3), (48, 12, 24), (65, 32, 40), (63, 33, 45)])
+def test_queued_particles(built, shape):
+    """A window of one word queues every particle with more than 32 candidates
+    in a stencil row, almost all here; a queue of up to 16,384 takes a
+    wavefront per particle, a longer one eight lanes.  Both give the lists of
+    the full window: same entries, same sums in bits."""
+    w = _dam3d(*shape)
+    print(f"queue {shape} {w.n}", flush=True)
+    out = []
+    for words in (0, 1):
+        g = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh)
+        if words:
+            g.set_scalar("mask_words", words)
+        g.call("bucket_update")
+        g.call("build_neighbor_list")
+        r = [g.scalar("list_entries"), g.scalar("list_entries_small"), g.scalar("list_max")]
+        for op in ("viscosity", "pnd_neigh_npcd", "correction_matrix"):
+            g.call(op)
+        r += [g.get(f) for f in ("acc", "num_neigh", "pnd_small", "npcd", "cm1", "cm2", "cm3")]
+        out.append(r)
+        g.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("l0", [0.02, 0.005, 0.0025, 0.00125])
