@@ -2371,17 +2371,21 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
     // walks of 64 / 16 lanes: 110 / 11 / 18 at 1,728 particles, 124 / 42 / 41
     // at 13,824, 165 / 119 / 97 at 44,100, 214 / 220 / 171 at 81,312, 231 /
     // 339 / 253 at 125,000; 2-D 43 / 9 / 8 at 6,332, 55 / 69 / 36 at 85,292.
-    // (A caller's narrower mask_words asks for the mask path.)
+    // (A caller's narrower mask_words asks for the mask path.)  Periodic
+    // domains above the last line, which have no other build, with 1 / 4 / 16
+    // lanes: 2-D 120 / 107 / 135 at 253,000 and 234 / 201 / 280 at 644,800,
+    // 3-D 911 / 732 / 789 at 333,336 and 2,657 / 2,231 / 2,393 at 1.04M.
     const int lanes = lanesPerParticle(ctx);
     if (P.domain_type_bc == 1 || (lanes != 0 && ctx->maskW == ctx->maskWAlloc)) {
         int* const nS = P.domain_type_bc != 1 && small ? ctx->nbrS : nullptr;
         int* const cS = nS ? ctx->nbrCntS : nullptr;
-        if (lanes == 16)
-            hipLaunchKernelGGL(kBuildListGroup<64>, dim3(gridFor(ctx->N, kBlock / 64)), dim3(kBlock), 0, ctx->stream, a,
-                               ctx->nbr, ctx->nbrCnt, nS, cS, r2, r2s, gate);
-        else
-            hipLaunchKernelGGL(kBuildListGroup<16>, dim3(gridFor(ctx->N, kBlock / 16)), dim3(kBlock), 0, ctx->stream, a,
-                               ctx->nbr, ctx->nbrCnt, nS, cS, r2, r2s, gate);
+#define BLG(L)                                                                                                  \
+    hipLaunchKernelGGL(kBuildListGroup<L>, dim3(gridFor(ctx->N, kBlock / L)), dim3(kBlock), 0, ctx->stream, a,  \
+                       ctx->nbr, ctx->nbrCnt, nS, cS, r2, r2s, gate)
+        if (lanes == 16) BLG(64);
+        else if (lanes == 4) BLG(16);
+        else BLG(4);
+#undef BLG
         MPS_HIP(hipGetLastError());
         ctx->listValid = true;
         return MPS_OK;

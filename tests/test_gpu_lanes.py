@@ -121,6 +121,23 @@ def test_particle_wall_operators(built, l0):
     both("shifting", ["shifting"], ["pos"])
 
 
+@pytest.mark.parametrize("l0", [0.01, 0.004, 0.0014])
+def test_periodic_lists(built, l0):
+    """Lists of a periodic domain by 64, 16 and 4 lanes per particle, seen
+    through the sums over them (the neighbours across the seam among them)."""
+    w = configs.periodic_channel2d(l0=l0, length=round(0.8 / l0) * l0, depth=round(0.2 / l0) * l0, mps_type=2,
+                                   jitter=0.1)
+    print(f"periodic lists {w.n}", flush=True)
+    g, o = new_pair(w)
+    g.call("bucket_update"); o.call("update_buckets")
+    g.call("build_neighbor_list")
+    for op, fields in (("viscosity", ["acc"]), ("pnd_neigh_npcd", ["num_neigh", "pnd_small", "npcd"]),
+                       ("correction_matrix", ["cm1", "cm2", "cm3"])):
+        g.call(op)
+        o.call(op)
+        check(g, o, fields, f"{w.n} {op}")
+
+
 def _sorted_coo(rp, cols, vals, transpose):
     r = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
     if transpose:
