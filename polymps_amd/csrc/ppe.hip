@@ -147,7 +147,7 @@ __device__ __forceinline__ void ppeWindowBegin(const KArgs& a, int i, int* sS, i
         if (threadIdx.x == 0) {
             sB[m] = W;
             sM = m;
-            sOut = (W > kWinMax || periodicDomain(P)) ? 1 : 0;
+            sOut = W > kWinMax ? 1 : 0;
         }
     }
     __syncthreads();
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(256) void kPpeWindow(KArgs a, int* win) {
     t[1] = wM;
     for (int k = 0; k < wM; k++) t[2 + k] = wS[k];
     for (int k = 0; k <= wM; k++) t[11 + k] = wB[k];
-    if (wB[wM] > win16Max(a.N) && !periodicDomain(a.P)) a.is[I_NOWIN] = 1;
+    if (wB[wM] > win16Max(a.N)) a.is[I_NOWIN] = 1;
 }
 
 // One row by L lanes, each with the neighbours c0 + l of a chunk: what the
@@ -1977,9 +1977,10 @@ int ppeAssemble(Ctx* ctx) {
     double* x = ctx->D[DPPEX];
     double* invd64 = (res && !mixed) ? ctx->cgInvD : nullptr;
     const int bFirst = mixed ? 0 : 1;
-    // the CG solves' LDS windows (ppe_window scalar)
-    // and those of a solve in one launch, whatever the scalar says
-    const bool wins = !bicg && ctx->ppeWindow;
+    // the CG solves' LDS windows (ppe_window scalar) and those of a solve in
+    // one launch, whatever the scalar says; not in a periodic domain, where
+    // the columns of rows at the seam are far apart in slot order
+    const bool wins = !bicg && ctx->ppeWindow && !periodicCtx(ctx);
     // (the learned preconditioner's solve runs in pieces)
     const bool wins16 = !bicg && ctx->oneLaunch && oneLaunchRows(ctx) && !(mixed && ctx->P.learned_mode == 2 && ctx->gnn != nullptr);
     if (wins || wins16) {
@@ -1988,7 +1989,7 @@ int ppeAssemble(Ctx* ctx) {
     }
     unsigned char* lc8 = wins ? ctx->aLc8 : nullptr;
     unsigned short* lcEsc = wins ? ctx->aLcEsc : nullptr;
-    int* win = wins || wins16 ? ctx->aWin : nullptr;
+    int* win = wins || (wins16 && !periodicCtx(ctx)) ? ctx->aWin : nullptr;
     unsigned short* lc16 = wins16 ? ctx->aLc16 : nullptr;
     ctx->win16Valid = wins16;
     // Several lanes per row where one lane per row leaves the chip idle (a

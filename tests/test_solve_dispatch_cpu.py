@@ -196,6 +196,27 @@ def no_window(rt, precision):
     g.close()
 
 
+def periodic(rt, precision):
+    """A periodic domain's assembly makes no window tables or codes that no solve reads."""
+    from polymps_amd import configs
+    from polymps_amd.lib import Simulation
+    rt.status(I_CG_DONE=1)
+    w = configs.periodic_channel3d_polygon(l0=0.05, size=(0.3, 0.4))
+    w.params.precision_mode = precision
+    made = []
+    for window in (0, 1):
+        g = Simulation(w.params, w.types, w.pos, w.vel)
+        g.set_scalar("ppe_window", window)
+        live = rt.dll.test_live()
+        rt.launches()
+        _solve(g)
+        got = rt.launches()
+        assert "kPpeWindow" not in got and sum(k.startswith(ONE_LAUNCH) for k in got) == 1
+        made.append(rt.dll.test_live() - live)
+        g.close()
+    assert made[0] == made[1]
+
+
 def switches(rt, precision):
     """one_launch chooses the solver and the memory of its windows; profile does not."""
     from polymps_amd.lib import MpsError
@@ -274,6 +295,11 @@ def test_backoff(runtime, precision):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_no_window(runtime, precision):
     _child(runtime, "no_window", precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_periodic_windows(runtime, precision):
+    _child(runtime, "periodic", precision)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
