@@ -40,6 +40,7 @@ KArgs Ctx::args() const {
     a.nbrCntS = oneList ? nbrCnt : nbrCntS;
     a.KS = oneList ? K : KS;
     a.P4 = P4;
+    a.p4Packed = p4Packed ? 1 : 0;
     a.p4Flags = p4Flags ? 1 : 0;
     a.V4 = V4;
     a.K = K;

@@ -289,7 +289,7 @@ __device__ __forceinline__ void listNbrsQ(const KArgs& a, const int* nbr, const 
 // (types in [-512, 511]); bits 10 and up hold the flags of update_bc.
 __device__ __forceinline__ int p4Type(double w) { return ((((int)w) & 1023) ^ 512) - 512; }
 __device__ __forceinline__ int p4FlagBits(double w) { return ((int)w) >> 10; }
-__device__ __forceinline__ int p4TypeOf(const KArgs& a, double w) { return a.p4Flags ? p4Type(w) : (int)w; }
+__device__ __forceinline__ int p4TypeOf(const KArgs& a, double w) { return a.p4Packed ? p4Type(w) : (int)w; }
 
 // Neighbours of slot i with their positions, f(j, xj, yj, zj): from the list
 // (LIST) or from a bucket walk.

@@ -101,8 +101,9 @@ struct KArgs {
     const int* nbrS;          // entries within the small radius (re_s, collision), column-major [KS][N]
     const int* nbrCntS;
     double4* P4;              // (x, y, z, w) per slot, written by the list build; valid with the list.
-                              // w = type, or after update_bc (p4Flags) type & 1023 | inner << 10 | far-from-wall << 11
-    int p4Flags;
+                              // w = type, or after update_bc (p4Packed) type & 1023 | inner << 10 | far-from-wall << 11
+    int p4Packed;
+    int p4Flags;              // the two flags are those of the current state
     const double4* V4;        // (u, v, w, 0) per slot, packed for the list-based viscosity
     int K;                    // PPE row capacity (ELL width)
     int KS;                   // small-radius list capacity
@@ -180,7 +181,8 @@ struct Ctx {
     int* nbrCntS = nullptr;
     int KS = 0;
     double4* P4 = nullptr;
-    bool p4Flags = false;       // P4.w carries the inner / far-from-wall flags of update_bc
+    bool p4Packed = false;      // P4.w carries the inner / far-from-wall flags of update_bc next to the type
+    bool p4Flags = false;       // ... and they are up to date
     double4* V4 = nullptr;      // packed velocities (viscosity with the list; allocated on first use)
     int K = 0;
     bool listValid = false;

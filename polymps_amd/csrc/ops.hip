@@ -2357,7 +2357,7 @@ __global__ void kPackP4Flags(KArgs a) {
 }
 
 int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
-    ctx->p4Flags = false;
+    ctx->p4Packed = ctx->p4Flags = false;
     KArgs a = ctx->args();
     const int g = gridFor(ctx->N, kBlock);
     const mps_params& P = ctx->P;
@@ -2533,7 +2533,7 @@ int launchListKeepStart(Ctx* ctx, double skin) {
 constexpr double kTightenSkin = 0.04;   // l0
 
 int launchListKeepRefresh(Ctx* ctx, double skin) {
-    ctx->p4Flags = false;
+    ctx->p4Packed = ctx->p4Flags = false;
     if (!ctx->patchList) MPS_HIP(hipMalloc(&ctx->patchList, sizeof(int) * (size_t)ctx->N));
     KArgs a = ctx->args();
     const int g = gridFor(ctx->N, kBlock);
@@ -2749,7 +2749,7 @@ int launchOp(Ctx* ctx, const char* op) {
                               std::min({P.fluid, P.wall, P.dummy_wall, P.ghost}) >= -512;
         if (ctx->listValid && typesFit) {
             hipLaunchKernelGGL(kPackP4Flags, dim3(g), dim3(kBlock), 0, ctx->stream, a);
-            ctx->p4Flags = true;
+            ctx->p4Packed = ctx->p4Flags = true;
         }
     }
     else if (o == "normal_particles") LT(kNormalParticles);

@@ -64,6 +64,37 @@ def test_polygon_wall_operators(built, shape):
     assert np.any(g.get("vel") != w.vel)   # some pairs collided
 
 
+@pytest.mark.parametrize("by", ["upload", "closest_point"])
+def test_types_after_the_flags_are_dropped(built, by):
+    """update_bc packs two flags next to the neighbours' types.  What makes the
+    flags stale, an upload or new wall distances, leaves the types: dummy
+    walls stay out of the matrix and walls keep their viscosity."""
+    w = configs.dam2d_wc_long(l0=0.02, jitter=0.05)
+    w.vel = _velocity(w.n, 33, 2)
+    w.params.mps_type, w.params.pnd_type, w.params.knm_vs2 = 2, 0, 3e-6
+    if by == "closest_point":   # particle walls inside a box mesh
+        w.mesh = configs.mesh_arrays(*configs.box_mesh((-1.0, -1.0, -1.0), (2.0, 2.0, 1.0)))
+    print(f"types after {by} {w.n}", flush=True)
+    g, o = new_pair(w)
+    g.call("init")
+    o.call("init")
+    assert (w.types != 0).any()
+    if by == "upload":
+        g.set("press", g.get("press"))
+        g.set("ppe_x", g.get("ppe_x"))
+    else:
+        g.call("mesh_closest_point")
+        o.call("closest_point")
+    g.call("ppe_assemble")
+    o.call("assemble_ppe")
+    for x, y in zip(_sorted_coo(*g.ppe_matrix(), transpose=False), _sorted_coo(*o.ppe_matrix(), transpose=True)):
+        assert np.array_equal(x, y)
+    check(g, o, ["ppe_b"], "ppe_assemble")
+    g.call("viscosity")
+    o.call("viscosity")
+    check(g, o, ["acc"], "viscosity")
+
+
 @pytest.mark.parametrize("shape", [(7, 5, 3), (48, 12, 24), (65, 32, 40), (63, 33, 45)])
 def test_queued_particles(built, shape):
     """A window of one word queues every particle with more than 32 candidates
