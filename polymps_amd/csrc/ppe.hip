@@ -1996,8 +1996,12 @@ int ppeAssemble(Ctx* ctx) {
     // row's ~120 entries one after the other take ~180 us whatever the count).
     // Us with one lane / 4 / 16 lanes and the window kernel: 178 / 70 / 33 at
     // 1,728 rows, 192 / 94 / 114 at 13,824, 201 / 140 / 275 at 44,100, 231 /
-    // 240 / 490 at 81,312 (FP64 and mixed alike).
-    const int lanes = ctx->N <= 8192 ? 16 : (ctx->N <= 65536 ? 4 : 0);
+    // 240 / 490 at 81,312 (FP64 and mixed alike).  A 2-D row has ~28 entries,
+    // which 16 lanes would spend on the adds; there, called from the host (35
+    // us more): 83 / 61 / 63 at 3,072 rows, 86 / 80 / 140 at 16,437, 89 / 98 /
+    // 205 at 28,412, 97 / 120 / 291 at 43,637.
+    const int lanes = (int)ctx->P.dim == 2 ? (ctx->N <= 20480 ? 4 : 0)
+                                           : ctx->N <= 8192 ? 16 : (ctx->N <= 65536 ? 4 : 0);
     if (lanes != 0) {
         ctx->asmBlocks = gridFor(ctx->N, kB / lanes);
         if (win) hipLaunchKernelGGL(kPpeWindow, dim3(g), dim3(kB), 0, ctx->stream, a, win);

@@ -177,15 +177,8 @@ def _sorted_coo(rp, cols, vals, transpose):
     return r[k], cols[k], vals[k]
 
 
-@pytest.mark.parametrize("shape", [(7, 5, 3), (32, 16, 16), (31, 17, 16), (64, 32, 32), (65, 32, 32)])
-@pytest.mark.parametrize("precision", [0, 1])
-def test_assembly(built, shape, precision):
-    """The assembled system with 16, 4 and one lane per row: entries and
-    right-hand side bit for bit, and the mixed solve's FP32 entries, codes and
-    first residual through the solution they give."""
-    w = _dam3d(*shape)
+def _check_assembly(w, precision):
     w.params.precision_mode = precision
-    print(f"assembly {shape} {w.n} precision {precision}", flush=True)
     g, o = new_pair(w)
     g.call("init")
     o.call("init")
@@ -211,3 +204,25 @@ def test_assembly(built, shape, precision):
     g.call("ppe_assemble")
     g.call("ppe_solve")
     assert np.array_equal(windowed, g.get("ppe_x"))
+
+
+@pytest.mark.parametrize("shape", [(7, 5, 3), (32, 16, 16), (31, 17, 16), (64, 32, 32), (65, 32, 32)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_assembly(built, shape, precision):
+    """The assembled system with 16, 4 and one lane per row: entries and
+    right-hand side bit for bit, and the mixed solve's FP32 entries, codes and
+    first residual through the solution they give."""
+    w = _dam3d(*shape)
+    print(f"assembly {shape} {w.n} precision {precision}", flush=True)
+    _check_assembly(w, precision)
+
+
+@pytest.mark.parametrize("l0", [0.02, 0.0027, 0.0024])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_assembly_2d(built, l0, precision):
+    """The same in 2-D, with 4 lanes per row up to 20,480 rows and one above."""
+    w = configs.dam2d_wc_long(l0=l0, tank=(round(1.0 / l0) * l0, round(0.6 / l0) * l0),
+                              column=(round(0.25 / l0) * l0, round(0.5 / l0) * l0), jitter=0.05)
+    w.params.mps_type, w.params.pnd_type, w.params.solver_tol = 2, 0, 1e-8
+    print(f"assembly 2-D {w.n} precision {precision}", flush=True)
+    _check_assembly(w, precision)
