@@ -285,8 +285,10 @@ __device__ __forceinline__ void listOfParticle(const KArgs& a, int i, int* nbr, 
 // / 8 / 64 lanes: 466 / 153 / 138 at 13,824 particles, 486 / 211 / 226 at
 // 44,100, 792 / 590 / 793 at 216,000, 5,686 / 5,256 / 7,700 at 1.73M (1,024
 // blocks instead of 4,096: 5,501 with eight).  nbrS null: the large list only.
-constexpr int kQueueBlocks = 4096;   // blocks of a launch over a queue of unknown length
 constexpr int kQueueLong = 16384;
+// blocks of a launch over a queue of unknown length, up to N (empty ones take
+// 2.3 us for 1,024, 4.3 for 4,096)
+static int queueBlocks(int N) { return std::min(gridFor(N, 4), std::clamp(gridFor(N, 32), 1024, 4096)); }
 __device__ __forceinline__ void listsOfQueue(const KArgs& a, const int* queue, int n, int* nbr, int* cnt, int* nbrS,
                                              int* cntS, double r2, double r2s) {
     if (n <= kQueueLong)
@@ -2415,7 +2417,7 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
         return MPS_E_UNSUPPORTED;
     }
 #undef M2L
-    hipLaunchKernelGGL(kFixList, dim3(std::min(gridFor(ctx->N, 4), kQueueBlocks)), dim3(kBlock), 0, ctx->stream, a,
+    hipLaunchKernelGGL(kFixList, dim3(queueBlocks(ctx->N)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->nbr, ctx->nbrCnt, small ? ctx->nbrS : nullptr, ctx->nbrCntS, ctx->fixList, r2, r2s, gate);
     MPS_HIP(hipGetLastError());
     ctx->listValid = true;
@@ -2542,7 +2544,7 @@ int launchListKeepRefresh(Ctx* ctx, double skin) {
     MPS_HIP(hipGetLastError());
     int rc = launchBuildList(ctx, 0.0, ctx->is + I_REBUILD);
     if (rc) return rc;
-    hipLaunchKernelGGL(kPatchList, dim3(std::min(gridFor(ctx->N, 4), kQueueBlocks)), dim3(kBlock), 0, ctx->stream, a,
+    hipLaunchKernelGGL(kPatchList, dim3(queueBlocks(ctx->N)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->nbr, ctx->nbrCnt, ctx->nbrS, ctx->nbrCntS, ctx->patchList, listRadius2(ctx->P),
                        listRadiusS2(ctx->P));
     // Below a skin of 0.04 l0 the extra entries are too few to upset the
