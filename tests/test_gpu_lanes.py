@@ -193,17 +193,22 @@ def _check_assembly(w, precision):
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
     check(g, o, ["ppe_b"], f"{w.n} ppe_assemble")
-    # every row group writes its window indices: the blocks are served from
-    # windows, and the same solve gathered from global memory agrees in bits
-    assert g.scalar("ppe_window_blocks") == (w.n + 255) // 256
+    # the 16-bit window indices, through the solve in one launch
     g.call("ppe_solve")
-    windowed = g.get("ppe_x")
-    assert g.scalar("true_residual") <= 1e-8
-    g.set_scalar("ppe_window", 0)
-    g.set("ppe_x", guess)
-    g.call("ppe_assemble")
-    g.call("ppe_solve")
-    assert np.array_equal(windowed, g.get("ppe_x"))
+    assert g.scalar("solve_path") == 1 and g.scalar("true_residual") <= 1e-8
+    # the one-byte codes, through the solve in pieces: every block is served
+    # from its window, and gathering from global memory gives the same bits
+    g.set_scalar("one_launch", 0)
+    x = []
+    for window in (1, 0):
+        g.set_scalar("ppe_window", window)
+        g.set("ppe_x", guess)
+        g.call("ppe_assemble")
+        assert g.scalar("ppe_window_blocks") == window * ((w.n + 255) // 256)
+        g.call("ppe_solve")
+        assert g.scalar("solve_path") == 0 and g.scalar("true_residual") <= 1e-8
+        x.append(g.get("ppe_x"))
+    assert np.array_equal(*x) and np.any(x[0] != guess)
 
 
 @pytest.mark.parametrize("shape", [(7, 5, 3), (32, 16, 16), (31, 17, 16), (64, 32, 32), (65, 32, 32)])
@@ -211,7 +216,7 @@ def _check_assembly(w, precision):
 def test_assembly(built, shape, precision):
     """The assembled system with 16, 4 and one lane per row: entries and
     right-hand side bit for bit, and the mixed solve's FP32 entries, codes and
-    first residual through the solution they give."""
+    first residual through the solutions they give."""
     w = _dam3d(*shape)
     print(f"assembly {shape} {w.n} precision {precision}", flush=True)
     _check_assembly(w, precision)

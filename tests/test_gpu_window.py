@@ -7,7 +7,8 @@ mixed solve's FP32 SpMV, its FP64 true residual and the FP64 CG's SpMV); the
 other blocks gather from global memory, as every block does with the windows
 off.  Both sum the same products in the same order, so whole runs must agree
 bit for bit, and at the benchmark's density almost every block must take
-its window.
+its window.  The solves run in pieces here (one_launch 0): a solve in one
+launch has windows of its own, whatever the scalar says.
 """
 import numpy as np
 import pytest
@@ -23,6 +24,8 @@ def _pair(w):
     on = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh)
     off = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh)
     off.set_scalar("ppe_window", 0)
+    on.set_scalar("one_launch", 0)
+    off.set_scalar("one_launch", 0)
     assert on.scalar("ppe_window") == 1 and off.scalar("ppe_window") == 0
     return on, off
 
@@ -53,6 +56,7 @@ def test_window_runs_are_bit_identical(built, l0, steps, precision):
     used = on.scalar("ppe_window_blocks")
     print(f"  blocks with a window: {used:.0f} of {nb}", flush=True)
     assert off.scalar("ppe_window_blocks") == 0
+    assert on.scalar("solve_path") == 0 and off.scalar("solve_path") == 0
     assert used >= 0.8 * nb
     assert on.scalar("solver_iter") == off.scalar("solver_iter")
     on.close()
