@@ -115,7 +115,10 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * after the prediction) "list_skin_factor" (automatic skin as a multiple of
  * the largest one-step displacement, in [2, 10], default 3) "mask_words" (candidate
  * window per stencil row in 32-slot words, at most the allocated width;
- * particles with a longer row are listed by a direct walk, same results)
+ * particles with a longer row are listed by a direct walk, same results;
+ * above 81,920 particles and outside periodic domains an allocated width of
+ * more than 16, re_l above 3.95 part_dist in 3-D with cfl_number 0.2, gives
+ * MPS_E_UNSUPPORTED at the list build unless a narrower one is set)
  * "profile" (nonzero: time every eighth SpMV launch with HIP events, counters
  * reset; results do not change)
  * "precision_mode" (MPS_PREC_*, used from the next PPE assembly)
@@ -126,9 +129,10 @@ int mps_upload_field(mps_ctx* ctx, const char* field, const void* in, size_t cou
  * "learned_tol_scale" (in (0, 1], default 0.1: with the learned
  * preconditioner the true residual is driven to this multiple of the
  * tolerance, since the flexible CG's error at a given residual is larger)
- * "ppe_window" (1 default: the CG solves' SpMVs read each 256-row block's
- * vector window from LDS; 0: from global memory; same results,
- * used from the next assembly; read-only "ppe_window_blocks": blocks of the
+ * "ppe_window" (1 default: the SpMVs of CG solves in pieces read each
+ * 256-row block's vector window from LDS; 0: from global memory; same results,
+ * used from the next assembly; not in a periodic domain, and a solve in one
+ * launch has windows of its own either way; read-only "ppe_window_blocks": blocks of the
  * last assembly served from a window, "window_escapes": window index
  * escapes of the last assembly, the rows' absolute indices next to their
  * one-byte steps) "one_launch" (1 default: CG solves of up

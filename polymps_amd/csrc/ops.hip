@@ -2392,6 +2392,11 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
         ctx->listValid = true;
         return MPS_OK;
     }
+    if (ctx->maskW > 16) {
+        ctx->err = "neighbour bitmask rows wider than 512 candidates (a large radius above 3.95 particle distances in "
+                   "3-D) are not supported above 81,920 particles";
+        return MPS_E_UNSUPPORTED;
+    }
     const int gw = gridFor(ctx->N, 64);
     if (!ctx->fixList) MPS_HIP(hipMalloc(&ctx->fixList, sizeof(int) * (size_t)ctx->N));
     MPS_HIP(hipMemsetAsync(ctx->is + I_FIXCNT, 0, sizeof(int), ctx->stream));
@@ -2411,11 +2416,7 @@ int launchBuildList(Ctx* ctx, double skin, const int* gate, bool small) {
     } while (0)
     if (ctx->maskW <= 4) M2L(4);
     else if (ctx->maskW <= 8) M2L(8);
-    else if (ctx->maskW <= 16) M2L(16);
-    else {
-        ctx->err = "neighbour bitmask rows wider than 512 candidates are not supported";
-        return MPS_E_UNSUPPORTED;
-    }
+    else M2L(16);
 #undef M2L
     hipLaunchKernelGGL(kFixList, dim3(queueBlocks(ctx->N)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->nbr, ctx->nbrCnt, small ? ctx->nbrS : nullptr, ctx->nbrCntS, ctx->fixList, r2, r2s, gate);

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from polymps_amd import configs
-from polymps_amd.lib import Simulation
+from polymps_amd.lib import MpsError, Simulation
 from tests.parity_util import check, new_pair
 
 pytestmark = pytest.mark.gpu
@@ -231,3 +231,32 @@ def test_assembly_2d(built, l0, precision):
     w.params.mps_type, w.params.pnd_type, w.params.solver_tol = 2, 0, 1e-8
     print(f"assembly 2-D {w.n} precision {precision}", flush=True)
     _check_assembly(w, precision)
+
+
+def test_wide_radius(built):
+    """A large radius of 4.1 l0 takes mask rows of more than 512 candidates.
+    Up to 81,920 particles the lists come from group walks, which need none;
+    above, the build refuses unless the caller narrows the window."""
+    w = _dam3d(24, 6, 12)
+    w.params.re_l = 4.1
+    print(f"wide radius {w.n}", flush=True)
+    g, o = new_pair(w)
+    assert g.scalar("list_capacity") > 512
+    g.call("bucket_update"); o.call("update_buckets")
+    g.call("build_neighbor_list")
+    for op, fields in (("viscosity", ["acc"]), ("pnd_neigh_npcd", ["num_neigh", "pnd_small", "npcd"])):
+        g.call(op)
+        o.call(op)
+        check(g, o, fields, op)
+    w = _dam3d(24, 6, 12)
+    w.params.re_l = 4.1
+    _check_assembly(w, 1)
+    w = _dam3d(78, 33, 32)
+    w.params.re_l = 4.1
+    print(f"wide radius {w.n}", flush=True)
+    g = Simulation(w.params, w.types, w.pos, w.vel, mesh=w.mesh)
+    with pytest.raises(MpsError, match="512 candidates"):
+        g.call("init")
+    g.set_scalar("mask_words", 16)
+    g.call("init")
+    assert g.scalar("list_max") > 200
