@@ -54,10 +54,15 @@ def _f(s):
     return n, L, LS, nnz, nesc, mask
 
 
-# kernel -> (bytes of one launch, what is counted)
+# kernel -> (bytes of one launch, what is counted).  A key names every kernel
+# whose template arguments start with its own (bytesOf): the lanes per
+# particle and batch sizes that follow change no count.
 def model(sizes):
     n, L, LS, nnz, nesc, mask = _f(sizes)
     nlc = sizes.get("nlc", 0)   # window index escapes
+    asm = (4 * nesc + 2 * nlc + 4 * L + 116 * n,
+           "escapes; reads the large list; "
+           "per particle P4, x, mirror, bc, source in (80), count, diag, b, FP32 diag / 1/diag, r out (36)")
     return {
         "kMxSpmv": (5 * nnz + 2 * nlc + 16 * n,
                     "FP32 value 4 + window code 1 per entry, 2 per window escape; per row count 4, diag 4, "
@@ -68,9 +73,13 @@ def model(sizes):
         "kTrueResidual": (9 * nnz + 2 * nlc + 36 * n,
                           "FP64 values and window codes; per row count, diag, x, b in, r out"),
         "kPpeAssemble<true, true, true>": (
-            15 * nnz + 4 * nesc + 2 * nlc + 4 * L + 116 * n,
-            "writes FP64 + FP32 values, codes and window codes (15 per entry), escapes; reads the large list; "
-            "per particle P4, x, mirror, bc, source in (80), count, diag, b, FP32 diag / 1/diag, r out (36)"),
+            15 * nnz + asm[0], "writes FP64 + FP32 values, codes and window codes (15 per entry), " + asm[1]),
+        "kPpeAssemble<true, true, true, true>": (
+            17 * nnz + asm[0], "writes FP64 + FP32 values, codes, window codes and 16-bit window indices (17 per "
+                               "entry), " + asm[1]),
+        "kPpeAssembleGroup<true, true, true>": (
+            17 * nnz + asm[0], "writes FP64 + FP32 values, codes, window codes and 16-bit window indices (17 per "
+                               "entry), " + asm[1]),
         "kViscosity<true>": (4 * L + 140 * n,
                              "large list; P4 32, packed velocity 32, own velocity 24, mirror 24, count 4 in; "
                              "acceleration 24 out"),
@@ -89,17 +98,34 @@ def model(sizes):
                              "positions, type in; P4 out, both candidate bitmasks (rows x words x 4) and counts out"),
         "kBuildList<false>": (28 * n + 32 * n + mask + 4 * n,
                               "positions, type in; P4, the large-radius bitmask and its counts out"),
-        "kMaskToList<8>": (None, "bitmask + count in, list out (large or small list: per call)"),
-        "kMxUpdate": (32 * n, "d, p, r, q, 1/diag in (FP32); d, r, z out"),
-        "kMxP": (12 * n, "z, p in; p out (FP32)"),
+        "kBuildListGroup": (28 * n + 32 * n + 4 * (L + LS) + 8 * n,
+                            "positions, type in; P4, both lists and counts out"),
+        "kMaskToList": (None, "bitmask + count in, list out (large or small list: per call)"),
+        "kCgUpdate<float>": (40 * n, "d (FP64), p, r, q, 1/diag in (FP32); d, r, z out"),
+        "kCgUpdate<double>": (64 * n, "x, p, r, q, 1/diag in (FP64); x, r, z out"),
+        "kCgP<float>": (12 * n, "z, p in; p out (FP32)"),
+        "kCgP<double>": (24 * n, "z, p in; p out (FP64)"),
+        "kFcgP": (12 * n, "z, p in; p out (FP32)"),
         "kPackVel": (56 * n, "velocity in, packed velocity out"),
     }
 
 
 def _key(name: str) -> str:
     """'void mpsgpu::kFoo<true>(mpsgpu::KArgs, ...)' -> 'kFoo<true>'."""
-    s = re.sub(r"^void ", "", name).split("(")[0]
+    s = re.sub(r"^void ", "", name.replace("(anonymous namespace)::", "")).split("(")[0]
     return s[len("mpsgpu::"):] if s.startswith("mpsgpu::") else s
+
+
+def bytesOf(mdl, kernel):
+    """The model's entry of a kernel: that of its full name, else of the
+    longest beginning of its template arguments."""
+    base, _, args = kernel.partition("<")
+    args = [x.strip() for x in args.rstrip(">").split(",")] if args else []
+    for k in range(len(args), -1, -1):
+        key = base + (f"<{', '.join(args[:k])}>" if k else "")
+        if key in mdl:
+            return mdl[key]
+    return None, ""
 
 
 def _working(durs):
@@ -179,7 +205,7 @@ def table(args):
         wk = _working(durs)
         mean_ns = sum(wk) / len(wk)
         share = 100.0 * sum(durs) / total
-        alg = mdl.get(k, (None, ""))[0]
+        alg = bytesOf(mdl, k)[0]
         cells = [k, str(len(durs)), str(len(wk)), f"{mean_ns / 1e3:.1f}", f"{share:.1f}%"]
         if alg:
             tbs = alg / mean_ns / 1e3
@@ -206,8 +232,9 @@ def table(args):
     out.append("Algorithmic bytes counted per kernel:")
     out.append("")
     for k, durs in rows:
-        if k in mdl and mdl[k][0]:
-            out.append(f"* `{k}`: {mdl[k][1]}")
+        alg, what = bytesOf(mdl, k)
+        if alg:
+            out.append(f"* `{k}`: {what}")
     return "\n".join(out)
 
 

@@ -1,6 +1,8 @@
 """The per-kernel byte model and table tool (no GPU)."""
 import json
+import re
 import sqlite3
+import subprocess
 
 from polymps_amd import roofline as R
 
@@ -8,8 +10,28 @@ from polymps_amd import roofline as R
 def test_kernel_names():
     assert R._key("void mpsgpu::kPpeAssemble<true, true, true>(mpsgpu::KArgs, double*)") == \
         "kPpeAssemble<true, true, true>"
+    assert R._key("void mpsgpu::(anonymous namespace)::kViscosityNN<true>(mpsgpu::KArgs)") == "kViscosityNN<true>"
     assert R._key("mpsgpu::kMxSpmv(mpsgpu::KArgs, mpsgpu::CgPtrs)") == "kMxSpmv"
     assert R._key("__amd_rocclr_copyBuffer") == "__amd_rocclr_copyBuffer"
+
+
+def test_every_model_entry_names_a_kernel(built):
+    """A kernel that is renamed or gets other template arguments must not
+    fall out of the table: every entry is some kernel of the library, and the
+    kernels that carry a step have one."""
+    out = subprocess.run(["nm", "-C", str(built)], capture_output=True, text=True, check=True).stdout
+    kernels = {R._key(m.group(1)) for m in re.finditer(r"__device_stub__(\S.*)", out)}
+    m = R.model({"n": 1, "L": 1, "LS": 1, "nnz": 1, "nesc": 1, "nlc": 1})
+    found = {id(R.bytesOf(m, k)) for k in kernels}
+    assert [k for k, v in m.items() if id(v) not in found] == []
+    for k in ("kViscosity<true, 4, 4, 4>", "kPndNeighNPCD<true, 2, 2, 4>", "kCorrectionMatrix<true, 1, 2, 4>",
+              "kPressGradient<true, 2, 2, 4>", "kCollisionPC<true, 2, 2, 4>", "kPpeAssemble<true, true, true, false>",
+              "kPpeAssemble<true, true, true, true>", "kCgUpdate<float, false>", "kCgP<float>", "kBuildList<true>"):
+        assert k in kernels and R.bytesOf(m, k)[0], k
+    assert R.bytesOf(m, "kPpeAssemble<true, true, true, true>")[0] == R.bytesOf(
+        m, "kPpeAssemble<true, true, true, false>")[0] + 2
+    # a bucket walk is not a list launch
+    assert R.bytesOf(m, "kViscosity<false, 4, 1, 1>")[0] is None
 
 
 def test_spmv_bytes_match_the_library_formula():
