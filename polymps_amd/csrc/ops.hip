@@ -2637,7 +2637,15 @@ __global__ __launch_bounds__(kBlock) void kExtrapolateWallDummy2(KArgs a) {
     if (!(ti == P.dummy_wall || (P.mps_type == MPS_WEAKLY && ti == P.wall))) return;
     const double xi = PX(i), yi = PY(i), zi = PZ(i);
     double ni = 0.0, pr = 0.0;
-    auto press = [&](int j) { return a.D[DPRESS][j]; };
+    // other threads write the wall and dummy slots' pressures meanwhile
+    struct FluidPress {
+        bool fluid;
+        double p;
+    };
+    auto press = [&](int j) {
+        const bool fluid = a.I[ITYPE][j] == P.fluid;
+        return FluidPress{fluid, fluid ? a.D[DPRESS][j] : 0.0};
+    };
     forBatches<LIST, true, L, B, G>(a, i, xi, yi, zi, press, [&](const auto& t) {
         constexpr int nb = std::remove_reference_t<decltype(t)>::B;
         double d[nb], w[nb], v0[nb], v1[nb], v2[nb];
@@ -2648,7 +2656,7 @@ __global__ __launch_bounds__(kBlock) void kExtrapolateWallDummy2(KArgs a) {
             v1[b] = t.y[b] - yi;
             v2[b] = t.z[b] - zi;
             const double d2 = v0[b] * v0[b] + v1[b] * v1[b] + v2[b] * v2[b];
-            ok[b] = t.ok[b] & (d2 < P.re_s2) & (a.I[ITYPE][t.j[b]] == P.fluid);
+            ok[b] = t.ok[b] & (d2 < P.re_s2) & t.e[b].fluid;
             any = any | ok[b];
             d[b] = sqrt(d2);
         }
@@ -2656,7 +2664,7 @@ __global__ __launch_bounds__(kBlock) void kExtrapolateWallDummy2(KArgs a) {
         wgtBatch(d, P.re_s, P.weight_type, w);
 #pragma unroll
         for (int b = 0; b < nb; b++) {
-            const double p = t.e[b] - rhoOf(a, t.j[b]) * (P.gravity[0] * v0[b] + P.gravity[1] * v1[b] + P.gravity[2] * v2[b]);
+            const double p = t.e[b].p - rhoOf(a, t.j[b]) * (P.gravity[0] * v0[b] + P.gravity[1] * v1[b] + P.gravity[2] * v2[b]);
             addOrdered<L>(ni, ok[b] ? w[b] : 0.0);
             addOrdered<L>(pr, ok[b] ? p * w[b] : 0.0);
         }
