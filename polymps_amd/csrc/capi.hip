@@ -1014,8 +1014,11 @@ static int buildBvhInto(Ctx* ctx, const double* V, const int* F, int nf, BvhNode
         if (*outTri) (void)hipFree(*outTri);
         *outBvh = nullptr;
         *outTri = nullptr;
-        MPS_HIP(hipMalloc(outBvh, sizeof(BvhNode) * nodes.size()));
-        MPS_HIP(hipMalloc(outTri, sizeof(int) * (size_t)nf));
+        BvhNode* made = nullptr;   // both or none: the search takes a mesh without nodes face by face
+        int rc = ensureBuffer(ctx, &made, nodes.size());
+        if (!rc && (rc = ensureBuffer(ctx, outTri, (size_t)nf))) (void)hipFree(made);
+        if (rc) return rc;
+        *outBvh = made;
     }
     MPS_HIP(hipMemcpyAsync(*outBvh, nodes.data(), sizeof(BvhNode) * nodes.size(), hipMemcpyHostToDevice, ctx->stream));
     MPS_HIP(hipMemcpyAsync(*outTri, idx.data(), sizeof(int) * (size_t)nf, hipMemcpyHostToDevice, ctx->stream));
@@ -1046,9 +1049,10 @@ static void faceNormals(const std::vector<double>& V, const std::vector<int>& F,
 
 static int uploadSlot(Ctx* ctx, MeshSlot& m, bool rebuildBvh) {
     if (!m.V) {
-        MPS_HIP(hipMalloc(&m.V, sizeof(double) * 3 * (size_t)m.nv));
-        MPS_HIP(hipMalloc(&m.F, sizeof(int) * 3 * (size_t)m.nf));
-        MPS_HIP(hipMalloc(&m.N, sizeof(double) * 3 * (size_t)m.nf));
+        int rc;
+        if ((rc = ensureBuffer(ctx, &m.V, 3 * (size_t)m.nv))) return rc;
+        if ((rc = ensureBuffer(ctx, &m.F, 3 * (size_t)m.nf))) return rc;
+        if ((rc = ensureBuffer(ctx, &m.N, 3 * (size_t)m.nf))) return rc;
         MPS_HIP(hipMemcpyAsync(m.F, m.hF.data(), sizeof(int) * 3 * (size_t)m.nf, hipMemcpyHostToDevice, ctx->stream));
     }
     MPS_HIP(hipMemcpyAsync(m.V, m.hV.data(), sizeof(double) * 3 * (size_t)m.nv, hipMemcpyHostToDevice, ctx->stream));
@@ -1122,12 +1126,16 @@ int mps_set_mesh(mps_ctx* ctx, int nv, const double* V, int nf, const int* F, co
     for (int q = 0; q < 3 * nf; q++)
         if (F[q] < 0 || F[q] >= nv) { ctx->err = "face index out of range"; return MPS_E_ARG; }
     MPS_HIP(hipSetDevice(ctx->dev));
+    ctx->hasMesh = false;   // until the new one is in place
     if (ctx->mV) hipFree(ctx->mV);
     if (ctx->mF) hipFree(ctx->mF);
     if (ctx->mN) hipFree(ctx->mN);
-    MPS_HIP(hipMalloc(&ctx->mV, sizeof(double) * 3 * nv));
-    MPS_HIP(hipMalloc(&ctx->mF, sizeof(int) * 3 * nf));
-    MPS_HIP(hipMalloc(&ctx->mN, sizeof(double) * 3 * nf));
+    ctx->mV = ctx->mN = nullptr;
+    ctx->mF = nullptr;
+    int rc;
+    if ((rc = ensureBuffer(ctx, &ctx->mV, 3 * (size_t)nv))) return rc;
+    if ((rc = ensureBuffer(ctx, &ctx->mF, 3 * (size_t)nf))) return rc;
+    if ((rc = ensureBuffer(ctx, &ctx->mN, 3 * (size_t)nf))) return rc;
     MPS_HIP(hipMemcpy(ctx->mV, V, sizeof(double) * 3 * nv, hipMemcpyHostToDevice));
     MPS_HIP(hipMemcpy(ctx->mF, F, sizeof(int) * 3 * nf, hipMemcpyHostToDevice));
     MPS_HIP(hipMemcpy(ctx->mN, N, sizeof(double) * 3 * nf, hipMemcpyHostToDevice));
@@ -1156,7 +1164,9 @@ int mps_set_mesh_type(mps_ctx* ctx, int type, int nv, const double* V, int nf, c
     m.hF.assign(F, F + 3 * (size_t)nf);
     m.hN.assign(N, N + 3 * (size_t)nf);
     m.on = true;
-    return uploadSlot(ctx, m, ctx->bvhMode != 0);
+    const int rc = uploadSlot(ctx, m, ctx->bvhMode != 0);
+    if (rc) freeSlot(m);   // not installed
+    return rc;
 }
 
 int mps_get_mesh(mps_ctx* ctx, int type, int* nv, double* V, int* nf, int* F, double* N) {

@@ -96,6 +96,57 @@ def allocations(rt, solver, precision, learned):
 ONE_LAUNCH = ("kCgOneLaunch", "kMxOneLaunch")
 
 
+def meshes(rt, kind):
+    """A wall mesh whose allocation fails is not installed half: the closest
+    point search refuses it or does without its tree, and the next mesh and
+    the context's end find no pointer of it."""
+    from polymps_amd import configs
+    from polymps_amd.lib import MpsError
+    V, F = configs.channel_mesh(nhx=8, nhy=8)[:2]
+    mesh = configs.mesh_arrays(V, F)
+    assert len(mesh[1]) // 3 > 64   # with a tree
+
+    def install(g):
+        g.set_mesh_type(kind, *mesh)
+
+    def made(fail):
+        g = _sim()
+        install(g)   # one to replace
+        live, before = rt.dll.test_live(), rt.dll.test_allocations()
+        rt.dll.test_fail_allocation(fail)
+        failed = False
+        try:
+            install(g)
+        except MpsError as e:
+            assert "out of memory" in str(e), e
+            failed = True
+        calls = rt.dll.test_allocations() - before
+        rt.dll.test_fail_allocation(0)
+        rt.launches()
+        refused = False
+        try:
+            g.closest_point_type(kind)
+        except MpsError:
+            refused = True
+        got = rt.launches()
+        if refused:
+            assert not any(k.startswith("kClosestPoint") for k in got)
+        else:
+            assert ("kClosestPointBvh" in got) == (not failed)
+        install(g)
+        n = rt.dll.test_live() - live
+        g.close()
+        return n, calls, failed, refused
+
+    n, calls, failed, refused = made(0)
+    assert n == 0 and calls >= 3 and not failed and not refused
+    for k in range(1, calls + 1):
+        n, _, failed, refused = made(k)
+        assert failed and n == 0, k
+        assert refused or (kind == 0 and k > 3), k
+    assert rt.dll.test_live() == 0
+
+
 def path(rt, precision):
     """solve_path says what was launched: the one launch alone, or the pieces
     after it and why, or the pieces alone."""
@@ -280,6 +331,11 @@ def _child(runtime, case, *args):
 @pytest.mark.parametrize("solver,precision,learned", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
 def test_allocation_failures(runtime, solver, precision, learned):
     _child(runtime, "allocations", solver, precision, learned)
+
+
+@pytest.mark.parametrize("kind", [0, 2])
+def test_mesh_allocation_failures(runtime, kind):
+    _child(runtime, "meshes", kind)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
